@@ -109,7 +109,7 @@ void tf_ctx_destroy(tf_ctx *ctx);
  * enqueues nothing; no entry point allocates, frees or synchronises.  tf_ctx_create's limits are
  * {262144, 2048, 256, 2112, 16, 512, 128}. */
 typedef struct tf_scratch_limits {
-    uint32_t max_vocab;                  /* lm_head rows: fp32 logits of the unaligned greedy path, the samplers' cells and top-k pair buffers */
+    uint32_t max_vocab;                  /* lm_head rows: fp32 logits of the unaligned greedy path, the samplers' cells and chunk maxima */
     uint32_t max_block_tokens;           /* rows of one prefill block: router logits [tokens, experts], shared-expert activations */
     uint32_t max_experts;                /* router width of the multi-token router */
     uint32_t max_shared_intermediate;    /* shared expert's intermediate size (activations [tokens, intermediate] of the block form) */
@@ -829,7 +829,7 @@ int32_t tf_logit_softcap_softmax(tf_ctx *ctx, tf_stream stream, const void *logi
 int32_t tf_sample(tf_ctx *ctx, tf_stream stream, const void *probs, void *out_token, uint32_t v, float temperature, uint32_t top_k,
                   float top_p, uint64_t seed, uint32_t position);
 /* SampleTopK64.encode (Kernels/Sampling/LogitOutput.swift:150-206) -> sample_topk64_stage1 / _reduce / _final
- * (Metal/Sampling/logit.metal:449-606): the top-64 sampler through sorted 1024-entry tiles; same token as
+ * (Metal/Sampling/logit.metal:449-606): the top-64 sampler; same token as
  * tf_sample(..., top_k = 64, ...).  vocab in 1...262144 (SampleTopK64Error.unsupportedVocabulary otherwise). */
 int32_t tf_sample_topk64(tf_ctx *ctx, tf_stream stream, const void *probs, void *out_token, uint32_t vocab, float temperature, float top_p,
                          uint64_t seed);

@@ -181,3 +181,32 @@ def test_top_k_keeps_only_the_top_and_ties_resolve_to_low_indices():
     k = ctx()
     assert k.lib.tf_sample_topk64(k.handle, None, d_flat.data_ptr(), d_flat.data_ptr(), 262145, 1.0, 0.95, 1) == tfk.TF_ERR_INVALID_ARGUMENT
     assert k.lib.tf_sample(k.handle, None, d_flat.data_ptr(), d_flat.data_ptr(), 0, 1.0, 0, 1.0, 1, 0) == tfk.TF_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("v", [1, 63, 65, 2049, 8192, 8193, 32768, 32769, 100003, 262144])
+@pytest.mark.parametrize("kind", ["ties", "few", "spread", "odd"])
+def test_top_k_selection_at_its_edges(v, kind):
+    """One block over everything up to 8192 / 32768 elements, chunk maxima beyond; ties that fill whole chunks must resolve to the
+    lowest indices, values that must never be chosen stay out, unaligned probabilities are read element by element."""
+    rng = np.random.default_rng(v * 7 + len(kind))
+    if kind == "ties":               # every chunk maximum equal, one larger element
+        values = np.full(v, 0.001, np.float32)
+        values[v // 2] = 0.01
+    elif kind == "few":              # fewer positive probabilities than k; the rest are zeros taken by index
+        values = np.zeros(v, np.float32)
+        values[rng.integers(0, v, 20)] = rng.random(20).astype(np.float32)
+    elif kind == "spread":           # coarse values: ties straddle the cut
+        values = rng.integers(1, 40, v).astype(np.float32) / 4096.0
+    else:
+        values = rng.random(v).astype(np.float32)
+        values[rng.integers(0, v, max(1, v // 3))] = -np.inf
+        values[rng.integers(0, v, max(1, v // 3))] = np.nan
+        values[rng.integers(0, v, max(1, v // 5))] = -0.25
+    bits = f16(values)
+    d_probs, d_odd = dev(bits), dev(np.concatenate([np.zeros(1, np.uint16), bits]))
+    for seed in (5, 6, 7):
+        want = tfo.sample_topk64(bits, 1.0, 0.95, seed)
+        assert gpu_sample(d_probs, v, 1.0, 0, 0.95, seed, topk64=True) == want
+        assert gpu_sample(d_odd[2:], v, 1.0, 0, 0.95, seed, topk64=True) == want
+        for top_k, top_p in ((1, 1.0), (65, 0.9), (256, 1.0)):
+            assert gpu_sample(d_probs, v, 1.0, top_k, top_p, seed) == tfo.sample(bits, 1.0, top_k, top_p, seed), (top_k, top_p, seed)

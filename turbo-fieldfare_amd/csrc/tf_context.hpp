@@ -23,7 +23,7 @@ struct tf_ctx {
     uint8_t *few_scratch = nullptr;     // kFewScratchBytes: sorted pairs, per-expert tables and work list of tf_prefill_routed_moe_few_tokens
     float *prefill_logits = nullptr;    // [tokens, experts] router logits (+ partial planes) of the multi-token router
     size_t prefill_logits_count = 0;
-    void *sample_scratch = nullptr;     // argmax cells, softmax partials, top-k pair buffers of the samplers
+    void *sample_scratch = nullptr;     // argmax cells, softmax partials, chunk maxima of the samplers
     size_t sample_scratch_bytes = 0;
     void *shared_block_acts = nullptr;  // [rows, intermediate] fp16 activations of the block shared expert
     size_t shared_block_acts_bytes = 0;

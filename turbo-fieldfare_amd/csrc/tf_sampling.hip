@@ -1,7 +1,7 @@
 // What sits either side of the tied int4 output head: the embedding row lookup (same table), the soft-capped softmax over
 // the vocabulary, and the samplers (greedy, Gumbel-max, top-k / top-p / temperature with inverse-CDF draw).
 // The reference runs each of these in a single threadgroup; here the vocabulary-sized passes are spread over the chip and
-// meet through per-block partials (softmax), an atomic argmax fold (greedy, Gumbel) or sorted tiles (top-k).
+// meet through per-block partials (softmax), an atomic argmax fold (greedy, Gumbel) or the maxima of 64-element chunks (top-k).
 #include "tf_argmax.hpp"
 #include "tf_context.hpp"
 #include "tf_rowdot.hpp"
@@ -73,15 +73,41 @@ __device__ __forceinline__ void block_merge_md(float &m, float &d, float *scratc
     for (int w = 1; w < 4; ++w) merge_md(m, d, scratch[w], scratch[4 + w]);
 }
 
-template <typename T>
+// Both launches are a chain of transcendental functions behind one load, not bandwidth (0.5 MB): a thread takes four neighbours
+// (one load) and the online rule once per four, and a vocabulary of 262144 spreads over 256 blocks (softcap + softmax of 262144
+// fp16 logits 4.6 us; 8.7 us with eight elements a thread taken one by one over 128 blocks).
+constexpr uint32_t kSoftmaxRun = 4;
+
+// logits [i, i + 4) below v; missing ones are -inf.  VEC: the row is aligned to whole runs
+template <bool VEC, typename T>
+__device__ __forceinline__ void load_run(const T *logits, uint32_t i, uint32_t v, float z[kSoftmaxRun]) {
+    if (VEC && i + kSoftmaxRun <= v) {
+        typedef T run_t __attribute__((ext_vector_type(kSoftmaxRun)));
+        const run_t x = *reinterpret_cast<const run_t *>(logits + i);
+#pragma unroll
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = (float)x[j];
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = i + j < v ? (float)logits[i + j] : -INFINITY;
+    }
+}
+
+template <bool VEC, typename T>
 __global__ __launch_bounds__(256) void softmax_partials_kernel(const T *logits, float *partials, uint32_t v, float softcap) {
     __shared__ float scratch[8];
     float m = -INFINITY, d = 0.0f;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < v; i += gridDim.x * blockDim.x) {
-        const float z = softcapped((float)logits[i], softcap);
-        const float mn = fmaxf(m, z);
-        const float scale = (m == -INFINITY) ? 0.0f : expf(m - mn);
-        d = d * scale + expf(z - mn);
+    for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * kSoftmaxRun; i < v; i += gridDim.x * blockDim.x * kSoftmaxRun) {
+        float z[kSoftmaxRun], mn = m;
+        load_run<VEC>(logits, i, v, z);
+#pragma unroll
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j) {
+            z[j] = i + j < v ? softcapped(z[j], softcap) : -INFINITY;
+            mn = fmaxf(mn, z[j]);
+        }
+        d = (m == -INFINITY) ? 0.0f : d * expf(m - mn);
+#pragma unroll
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j)
+            if (i + j < v) d += expf(z[j] - mn);
         m = mn;
     }
     block_merge_md(m, d, scratch);
@@ -91,19 +117,46 @@ __global__ __launch_bounds__(256) void softmax_partials_kernel(const T *logits, 
     }
 }
 
-template <typename T>
+template <bool VEC, typename T>
 __global__ __launch_bounds__(256) void softmax_normalize_kernel(const T *logits, const float *partials, uint32_t n_partials, half_t *probs,
                                                                 uint32_t v, float softcap) {
     __shared__ float scratch[8];
+    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * kSoftmaxRun;
+    float z[kSoftmaxRun];
+    load_run<VEC>(logits, i, v, z);
     float m = -INFINITY, d = 0.0f;
     if (threadIdx.x < n_partials) {
         m = partials[2 * threadIdx.x];
         d = partials[2 * threadIdx.x + 1];
     }
+#pragma unroll
+    for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = softcapped(z[j], softcap);
     block_merge_md(m, d, scratch);
     const float inv_d = 1.0f / d;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < v; i += gridDim.x * blockDim.x)
-        probs[i] = to_half_pinned(expf(softcapped((float)logits[i], softcap) - m) * inv_d);
+    if (i >= v) return;
+    half_t p[kSoftmaxRun];
+#pragma unroll
+    for (uint32_t j = 0; j < kSoftmaxRun; ++j) p[j] = to_half_pinned(expf(z[j] - m) * inv_d);
+    if (VEC && i + kSoftmaxRun <= v) {
+        typedef half_t run_t __attribute__((ext_vector_type(kSoftmaxRun)));
+        *reinterpret_cast<run_t *>(probs + i) = run_t{p[0], p[1], p[2], p[3]};
+    } else {
+#pragma unroll
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j)
+            if (i + j < v) probs[i + j] = p[j];
+    }
+}
+
+template <typename T>
+void launch_softmax(hipStream_t st, const T *logits, float *partials, half_t *probs, uint32_t v, float softcap) {
+    const uint32_t runs = (v + 256 * kSoftmaxRun - 1) / (256 * kSoftmaxRun), blocks = runs < kSoftmaxMaxBlocks ? runs : kSoftmaxMaxBlocks;
+    if (aligned16(logits) && aligned(probs, sizeof(half_t) * kSoftmaxRun)) {
+        hipLaunchKernelGGL((softmax_partials_kernel<true, T>), dim3(blocks), dim3(256), 0, st, logits, partials, v, softcap);
+        hipLaunchKernelGGL((softmax_normalize_kernel<true, T>), dim3(runs), dim3(256), 0, st, logits, partials, blocks, probs, v, softcap);
+    } else {
+        hipLaunchKernelGGL((softmax_partials_kernel<false, T>), dim3(blocks), dim3(256), 0, st, logits, partials, v, softcap);
+        hipLaunchKernelGGL((softmax_normalize_kernel<false, T>), dim3(runs), dim3(256), 0, st, logits, partials, blocks, probs, v, softcap);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------ samplers
@@ -149,158 +202,356 @@ __global__ __launch_bounds__(256) void sample_argmax_kernel(const half_t *probs,
     fold_block_best(sv, si, cells, out_token);
 }
 
-// ---- top-k through sorted tiles
-// A tile is 1024 (value, index) pairs sorted by (value descending, index ascending) with a bitonic network in LDS; its
-// first KEEP pairs go on to the next stage.  Pairs that must never be chosen carry (-inf, 0xFFFFFFFF): slots past the
-// input, NaN and -inf probabilities.
-constexpr uint32_t kTile = 1024;
+// ---- top-k
+// The k best (k <= 256) of v probabilities by (value descending, index ascending) in two launches, without sorting the
+// vocabulary.  fp16 values have 16-bit order-preserving keys, so "the k-th largest" is a binary search over at most 16
+// thresholds, each a count of the elements that reach it (ballots and one block barrier):
+//   1. chunk_max_kernel: the largest key of every 64 consecutive elements (one read of the probabilities by the whole chip);
+//   2. topk_final_kernel, one block: T0 = the k-th largest of the chunk maxima.  At least k elements reach T0, so no element
+//      below it is among the k best: only chunks whose maximum exceeds T0 (fewer than k) matter, and of those whose maximum is
+//      T0 the first k (each holds an element equal to T0, and equal elements are taken by index).  The at most 2 k - 1 chunks
+//      are read again (they are in the L2), their k-th largest key T1 is found the same way, ties at T1 are taken in index
+//      order, and the k survivors are put in order by counting.
+// Both launches are latency, not bandwidth (262144 probabilities are 0.5 MB); sorting every 1024-element tile with a bitonic
+// network and merging the tiles in two more passes took 143 us at 262144, k = 64, where this takes 15.5 us, most of it the second launch.
+// NaN and -inf are never chosen (key 0); -0 ties with 0.
+constexpr uint32_t kTopkThreads = 1024, kTopkWaves = kTopkThreads / kWave;
+constexpr uint32_t kTopkChunk = 64;
+constexpr uint32_t kTopkCachedChunks = 4;                // chunk maxima a thread keeps in registers: 4096 of them, 262144 elements
+constexpr uint32_t kTopkVocabFactor = 4;
+constexpr uint32_t kTopkMaxK = 256;                      // the reference's working set (kSampleTopMaxK)
 
-__device__ __forceinline__ bool pair_better(float lv, uint32_t li, float rv, uint32_t ri) { return lv > rv || (lv == rv && li < ri); }
+__device__ __forceinline__ uint32_t prob_key(uint16_t bits) {
+    if (bits == 0x8000u) bits = 0u;
+    const uint32_t key = (bits & 0x8000u) ? (uint32_t)(uint16_t)~bits : (uint32_t)bits | 0x8000u;
+    const bool usable = (bits & 0x7FFFu) < 0x7C00u || bits == 0x7C00u;      // finite or +inf
+    return usable ? key : 0u;
+}
+__device__ __forceinline__ float key_value(uint32_t key) {
+    const uint16_t bits = (uint16_t)((key & 0x8000u) ? key & 0x7FFFu : ~key);
+    return (float)__builtin_bit_cast(half_t, bits);
+}
 
-__device__ __forceinline__ void sort_tile(float *values, uint32_t *indices) {
-    for (uint32_t width = 2; width <= kTile; width <<= 1) {
-        for (uint32_t stride = width >> 1; stride > 0; stride >>= 1) {
-            __syncthreads();
-            for (uint32_t i = threadIdx.x; i < kTile; i += 256) {
-                const uint32_t partner = i ^ stride;
-                if (partner <= i) continue;
-                const float lv = values[i], rv = values[partner];
-                const uint32_t li = indices[i], ri = indices[partner];
-                const bool descending = (i & width) == 0;
-                const bool swap = descending ? pair_better(rv, ri, lv, li) : pair_better(lv, li, rv, ri);
-                if (swap) {
-                    values[i] = rv;
-                    indices[i] = ri;
-                    values[partner] = lv;
-                    indices[partner] = li;
-                }
+// VEC: probs is 16-byte aligned (a thread's eight elements in one load)
+template <bool VEC>
+__global__ __launch_bounds__(256) void chunk_max_kernel(const uint16_t *probs, uint16_t *chunk_max, uint32_t v) {
+    const uint32_t piece = blockIdx.x * 256 + threadIdx.x, first = piece * 8;
+    uint32_t best = 0;
+    if (VEC && first + 8 <= v) {
+        const u32x4 w = *reinterpret_cast<const u32x4 *>(probs + first);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) best = max(best, max(prob_key((uint16_t)w[i]), prob_key((uint16_t)(w[i] >> 16))));
+    } else {
+#pragma unroll
+        for (uint32_t i = 0; i < 8; ++i)
+            if (first + i < v) best = max(best, prob_key(probs[first + i]));
+    }
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, off, kWave));
+    if ((threadIdx.x & 7) == 0 && first < v) chunk_max[piece >> 3] = (uint16_t)best;
+}
+
+// Sum of a wave-uniform count over the block's waves, in every thread.  `parity` alternates between two calls in a row, so one
+// barrier a call is enough.
+__device__ __forceinline__ uint32_t block_count(uint32_t wave_count, uint32_t (*cells)[kTopkWaves], uint32_t parity) {
+    if ((threadIdx.x & 63) == 0) cells[parity][threadIdx.x >> 6] = wave_count;
+    __syncthreads();
+    uint32_t sum = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < kTopkWaves; ++w) sum += cells[parity][w];
+    return sum;
+}
+
+// A threshold t in [lo, hi) that at least k keys of the block reach: the first one tried that at most `enough` reach, or else the
+// largest (lo when fewer than k keys reach it).  count(t): how many of the wave's keys reach t; reached: how many of the
+// block's reach the result (0 where that was never counted).
+template <typename Count>
+__device__ __forceinline__ uint32_t threshold(uint32_t lo, uint32_t hi, uint32_t k, uint32_t enough, uint32_t (*cells)[kTopkWaves], uint32_t &reached,
+                                              Count count) {
+    uint32_t parity = 0;
+    reached = 0;
+    while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) >> 1;
+        const uint32_t n = block_count(count(mid), cells, parity);
+        parity ^= 1;
+        if (n >= k) {
+            lo = mid;
+            reached = n;
+            if (n <= enough) break;
+        } else {
+            hi = mid;
+        }
+    }
+    __syncthreads();      // the cells are free
+    return lo;
+}
+
+__device__ __forceinline__ uint32_t lanes_before(uint64_t mask) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// table[0..N): exclusive running sum in place, by the first wave; the sum of all goes to *total.  Barriers before and after.
+template <uint32_t N>
+__device__ __forceinline__ void exclusive_scan(uint32_t *table, uint32_t *total) {
+    static_assert(N % kWave == 0, "whole waves");
+    __syncthreads();
+    if (threadIdx.x < kWave) {
+        uint32_t carry = 0;
+#pragma unroll
+        for (uint32_t i = threadIdx.x; i < N; i += kWave) {
+            const uint32_t own = table[i];
+            uint32_t sum = own;
+#pragma unroll
+            for (int off = 1; off < kWave; off <<= 1) {
+                const uint32_t up = (uint32_t)__shfl_up((int)sum, off, kWave);
+                if ((int)threadIdx.x >= off) sum += up;
+            }
+            table[i] = carry + sum - own;
+            carry += (uint32_t)__shfl((int)sum, kWave - 1, kWave);
+        }
+        if (threadIdx.x == 0) *total = carry;
+    }
+    __syncthreads();
+}
+
+// Running sums of `own` over a wave's lanes on top of `carry`, in lane order, one fp32 add per element: lane l holds what a
+// sequential accumulation holds after element l, so a search over the lanes finds exactly the element a sequential walk would
+// stop at.  A lane adds the elements up to its own and zeros from there on.
+__device__ __forceinline__ float running_sums(float own, float carry) {
+    float acc = carry;
+#pragma unroll
+    for (int j = 0; j < kWave; ++j) {
+        const float x = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(own), j));
+        acc += (int)(threadIdx.x & 63) >= j ? x : 0.0f;
+    }
+    return acc;
+}
+
+// The sampler's tail, by one wave: slot 64 j + lane holds candidate number 64 j + lane, best first; only the first k slots (0 < k)
+// count.  Follows the reference's sampler (Metal/Sampling/logit.metal:564-606): the usable prefix ends at the first slot that is
+// empty or not finite; the top-p cut keeps the shortest prefix whose mass (probabilities still carry their full-vocabulary
+// normalisation) reaches top_p; survivors are reweighted by p^(1/T); the draw is the inverse CDF of the seeded xorshift64* uniform.
+// The sums that decide the cut and the draw are accumulated in index order.  Returns the chosen slot.
+template <uint32_t SLOTS>
+__device__ __forceinline__ uint32_t choose_slot(float value[SLOTS], const uint32_t index[SLOTS], uint32_t k, float temperature, float top_p,
+                                                uint64_t seed) {
+    const uint32_t lane = threadIdx.x & 63;
+    auto first = [&](uint32_t none, auto holds) {      // lowest slot below `none` for which holds(j, slot)
+        uint32_t found = none;
+#pragma unroll
+        for (uint32_t j = 0; j < SLOTS; ++j) {
+            const uint64_t m = __ballot(64 * j + lane < none && holds(j));
+            if (m != 0 && found == none) found = 64 * j + (uint32_t)__builtin_ctzll(m);
+        }
+        return found;
+    };
+    uint32_t n = first(k, [&](uint32_t j) { return index[j] == 0xFFFFFFFFu || !__builtin_isfinite(value[j]); });
+    float sum[SLOTS];
+    auto accumulate = [&]() {      // returns the sum of the first n
+        float carry = 0.0f;
+#pragma unroll
+        for (uint32_t j = 0; j < SLOTS; ++j) {
+            sum[j] = carry;
+            if (64 * j < n) {
+                sum[j] = running_sums(64 * j + lane < n ? value[j] : 0.0f, carry);
+                carry = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(sum[j]), kWave - 1));
             }
         }
-    }
-    __syncthreads();
-}
-
-// source: fp16 probabilities (in_values == nullptr) or the pairs of an earlier stage
-__device__ __forceinline__ void load_tile(const half_t *probs, const float *in_values, const uint32_t *in_indices, uint32_t base,
-                                          uint32_t count, float *values, uint32_t *indices) {
-    for (uint32_t i = threadIdx.x; i < kTile; i += 256) {
-        const uint32_t source = base + i;
-        float val = -INFINITY;
-        uint32_t idx = 0xFFFFFFFFu;
-        if (source < count) {
-            val = in_values ? in_values[source] : (float)probs[source];
-            idx = in_values ? in_indices[source] : source;
-            if (!(val > -INFINITY)) {
-                val = -INFINITY;
-                idx = 0xFFFFFFFFu;
-            }
-        }
-        values[i] = val;
-        indices[i] = idx;
-    }
-}
-
-template <uint32_t KEEP>
-__global__ __launch_bounds__(256) void topk_tile_kernel(const half_t *probs, const float *in_values, const uint32_t *in_indices,
-                                                        float *out_values, uint32_t *out_indices, uint32_t count) {
-    __shared__ float values[kTile];
-    __shared__ uint32_t indices[kTile];
-    load_tile(probs, in_values, in_indices, blockIdx.x * kTile, count, values, indices);
-    sort_tile(values, indices);
-    for (uint32_t i = threadIdx.x; i < KEEP; i += 256) {
-        out_values[blockIdx.x * KEEP + i] = values[i];
-        out_indices[blockIdx.x * KEEP + i] = indices[i];
-    }
-}
-
-// Running sums of values[0..n) in index order, one fp32 add per element (thread 0; n <= 256), left in sums[] for the whole
-// block: sums[i] is what a sequential accumulation holds after element i, so a search over sums[] finds exactly the element a
-// sequential walk would stop at.  Ends with a barrier.
-__device__ __forceinline__ void running_sums(const float *values, uint32_t n, float *sums) {
-    if (threadIdx.x == 0) {
-        float acc = 0.0f;
-        for (uint32_t i = 0; i < n; ++i) {
-            acc += values[i];
-            sums[i] = acc;
-        }
-    }
-    __syncthreads();
-}
-
-// Smallest candidate any thread of the block offers (threads without one offer `none`), through one LDS word.  Two barriers.
-__device__ __forceinline__ uint32_t block_first(uint32_t candidate, uint32_t none, uint32_t *word) {
-    if (threadIdx.x == 0) *word = none;
-    __syncthreads();
-    if (candidate < none) atomicMin(word, candidate);
-    __syncthreads();
-    const uint32_t found = *word;
-    __syncthreads();
-    return found;
-}
-
-// Last tile: sort, then thread t looks after slot t of the k best (k <= 256 = the block).  Results follow the reference's
-// sampler (Metal/Sampling/logit.metal:564-606): the usable prefix ends at the first slot that is padding or not finite; the
-// top-p cut keeps the shortest prefix whose mass (probabilities still carry their full-vocabulary normalisation) reaches top_p;
-// survivors are reweighted by p^(1/T); the draw is the inverse CDF of the seeded xorshift64* uniform.  The sums that decide
-// the cut and the draw are accumulated in index order (running_sums); the slots are tested and reweighted side by side.
-__global__ __launch_bounds__(256) void topk_final_kernel(const half_t *probs, const float *in_values, const uint32_t *in_indices, uint32_t count,
-                                                         uint32_t k, float temperature, float top_p, uint64_t seed, uint32_t *out_token) {
-    __shared__ float values[kTile];
-    __shared__ uint32_t indices[kTile];
-    __shared__ float sums[256];
-    __shared__ uint32_t word;
-    load_tile(probs, in_values, in_indices, 0, count, values, indices);
-    sort_tile(values, indices);
-    const uint32_t t = threadIdx.x;
-    const bool unusable = t < k && (indices[t] == 0xFFFFFFFFu || !__builtin_isfinite(values[t]));
-    uint32_t n = block_first(unusable ? t : k, k, &word);
+        return carry;
+    };
     if (top_p > 0.0f && top_p < 1.0f) {
-        running_sums(values, n, sums);
-        n = block_first(t < n && sums[t] >= top_p ? t + 1 : n, n, &word);
+        (void)accumulate();
+        const uint32_t last = first(n, [&](uint32_t j) { return sum[j] >= top_p; });
+        n = last < n ? last + 1 : n;
     }
     if (temperature != 1.0f) {
-        if (t < n) values[t] = powf(values[t], 1.0f / temperature);
-        __syncthreads();
+#pragma unroll
+        for (uint32_t j = 0; j < SLOTS; ++j)
+            if (64 * j + lane < n) value[j] = powf(value[j], 1.0f / temperature);
     }
-    running_sums(values, n, sums);
+    const float mass = accumulate();
     uint64_t rng = seed;
     (void)xorshift64(rng);
-    const float u = uniform01(rng) * (n > 0 ? sums[n - 1] : 0.0f);
-    const uint32_t slot = block_first(t < n && u <= sums[t] ? t : n, n, &word);
-    if (t == 0) {
-        const uint32_t token = indices[slot < n ? slot : 0];
-        out_token[0] = token == 0xFFFFFFFFu ? 0u : token;
+    const float u = uniform01(rng) * mass;
+    const uint32_t slot = first(n, [&](uint32_t j) { return u <= sum[j]; });
+    return slot < n ? slot : 0;
+}
+
+// One block.  EPT: elements a thread looks after (EPT * 1024 >= (2 k - 1) * 64, or >= v where every element is looked at and
+// chunk_max is null).
+template <uint32_t EPT>
+__global__ __launch_bounds__(kTopkThreads) void topk_final_kernel(const uint16_t *probs, const uint16_t *chunk_max, uint32_t v, uint32_t k,
+                                                                  float temperature, float top_p, uint64_t seed, uint32_t *out_token) {
+    constexpr uint32_t kMaxK = EPT <= 8 ? 64 : kTopkMaxK, kRounds = kTopkCachedChunks;
+    constexpr uint32_t kChunkCapacity = EPT * kTopkThreads / kTopkChunk;      // 128 / 512: at least 2 k
+    __shared__ uint32_t cells[2][kTopkWaves];
+    __shared__ uint32_t table[EPT * kTopkWaves], taken_table[kRounds * kTopkWaves];
+    __shared__ uint32_t chunk_list[kChunkCapacity];
+    __shared__ uint64_t best[kMaxK];
+    __shared__ uint32_t ranks[kMaxK];
+    __shared__ float values[kMaxK];
+    __shared__ uint32_t indices[kMaxK];
+    __shared__ uint32_t word, total;
+    const uint32_t t = threadIdx.x, wave = t >> 6;
+    uint32_t listed = 0, floor_key = 1;      // chunks to look into; a key that at least k elements reach, if k are usable
+    if (t == 0) total = 0;
+    if (t < kMaxK) {
+        ranks[t] = 0;
+        values[t] = -INFINITY;
+        indices[t] = 0xFFFFFFFFu;
+        best[t] = 0;
+    }
+    if (chunk_max) {
+        const uint32_t chunks = (v + kTopkChunk - 1) / kTopkChunk, rounds = (chunks + kTopkThreads - 1) / kTopkThreads;
+        auto maximum = [&](uint32_t r) { return r * kTopkThreads + t < chunks ? (uint32_t)chunk_max[r * kTopkThreads + t] : 0u; };
+        uint32_t cached[kRounds];
+#pragma unroll
+        for (uint32_t r = 0; r < kRounds; ++r) cached[r] = maximum(r);
+        uint32_t reached;
+        const uint32_t t0 = threshold(1, 0x10000u, k, kChunkCapacity, cells, reached, [&](uint32_t mid) {
+            uint32_t n = 0;
+#pragma unroll
+            for (uint32_t r = 0; r < kRounds; ++r) n += (uint32_t)__popcll(__ballot(cached[r] >= mid));
+            for (uint32_t r = kRounds; r < rounds; ++r) n += (uint32_t)__popcll(__ballot(maximum(r) >= mid));
+            return n;
+        });
+        floor_key = t0;
+        const bool few = reached <= kChunkCapacity;      // every chunk that reaches T0 fits the list
+        // the chosen chunks in index order: those that reach T0, or all above T0 and the first k at T0
+        uint32_t ties = 0;
+        for (uint32_t r0 = 0; r0 < rounds; r0 += kRounds) {
+            uint32_t m[kRounds];
+            bool take[kRounds];
+#pragma unroll
+            for (uint32_t r = 0; r < kRounds; ++r) {
+                m[r] = r0 == 0 ? cached[r] : maximum(r0 + r);
+                take[r] = m[r] >= t0;
+            }
+            if (!few) {
+#pragma unroll
+                for (uint32_t r = 0; r < kRounds; ++r) {
+                    const uint64_t eq = __ballot(m[r] == t0);
+                    if ((t & 63) == 0) taken_table[r * kTopkWaves + wave] = (uint32_t)__popcll(eq);
+                }
+                exclusive_scan<kRounds * kTopkWaves>(taken_table, &word);
+#pragma unroll
+                for (uint32_t r = 0; r < kRounds; ++r) {
+                    const uint64_t eq = __ballot(m[r] == t0);
+                    take[r] = m[r] > t0 || (m[r] == t0 && ties + taken_table[r * kTopkWaves + wave] + lanes_before(eq) < k);
+                }
+                ties += word;
+                __syncthreads();
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < kRounds; ++r) {
+                const uint64_t mask = __ballot(take[r]);
+                if ((t & 63) == 0) taken_table[r * kTopkWaves + wave] = (uint32_t)__popcll(mask);
+            }
+            exclusive_scan<kRounds * kTopkWaves>(taken_table, &word);
+#pragma unroll
+            for (uint32_t r = 0; r < kRounds; ++r) {
+                const uint64_t mask = __ballot(take[r]);
+                if (take[r]) chunk_list[listed + taken_table[r * kTopkWaves + wave] + lanes_before(mask)] = (r0 + r) * kTopkThreads + t;
+            }
+            listed += word;
+            __syncthreads();
+        }
+    }
+    auto element = [&](uint32_t j) {      // slot j of this thread -> index in probs; slots ascend by index
+        const uint32_t slot = j * kTopkThreads + t;
+        if (!chunk_max) return slot;
+        return slot / kTopkChunk < listed ? chunk_list[slot / kTopkChunk] * kTopkChunk + slot % kTopkChunk : v;
+    };
+    uint32_t key[EPT];
+#pragma unroll
+    for (uint32_t j = 0; j < EPT; ++j) {
+        const uint32_t i = element(j);
+        key[j] = i < v ? (uint32_t)probs[i] : 0xFFFFu;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < EPT; ++j) key[j] = prob_key((uint16_t)key[j]);      // 0xFFFF is a NaN: never chosen
+    uint32_t reached;
+    const uint32_t t1 = threshold(floor_key, 0x10000u, k, k, cells, reached, [&](uint32_t mid) {
+        uint32_t n = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < EPT; ++j) n += (uint32_t)__popcll(__ballot(key[j] >= mid));
+        return n;
+    });
+    // exactly the keys that reach T1 where k of them do; otherwise everything above T1 and the first of those at T1: `table` counts
+    // the ties of every (j, wave), in index order
+    uint32_t ties_wanted = 0xFFFFFFFFu;
+    if (reached != k) {
+        uint32_t above = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < EPT; ++j) {
+            const uint64_t eq = __ballot(key[j] == t1);
+            above += (uint32_t)__popcll(__ballot(key[j] > t1));
+            if ((t & 63) == 0) table[j * kTopkWaves + wave] = (uint32_t)__popcll(eq);
+        }
+        ties_wanted = k - block_count(above, cells, 0);
+        exclusive_scan<EPT * kTopkWaves>(table, &word);
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < EPT; ++j) {
+        bool take = key[j] >= t1;
+        if (reached != k) {
+            const uint64_t eq = __ballot(key[j] == t1);
+            take = key[j] > t1 || (key[j] == t1 && table[j * kTopkWaves + wave] + lanes_before(eq) < ties_wanted);
+        }
+        if (take) best[atomicAdd(&total, 1u)] = ((uint64_t)key[j] << 32) | (uint64_t)(0xFFFFFFFFu - element(j));
+    }
+    __syncthreads();
+    // a candidate's place is the number of better ones: candidate t % kMaxK against a share of the list (empty places hold 0)
+    {
+        constexpr uint32_t kShares = kTopkThreads / kMaxK, kShare = kMaxK / kShares;
+        const uint64_t own = best[t % kMaxK];
+        uint32_t better = 0;
+#pragma unroll 4
+        for (uint32_t j = 0; j < kShare; ++j) better += best[(t / kMaxK) * kShare + j] > own ? 1u : 0u;
+        if (better) atomicAdd(&ranks[t % kMaxK], better);
+    }
+    __syncthreads();
+    if (t < total) {
+        values[ranks[t]] = key_value((uint32_t)(best[t] >> 32));
+        indices[ranks[t]] = 0xFFFFFFFFu - (uint32_t)best[t];
+    }
+    __syncthreads();
+    if (t < kWave) {
+        constexpr uint32_t kSlots = kMaxK / kWave;
+        float value[kSlots];
+        uint32_t index[kSlots];
+#pragma unroll
+        for (uint32_t j = 0; j < kSlots; ++j) {
+            value[j] = values[64 * j + t];
+            index[j] = indices[64 * j + t];
+        }
+        const uint32_t slot = choose_slot<kSlots>(value, index, k, temperature, top_p, seed);
+        if (t == 0) {
+            const uint32_t token = indices[slot];
+            out_token[0] = token == 0xFFFFFFFFu ? 0u : token;
+        }
     }
 }
 
-// Wrapper-owned scratch of the samplers: [argmax cells + ticket | softmax partials | two pair buffers].
+// Wrapper-owned scratch of the samplers: [argmax cells + ticket | softmax partials | chunk maxima].
 struct SampleScratch {
     unsigned long long *cells;
     float *partials;
-    float *values[2];
-    uint32_t *indices[2];
+    uint16_t *chunk_max;
 };
 
 constexpr size_t kCellBytes = (kHeadCells + 1) * sizeof(unsigned long long);
 constexpr size_t kPartialBytes = kSoftmaxMaxBlocks * 2 * sizeof(float);
 
-size_t sample_need(uint32_t pair_capacity) {
-    const size_t pairs = ((size_t)pair_capacity + 255) / 256 * 256;
-    return kCellBytes + kPartialBytes + pairs * 16;
-}
+size_t sample_need(size_t elements) { return kCellBytes + kPartialBytes + (elements / kTopkChunk + 1) * sizeof(uint16_t); }
 
-int32_t sample_scratch(tf_ctx *ctx, uint32_t pair_capacity, SampleScratch &out) {
-    const size_t need = sample_need(pair_capacity);
+int32_t sample_scratch(tf_ctx *ctx, size_t elements, SampleScratch &out) {
+    const size_t need = sample_need(elements);
     if (ctx->sample_scratch_bytes < need) return scratch_too_small(ctx, "sampler", need, ctx->sample_scratch_bytes);
     uint8_t *base = static_cast<uint8_t *>(ctx->sample_scratch);
-    const size_t have_pairs = (ctx->sample_scratch_bytes - kCellBytes - kPartialBytes) / 16;
     out.cells = reinterpret_cast<unsigned long long *>(base);
     out.partials = reinterpret_cast<float *>(base + kCellBytes);
-    uint8_t *pair_base = base + kCellBytes + kPartialBytes;
-    out.values[0] = reinterpret_cast<float *>(pair_base);
-    out.values[1] = reinterpret_cast<float *>(pair_base + have_pairs * 4);
-    out.indices[0] = reinterpret_cast<uint32_t *>(pair_base + have_pairs * 8);
-    out.indices[1] = reinterpret_cast<uint32_t *>(pair_base + have_pairs * 12);
+    out.chunk_max = reinterpret_cast<uint16_t *>(base + kCellBytes + kPartialBytes);
     return TF_OK;
 }
 
@@ -312,35 +563,25 @@ uint32_t spread_blocks(const tf_ctx *ctx, uint32_t v, uint32_t cap) {
     return blocks > 0 ? blocks : 1;
 }
 
-// the k best of probs[0..v) -> one token; k <= 256
+// the k best of probs[0..v) -> one token; k <= 256.  A vocabulary that one block can hold in registers takes the second launch
+// alone.
 int32_t launch_truncating_sampler(tf_ctx *ctx, hipStream_t st, const half_t *probs, uint32_t v, uint32_t k, float temperature, float top_p,
                                   uint64_t seed, uint32_t *out_token, const char *who) {
-    if (v <= kTile) {
-        hipLaunchKernelGGL(topk_final_kernel, dim3(1), dim3(256), 0, st, probs, (const float *)nullptr, (const uint32_t *)nullptr, v, k, temperature,
-                           top_p, seed, out_token);
-        return check_launch(ctx, who);
+    const uint16_t *bits = reinterpret_cast<const uint16_t *>(probs);
+    const uint32_t most = (k <= 64 ? 8u : 32u) * kTopkThreads;      // elements the final block looks at: (2 k - 1) chunks fit
+    uint16_t *chunk_max = nullptr;
+    if (v > most) {
+        SampleScratch sc;
+        // the limits admit vocabularies up to max_vocab, four times that for k <= 64
+        const int32_t rc = sample_scratch(ctx, (k <= 64 ? 1u : kTopkVocabFactor) * (size_t)v, sc);
+        if (rc != TF_OK) return rc;
+        chunk_max = sc.chunk_max;
+        const dim3 grid((v + 2047) / 2048);
+        if (aligned16(probs)) hipLaunchKernelGGL(chunk_max_kernel<true>, grid, dim3(256), 0, st, bits, chunk_max, v);
+        else hipLaunchKernelGGL(chunk_max_kernel<false>, grid, dim3(256), 0, st, bits, chunk_max, v);
     }
-    const uint32_t keep = k <= 64 ? 64u : 256u;
-    const uint32_t tiles0 = (v + kTile - 1) / kTile;
-    SampleScratch sc;
-    const int32_t rc = sample_scratch(ctx, tiles0 * keep, sc);
-    if (rc != TF_OK) return rc;
-    uint32_t count = v, tiles = tiles0;
-    int cur = 0;
-    bool first = true;
-    while (true) {
-        const float *iv = first ? nullptr : sc.values[cur ^ 1];
-        const uint32_t *ii = first ? nullptr : sc.indices[cur ^ 1];
-        if (keep == 64) hipLaunchKernelGGL(topk_tile_kernel<64>, dim3(tiles), dim3(256), 0, st, probs, iv, ii, sc.values[cur], sc.indices[cur], count);
-        else hipLaunchKernelGGL(topk_tile_kernel<256>, dim3(tiles), dim3(256), 0, st, probs, iv, ii, sc.values[cur], sc.indices[cur], count);
-        count = tiles * keep;
-        first = false;
-        if (count <= kTile) break;
-        tiles = (count + kTile - 1) / kTile;
-        cur ^= 1;
-    }
-    hipLaunchKernelGGL(topk_final_kernel, dim3(1), dim3(256), 0, st, probs, sc.values[cur], sc.indices[cur], count, k, temperature, top_p, seed,
-                       out_token);
+    if (k <= 64) hipLaunchKernelGGL(topk_final_kernel<8>, dim3(1), dim3(kTopkThreads), 0, st, bits, chunk_max, v, k, temperature, top_p, seed, out_token);
+    else hipLaunchKernelGGL(topk_final_kernel<32>, dim3(1), dim3(kTopkThreads), 0, st, bits, chunk_max, v, k, temperature, top_p, seed, out_token);
     return check_launch(ctx, who);
 }
 
@@ -348,8 +589,7 @@ int32_t launch_truncating_sampler(tf_ctx *ctx, hipStream_t st, const half_t *pro
 
 namespace tfk {
 
-// the truncating samplers keep up to 256 candidates of every 1024-element tile of the first pass
-size_t sample_scratch_bytes_for(uint32_t vocab) { return sample_need((vocab + kTile - 1) / kTile * 256u); }
+size_t sample_scratch_bytes_for(uint32_t vocab) { return sample_need(kTopkVocabFactor * (size_t)vocab); }
 size_t sample_scratch_clear_bytes() { return kCellBytes; }
 
 }  // namespace tfk
@@ -404,17 +644,9 @@ int32_t tf_logit_softcap_softmax(tf_ctx *ctx, tf_stream stream, const void *logi
     const int32_t rc = sample_scratch(ctx, 0, sc);
     if (rc != TF_OK) return rc;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    const uint32_t blocks = spread_blocks(ctx, v, kSoftmaxMaxBlocks);
     half_t *ph = static_cast<half_t *>(probs);
-    if (logits_dtype == TF_FP16) {
-        const half_t *lh = static_cast<const half_t *>(logits);
-        hipLaunchKernelGGL(softmax_partials_kernel<half_t>, dim3(blocks), dim3(256), 0, st, lh, sc.partials, v, softcap);
-        hipLaunchKernelGGL(softmax_normalize_kernel<half_t>, dim3(spread_blocks(ctx, v, 1024)), dim3(256), 0, st, lh, sc.partials, blocks, ph, v, softcap);
-    } else {
-        const float *lf = static_cast<const float *>(logits);
-        hipLaunchKernelGGL(softmax_partials_kernel<float>, dim3(blocks), dim3(256), 0, st, lf, sc.partials, v, softcap);
-        hipLaunchKernelGGL(softmax_normalize_kernel<float>, dim3(spread_blocks(ctx, v, 1024)), dim3(256), 0, st, lf, sc.partials, blocks, ph, v, softcap);
-    }
+    if (logits_dtype == TF_FP16) launch_softmax(st, static_cast<const half_t *>(logits), sc.partials, ph, v, softcap);
+    else launch_softmax(st, static_cast<const float *>(logits), sc.partials, ph, v, softcap);
     return check_launch(ctx, "logit_softcap_softmax");
 }
 
