@@ -135,6 +135,25 @@ def test_qkv_epilogue_block_equals_tokens_one_by_one(tokens, hq, hkv, d, start, 
         same_up_to_rounding(host(fused, np.uint16), host(separate, np.uint16), ulps=1, share=0.01)
 
 
+@pytest.mark.parametrize("tokens,hq,hkv,d,pad", [(2100, 5, 1, 128, 8), (2050, 13, 2, 256, 8), (2050, 13, 2, 128, 9), (8200, 3, 1, 64, 3)])
+def test_qkv_epilogue_of_many_tokens_equals_tokens_one_by_one(tokens, hq, hkv, d, pad):
+    """Blocks large enough for two, four and eight heads a wave, head counts that are no multiple of what a block takes, rows on
+    and off the vector path's alignment."""
+    q, qw, q_stride = block(tokens, hq, d, pad, 0x7B50 + d)
+    kk, kw, kv_stride = block(tokens, hkv, d, pad, 0x7B51 + d)
+    vv = block(tokens, hkv, d, pad, 0x7B52 + d)[0]
+    k = ctx()
+    d_qw, d_kw = dev(qw), dev(kw)
+    bq, bk, bv, rq, rk, rv = (dev(a) for a in (q, kk, vv, q, kk, vv))
+    k.check(k.lib.tf_prefill_qkv_epilogue_block(k.handle, None, bq.data_ptr(), 0, bk.data_ptr(), 0, bv.data_ptr(), 0, d_qw.data_ptr(), 0,
+                                                d_kw.data_ptr(), 0, 77, tokens, d, hq, hkv, q_stride, kv_stride, 1e4, d // 2, EPS))
+    for t in range(tokens):
+        k.check(k.lib.tf_fused_qkv_epilogue(k.handle, None, rq.data_ptr(), t * q_stride * 2, rk.data_ptr(), t * kv_stride * 2, rv.data_ptr(),
+                                            t * kv_stride * 2, d_qw.data_ptr(), 0, d_kw.data_ptr(), 0, d, hq, hkv, 77 + t, 1e4, d // 2, EPS))
+    for got, one_by_one in ((bq, rq), (bk, rk), (bv, rv)):
+        assert np.array_equal(host(got, np.uint16), host(one_by_one, np.uint16))
+
+
 def test_contracts():
     k = ctx()
     lib, h = k.lib, k.handle
