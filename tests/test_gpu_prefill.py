@@ -635,6 +635,43 @@ def test_int4_qmm_on_matrix_cores_with_scales_below_fp16_normal_range(m, n, k, l
     assert tfo.rel_error(got.astype(np.float32), want) <= 1e-3
 
 
+@pytest.mark.parametrize("m,n,k,fp16_scales,shift", [
+    (1, 31, 1024, False, 0), (32, 32, 1024, False, 0), (33, 70, 1088, False, 0),     # 32 x 32 tiles: one row, a full tile, remainders and an odd number of groups
+    (53, 2816, 2112, True, 0), (31, 40, 4160, False, 2), (40, 33, 8192, True, 0),    # an odd number of groups over eight waves; more than 4096; rows stored value by value
+    (70, 2752, 1024, False, 0), (130, 2720, 4160, True, 0),                          # 64 x 32 tiles (258 and 425 tiles of 32 x 32)
+    (65, 4130, 1088, False, 0), (129, 4100, 4224, False, 2),                         # 64 x 64 tiles (258 and 387 tiles of 64 x 32), and with wide scale areas
+])
+def test_int4_qmm_with_the_contraction_split_between_waves(m, n, k, fp16_scales, shift):
+    # against 64-bit sums of the exact weights; the bound at the end is what rounding weights and outputs to fp16 amounts to
+    rng = np.random.default_rng(m * 10007 + n + k)
+    groups = k // 64
+    W = rng.integers(0, 256, (n, k // 2), dtype=np.uint8)
+    s = rng.uniform(0.004, 0.02, (n, groups)).astype(np.float32)
+    b = (-7.5 * s * rng.uniform(0.5, 1.5, (n, groups))).astype(np.float32)
+    if fp16_scales:
+        S, B = s.astype(np.float16).view(np.uint16), b.astype(np.float16).view(np.uint16)
+        sf, bf = s.astype(np.float16).astype(np.float64), b.astype(np.float16).astype(np.float64)
+    else:
+        S, B = tfo.bf16_bits_array(s).reshape(n, groups), tfo.bf16_bits_array(b).reshape(n, groups)
+        sf, bf = (tfo.bf16_array_to_float(a.ravel()).reshape(n, groups).astype(np.float64) for a in (S, B))
+    x = tfo.to_f16_bits(rng.standard_normal(m * k).astype(np.float32))
+    kk = ctx()
+    y = zeros_bytes(m * n * 2 + 64, 0xEE)
+    dW, dS, dB, dx = dev(W), dev(S), dev(B), dev(x)
+    kk.check(kk.lib.tf_int4_qmm(kk.handle, None, dW.data_ptr(), 0, dS.data_ptr(), 0, dB.data_ptr(), 0, dx.data_ptr(), 0, y.data_ptr(), shift, m, n, k,
+                                tfk.TF_FP16 if fp16_scales else tfk.TF_BF16))
+    raw = host(y, np.uint8)
+    assert np.all(raw[:shift] == 0xEE) and np.all(raw[shift + m * n * 2:] == 0xEE)
+    got = raw[shift:shift + m * n * 2].view(np.float16).reshape(m, n).astype(np.float64)
+    nib = np.stack([W & 0xF, W >> 4], axis=2).reshape(n, k).astype(np.float64)
+    wf = nib * np.repeat(sf, 64, axis=1) + np.repeat(bf, 64, axis=1)
+    exact = tfo.from_f16_bits(x).reshape(m, k).astype(np.float64) @ wf.T
+    # neighbouring fp16 numbers are at most 2^-10 of their size apart, so a weight's rounding has a deviation of at most 2^-10 / sqrt(12) of
+    # it; roundings are independent, so the sum's deviation is that of sqrt(sum of (x w)^2); six deviations and the output's own rounding
+    bound = 6 * 2.0 ** -10 / np.sqrt(12) * np.sqrt((tfo.from_f16_bits(x).reshape(m, k).astype(np.float64) ** 2) @ (wf ** 2).T) + 2.0 ** -11 * np.abs(exact)
+    assert np.all(np.abs(got - exact) <= bound), float(np.max(np.abs(got - exact) / bound))
+
+
 def test_int4_qmm_unavailable_and_exact_variant():
     W, S, B, x = mpp_inputs(8, 64, 128)
     kk = ctx()

@@ -79,4 +79,15 @@ constexpr int kQuadMaxD = 3072, kQuadMaxF = 1024;
 int32_t launch_grouped_quad(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const tf_expert_offsets &off, const ChunkList &cl,
                             uint32_t n_chunks_upper, const GroupedGeom &g, tf_dtype sd, uint32_t stream_pairs);
 
+// Dense products whose waves split the contraction (tf_qmm_split.hip).  qmm_split_variant: kSplitNone where the 128 x 256 tiles are the
+// better kernel, otherwise what launch_qmm_split is to be given; operands as qmm_operands_ok() demands.
+enum { kSplitNone = 0, kSplit32x32, kSplit64x32, kSplit64x64 };
+int qmm_split_variant(int m, int n, int k, long ldx);
+int32_t launch_qmm_split(tf_ctx *ctx, hipStream_t st, int variant, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
+                         half_t *y, long ldy, int m, int n, int k, tf_dtype sd);
+// the same for a gate and an up matrix with GeGLU
+bool geglu_split_ok(const tf_projection *gate, long ldx);
+int32_t launch_geglu_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const half_t *x, long ldx, half_t *a_out,
+                           long lda, int m, tf_dtype sd);
+
 }  // namespace tfk

@@ -513,10 +513,15 @@ int32_t launch_grouped_down_mfma(tf_ctx *ctx, hipStream_t st, const ExpertTable 
 namespace {
 
 // Y[m, n] = X[m, k] . W[n, k]^T on the matrix cores.  Operands as qmm_operands_ok() demands; ldx / ldy in halves.
-// 128-row tiles even when they leave compute units idle (144 blocks at 2048 x 2112): 64-row blocks, twice as many, repeat
-// each weight tile's dequantisation and measured slower (0.18 ms against 0.155 ms for the three shared-expert GEMMs).
+// Products that fill few compute units with 128-row tiles go to the split kernels (qmm_split_variant).  From there on 128-row
+// tiles even when they leave compute units idle (144 blocks at 2048 x 2112): 64-row blocks, twice as many, repeat each weight tile's
+// dequantisation and measured slower (0.18 ms against 0.155 ms for the three shared-expert GEMMs).
 int32_t launch_qmm_dense(tf_ctx *ctx, hipStream_t st, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
-                         half_t *y, long ldy, int m, int n, int k, tf_dtype sd) {
+                         half_t *y, long ldy, int m, int n, int k, tf_dtype sd, bool tiles_only = false) {
+    if (!tiles_only) {
+        const int variant = qmm_split_variant(m, n, k, ldx);
+        if (variant != kSplitNone) return launch_qmm_split(ctx, st, variant, w, s, b, x, ldx, y, ldy, m, n, k, sd);
+    }
     const dim3 grid(dense_grid((uint32_t)(m + kQmmBM - 1) / kQmmBM, (uint32_t)(n + kQmmBN - 1) / kQmmBN));
     const DenseArgs a = dense_args(w, s, b, x, ldx, y, ldy, m, n, k);
     if (a.rows_vectorizable) {
@@ -552,6 +557,9 @@ int32_t shared_block_acts(tf_ctx *ctx, size_t halves, half_t *&out) {
 }
 
 constexpr uint32_t kSharedBlockMinRows = 8;   // fewer rows go through the single-row chain, bit-identical to decode
+// Up to here the shared expert's gate / up and down go to the split kernels (53 rows of 2112 x 2816: 11 + 8 us against 27 + 22 us in
+// launches of their own); from five pairs an expert on (80 tokens of top 8 among 128) its tiles ride in the grouped launches.
+constexpr uint32_t kSharedSplitMaxRows = 79;
 
 // ---- 8-bit projections over a block of rows ----------------------------------------------------------------------
 // Y[M, N] = X[M, K] . W[N, K]^T on the matrix cores with the 8-bit weights expanded on the way into the instruction,
@@ -757,8 +765,10 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
                       up->scales_offset % 2 == 0 && up->biases_offset % 2 == 0 && down->scales_offset % 2 == 0 && down->biases_offset % 2 == 0;
     const bool block_path = weight_bits == 4 && pointers && even && query_count >= kSharedBlockMinRows && (scale_dtype == TF_BF16 || scale_dtype == TF_FP16) &&
                             qmm_operands_ok(gw, xp, x_stride_elements, (int)d) && aligned16(uw) && aligned16(dw) &&
-                            intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX && geglu_arrays_near(gate, up);
-    if (plan && !block_path) return TF_OK;
+                            intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX &&
+                            geglu_arrays_near(gate, up);
+    const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);
+    if (plan && (!block_path || split)) return TF_OK;
     if (weight_bits == 8 && pointers && even && query_count >= 2) {
         // 8-bit projections.  Up to kShared8MfmaMinRows - 1 rows: rows in groups against each weight row, bit-identical to the
         // rows one by one.  From there on the matrix cores: every weight is rounded to fp16 as half(q s + b) first (the
@@ -802,10 +812,12 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
         *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count};
         return TF_OK;
     }
-    rc = launch_qmm_dense_geglu(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype);
+    rc = split ? launch_geglu_split(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype)
+               : launch_qmm_dense_geglu(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype);
     if (rc != TF_OK) return rc;
+    // a block that may ride in the grouped launches takes the tiles here too: the same bits either way
     return launch_qmm_dense(ctx, st, dw, at(down->scales, down->scales_offset), at(down->biases, down->biases_offset), acts, (long)intermediate,
-                            yp, (long)y_stride_elements, (int)query_count, (int)d, (int)intermediate, scale_dtype);
+                            yp, (long)y_stride_elements, (int)query_count, (int)d, (int)intermediate, scale_dtype, !split);
 }
 
 }  // namespace
