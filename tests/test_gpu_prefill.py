@@ -393,6 +393,33 @@ def test_quad_kernels_long_chunks_and_row_widths(T, E, d, f):
     check_against_oracle(r, T, d, f, top_k, abs_tol=1e-3 * max(1.0, scale))
 
 
+@pytest.mark.parametrize("T,E,run", [(75, 128, 1), (40, 128, 3), (31, 128, 128), (20, 40, 9)])
+def test_quad_kernels_share_out_any_work_list(T, E, run):
+    # The blocks share out batches of up to eight pairs (more than 512 chunks, or more batches than blocks: whole chunks).  A pair's sums do
+    # not depend on whom it shares a batch with, so however the runs are cut the outputs are those of the device grouping's list.
+    d, f, top_k = 128, 64, 8
+    r = resident_pipeline(T, E, d, f, top_k, 0x4A00 + T + run, zipf=True, from_router=False)
+    n = T * top_k
+    assert n < 5 * E
+    pairs = r["sorted_pairs"]
+    chunks, at = [], 0
+    while at < n:
+        end = at
+        while end < n and end - at < run and pairs["expert"][end] == pairs["expert"][at]:
+            end += 1
+        chunks.append((int(pairs["expert"][at]), at, end - at))
+        at = end
+    assert (len(chunks) > 512) == (run == 1)
+    k = ctx()
+    koff = tfk.ExpertOffsets(*r["off"].as_tuple())
+    d_pool, d_hidden, d_pairs, d_chunks, d_n = dev(r["pool"]), dev(r["hidden"]), dev(pairs.view(np.uint32)), dev(np.array(chunks, np.uint32)), dev(np.array([len(chunks)], np.uint32))
+    acts, partials = zeros_bytes(n * f * 2), zeros_bytes(n * d * 2)
+    k.check(k.lib.tf_prefill_grouped_routed_moe_resident(k.handle, None, d_hidden.data_ptr(), 0, d, d_pairs.data_ptr(), d_chunks.data_ptr(), d_n.data_ptr(),
+                                                         len(chunks), n, d_pool.data_ptr(), r["stride"], E, C.byref(koff), acts.data_ptr(),
+                                                         partials.data_ptr(), d, f, top_k, tfk.TF_BF16))
+    assert np.array_equal(host(partials, np.uint16, n * d), r["partials"])
+
+
 @pytest.mark.parametrize("T,E,d,f,fp16_scales,pad", [(3, 16, 1536, 128, False, 0), (5, 64, 2048, 256, True, 8), (2, 32, 4096, 64, False, 0),
                                                      (7, 128, 2304, 192, True, 24), (4, 12, 2816, 1024, False, 16)])
 def test_few_tokens_in_one_call_other_row_widths_and_fp16_scales(T, E, d, f, fp16_scales, pad):

@@ -78,23 +78,98 @@ __device__ __forceinline__ uint32_t quad_chunk_count(const ChunkList &cl, uint32
     return uniform_u32(min(cl.dev ? *cl.dev_n : cl.n, n_chunks_upper));
 }
 
-// The tiles of all chunks, in chunk order, are shared out over the blocks of a launch, which has as many blocks as the
-// compute units hold at once.  Few chunks: every chunk gets the same number of blocks, and the few blocks left over idle.
-// Many chunks: the tiles are split evenly, and a block's span may end in one chunk and go on in the next (it then sets up
-// twice, which only pays when whole blocks per chunk would leave many blocks idle).
-constexpr uint32_t kQuadMinBlocksPerChunk = 8;
-__device__ __forceinline__ void quad_span(uint32_t n_chunks, uint32_t tiles_per_chunk, uint32_t &lo, uint32_t &hi) {
-    const uint32_t per_chunk = n_chunks ? gridDim.x / n_chunks : 0u;
-    if (per_chunk >= kQuadMinBlocksPerChunk) {
-        const uint32_t chunk = blockIdx.x / per_chunk, part = blockIdx.x - chunk * per_chunk;
-        const bool idle = chunk >= n_chunks;
-        lo = idle ? 0u : chunk * tiles_per_chunk + tiles_per_chunk * part / per_chunk;
-        hi = idle ? 0u : chunk * tiles_per_chunk + tiles_per_chunk * (part + 1) / per_chunk;
-    } else {
-        const uint64_t total = (uint64_t)n_chunks * tiles_per_chunk;
-        lo = (uint32_t)(total * blockIdx.x / gridDim.x);
-        hi = (uint32_t)(total * (blockIdx.x + 1) / gridDim.x);
+// The work of a call is cut into units: a unit is one batch of a chunk, up to max_pairs of its pairs (what the LDS image holds)
+// against all of its expert's tiles.  A popular expert's chunk is many units: given the same number of blocks as every other chunk, as
+// it once was, its blocks went over the expert's weights once per batch one after the other and set the launch's time (16 tokens: gate / up
+// 45 us; 53 tokens 132 us).
+// The units' tiles, in unit order, are shared out over the blocks of a launch, which has as many blocks as the compute units hold
+// at once.  Few units: every unit gets the same number of blocks, and the few blocks left over idle.  Many units: the tiles are split
+// evenly, and a block's span may end in one unit and go on in the next (it then sets up twice, which only pays when whole
+// blocks per unit would leave many blocks idle).  With no more units than blocks a span touches two units at most.
+constexpr uint32_t kQuadMinBlocksPerUnit = 8;
+struct QuadSpan {
+    uint32_t lo, hi;                  // positions: unit * tiles_per_unit + tile
+    uint32_t unit0;                   // the unit that holds lo
+    tf_prefill_group run[2];          // the pairs of unit0 and of the unit after it
+    bool units;                       // false: too many chunks or units for this scheme, a "unit" is a whole chunk (batches in the block's own loop)
+};
+// scratch: 64 bytes of LDS that nothing else uses until the block's next barrier; 256 threads, all call
+__device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_chunks, uint32_t max_pairs, uint32_t tiles_per_unit, uint32_t *scratch) {
+    QuadSpan sp;
+    uint32_t units = n_chunks;
+    sp.units = n_chunks <= 512u;
+    tf_prefill_group mine[2] = {{0u, 0u, 0u}, {0u, 0u, 0u}};      // thread t: chunks 2 t and 2 t + 1
+    uint32_t batches[2] = {0u, 0u}, first = 0u;
+    if (sp.units) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (2u * threadIdx.x + i < n_chunks && get_chunk(cl, 2u * threadIdx.x + i, mine[i])) batches[i] = (mine[i].pair_count + max_pairs - 1) / max_pairs;
+        uint32_t sum = batches[0] + batches[1];                       // inclusive scan over the wave, then over the four waves
+#pragma unroll
+        for (int step = 1; step < 64; step <<= 1) {
+            const uint32_t below = (uint32_t)__shfl_up((int)sum, step, kWave);
+            if ((int)(threadIdx.x & 63) >= step) sum += below;
+        }
+        if ((threadIdx.x & 63) == 63) scratch[threadIdx.x >> 6] = sum;
+        __syncthreads();
+        uint32_t before = 0u, total = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) {
+            const uint32_t t = scratch[w];
+            before += w < (threadIdx.x >> 6) ? t : 0u;
+            total += t;
+        }
+        first = before + sum - batches[0] - batches[1];
+        units = uniform_u32(total);
+        sp.units = units <= gridDim.x;
+        if (!sp.units) units = n_chunks;
     }
+    const uint32_t per_unit = units ? gridDim.x / units : 0u;
+    if (per_unit >= kQuadMinBlocksPerUnit) {
+        const uint32_t unit = blockIdx.x / per_unit, part = blockIdx.x - unit * per_unit;
+        const bool idle = unit >= units;
+        sp.lo = idle ? 0u : unit * tiles_per_unit + tiles_per_unit * part / per_unit;
+        sp.hi = idle ? 0u : unit * tiles_per_unit + tiles_per_unit * (part + 1) / per_unit;
+    } else {
+        const uint64_t total = (uint64_t)units * tiles_per_unit;
+        sp.lo = (uint32_t)(total * blockIdx.x / gridDim.x);
+        sp.hi = (uint32_t)(total * (blockIdx.x + 1) / gridDim.x);
+    }
+    sp.unit0 = sp.lo / tiles_per_unit;
+    if (sp.units) {
+        // the owners of the two units' chunks tell the block
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+            for (uint32_t u = 0; u < 2; ++u) {
+                const uint32_t batch = sp.unit0 + u - first;          // wraps far beyond `batches` for a unit of an earlier chunk
+                if (batch < batches[i]) {
+                    scratch[4 + 3 * u] = mine[i].expert;
+                    scratch[5 + 3 * u] = mine[i].pair_start + batch * max_pairs;
+                    scratch[6 + 3 * u] = min(max_pairs, mine[i].pair_count - batch * max_pairs);
+                }
+            }
+            first += batches[i];
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < 2; ++u)
+            sp.run[u] = tf_prefill_group{uniform_u32(scratch[4 + 3 * u]), uniform_u32(scratch[5 + 3 * u]), uniform_u32(scratch[6 + 3 * u])};
+        __syncthreads();
+    }
+    return sp;
+}
+// the pairs of unit `unit` (false: there is no such chunk)
+__device__ __forceinline__ bool quad_run(const QuadSpan &sp, const ChunkList &cl, uint32_t unit, tf_prefill_group &run) {
+    if (sp.units) {
+        run = unit == sp.unit0 ? sp.run[0] : sp.run[1];
+        return true;
+    }
+    if (!get_chunk(cl, unit, run)) return false;
+    run.expert = uniform_u32(run.expert);
+    run.pair_start = uniform_u32(run.pair_start);
+    run.pair_count = uniform_u32(run.pair_count);
+    return true;
 }
 
 struct QuadPass {
@@ -248,19 +323,15 @@ __global__ __launch_bounds__(256, 3) void grouped_phase1_quad_kernel(ExpertTable
     // One tile buffer, used for a tile's gate rows, then its up rows, then the next tile's gate rows ...: while a matrix's
     // pass p is being used, the same pass of the matrix after it is already on its way into the registers that pass freed.
     QuadPass t[NPASS];
-    // the block's share of the tiles of all chunks, in chunk order
+    // the block's share of the tiles of all units
     const uint32_t tpe = (uint32_t)f / Map::kRows;
-    uint32_t span_lo, span_hi;
-    quad_span(quad_chunk_count(cl, n_chunks_upper), tpe, span_lo, span_hi);
-    for (uint32_t pos = span_lo; pos < span_hi;) {
-    const uint32_t chunk = pos / tpe;
-    const int t_lo = (int)(pos - chunk * tpe), t_hi = (int)min(tpe, (uint32_t)t_lo + (span_hi - pos));
+    const QuadSpan span = quad_span(cl, quad_chunk_count(cl, n_chunks_upper), (uint32_t)MAXP, tpe, reinterpret_cast<uint32_t *>(quad_lds));
+    for (uint32_t pos = span.lo; pos < span.hi;) {
+    const uint32_t unit = pos / tpe;
+    const int t_lo = (int)(pos - unit * tpe), t_hi = (int)min(tpe, (uint32_t)t_lo + (span.hi - pos));
     pos += (uint32_t)(t_hi - t_lo);
     tf_prefill_group ch;
-    if (!get_chunk(cl, chunk, ch)) continue;
-    ch.expert = uniform_u32(ch.expert);
-    ch.pair_start = uniform_u32(ch.pair_start);
-    ch.pair_count = uniform_u32(ch.pair_count);
+    if (!quad_run(span, cl, unit, ch)) continue;
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
     if (!base) continue;
     const rsrc_t blob = quad_blob_rsrc(base);
@@ -274,7 +345,7 @@ __global__ __launch_bounds__(256, 3) void grouped_phase1_quad_kernel(ExpertTable
         if (p == 0) tsb.request(from, (up ? off.up_s_off : off.gate_s_off) + sb_byte, (up ? off.up_b_off : off.gate_b_off) + sb_byte);
         quad_request(t[p], qm, p, from, (up ? off.up_W_off : off.gate_W_off) + w_byte);
     };
-    // a chunk longer than the LDS image goes through in batches, its weights once a batch
+    // (a whole chunk longer than the LDS image goes through in batches, its weights once a batch)
     for (uint32_t p0 = 0; p0 < ch.pair_count; p0 += (uint32_t)MAXP) {
         const uint32_t nb = min((uint32_t)MAXP, ch.pair_count - p0), first = ch.pair_start + p0;
         const int groups_of_pairs = (int)((nb + 3) >> 2);
@@ -352,19 +423,15 @@ __global__ __launch_bounds__(256, 5) void grouped_down_quad_kernel(ExpertTable t
     QuadPass t[NPASS];
     QuadTileSB<4> tsb;                                    // 8 rows of up to 16 groups: 4 bytes a lane
     tsb.init(lane, (uint32_t)Map::kRows * ((uint32_t)f >> 6) * 2u);
-    // the tiles of all chunks, split evenly over the blocks (see the gate / up kernel)
+    // the block's share of the tiles of all units (see the gate / up kernel)
     const uint32_t tiles = (uint32_t)d / Map::kRows;
-    uint32_t span_lo, span_hi;
-    quad_span(quad_chunk_count(cl, n_chunks_upper), tiles, span_lo, span_hi);
-    for (uint32_t pos = span_lo; pos < span_hi;) {
-    const uint32_t chunk = pos / tiles;
-    const int t_lo = (int)(pos - chunk * tiles), t_hi = (int)min(tiles, (uint32_t)t_lo + (span_hi - pos));
+    const QuadSpan span = quad_span(cl, quad_chunk_count(cl, n_chunks_upper), kQuadMaxPairs, tiles, reinterpret_cast<uint32_t *>(quad_lds));
+    for (uint32_t pos = span.lo; pos < span.hi;) {
+    const uint32_t unit = pos / tiles;
+    const int t_lo = (int)(pos - unit * tiles), t_hi = (int)min(tiles, (uint32_t)t_lo + (span.hi - pos));
     pos += (uint32_t)(t_hi - t_lo);
     tf_prefill_group ch;
-    if (!get_chunk(cl, chunk, ch)) continue;
-    ch.expert = uniform_u32(ch.expert);
-    ch.pair_start = uniform_u32(ch.pair_start);
-    ch.pair_count = uniform_u32(ch.pair_count);
+    if (!quad_run(span, cl, unit, ch)) continue;
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
     if (!base) continue;
     const rsrc_t blob = quad_blob_rsrc(base);
