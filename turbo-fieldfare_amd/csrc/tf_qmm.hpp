@@ -299,12 +299,17 @@ struct BFrag {
 
 template <int SD, int RT, int NW>
 struct QmmLoop {
-    static constexpr int AC = RT == 1 ? QmmGeom<NW>::kAChunks : (4 * RT + NW - 1) / NW;
+    static constexpr int AC = (4 * RT + NW - 1) / NW;
+    // W buffers per wave.  With one, a pair's weights are asked for two steps before they are read, less than a trip to HBM: a grouped
+    // block of up to 64 rows spent 1.9 us on each step (128 tokens x 8 of 128 experts, gate / up 83 us) with every unit of the CU
+    // mostly idle.  Up to two row tiles the second half of each X stage is free: a second buffer there doubles the distance.
+    static constexpr int WB = RT <= 2 && NW == 4 ? 2 : 1;
     const QmmARows<NW> &a;
     QmmBRows &rows;
     uint32_t lds;
     uint32_t frag[4];
-    uint32_t wread, wbuf;      // the wave's W buffer and this lane's 16 bytes of column tile 0, first step of a pair, in it
+    uint32_t wread, wbuf;      // the W buffer of the next pair and this lane's 16 bytes of column tile 0, first step of a pair, in it
+    uint32_t wread_sum, wbuf_sum;   // WB == 2: the two buffers' addresses added up (the other one is the sum less this one)
     uint32_t sbuf, sbread;     // the wave's two scale windows and this lane's row of tile 0 in the first
     uint32_t sbp;              // which window is current: 0 or kQmmSBBufBytes
     int last, last_pair;
@@ -368,7 +373,7 @@ struct QmmLoop {
     // block has met (every wave has its last fragments of this stage, and the copies of the next stage have landed).
     // Steps come in cycles of six, (U3, HALF) = (0,0) (1,1) (2,0) (0,1) (1,0) (2,1), one window of scales a cycle:
     //   every step:          X(kt + 3) is requested at the meeting point (AC copies);
-    //   second steps (HALF): the next pair's W words and scales are read from LDS, then W of the pair after it is requested
+    //   second steps (HALF): the next pair's W words and scales are read from LDS, then W of the pair WB after it is requested
     //                        into the same buffer (4 copies);
     //   step (0,1):          also the next cycle's window of scales and biases (2 copies), read from step (2,1) on.
     // What a step waits for was requested two steps earlier; the counts below are what may still be on its way at each wait.
@@ -388,7 +393,7 @@ struct QmmLoop {
         // X(kt + 1) has landed [second steps: also W and, where due, the window requested two steps ago]; younger requests may be
         // under way: after a second step its X, W (and window) copies, after a first step its X copies
         if constexpr (HALF == 0) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AC + 4 + (kAfterWindowStep ? 2 : 0)) : "memory");
-        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AC) : "memory");
+        else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(AC + (WB == 2 ? 4 : 0)) : "memory");      // two buffers: the youngest W may still be under way
         wait_frags<0>(1);
         __builtin_amdgcn_s_barrier();
         qmm_a_copy<NW, AC>(a, min(kt + 3, last), lds + base);
@@ -415,8 +420,12 @@ struct QmmLoop {
             if constexpr (RT == 2) asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sb.s[0]), "+v"(sb.s[1]), "+v"(sb.b[0]), "+v"(sb.b[1]) : : "memory");
             if constexpr (RT == 3) asm volatile("s_waitcnt lgkmcnt(3)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sb.s[0]), "+v"(sb.s[1]), "+v"(sb.b[0]), "+v"(sb.b[1]) : : "memory");
             if constexpr (RT == 4) asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sb.s[0]), "+v"(sb.s[1]), "+v"(sb.b[0]), "+v"(sb.b[1]) : : "memory");
-            // the W buffer has been read: the pair after the next goes into it
-            qmm_w_copy(rows, min(pair + 2, last_pair), wbuf);
+            // the W buffer has been read: the pair WB after the next goes into it
+            qmm_w_copy(rows, min(pair + 1 + WB, last_pair), wbuf);
+            if constexpr (WB == 2) {
+                wread = wread_sum - wread;
+                wbuf = wbuf_sum - wbuf;
+            }
 #pragma unroll
             for (int j = 0; j < 2; ++j) scales_of(sb.s[j], sb.b[j], j, false, s2n[j], b2n[j]);
             wa = w[0][0][0];
@@ -458,7 +467,13 @@ struct QmmLoop {
         qmm_sb_copy(rows, 0, sbuf);
         qmm_a_copy<NW, AC>(a, min(1, last), lds + kQmmStageBytes);
         qmm_a_copy<NW, AC>(a, min(2, last), lds + 2 * kQmmStageBytes);
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * AC) : "memory");
+        if constexpr (WB == 2) {
+            const uint32_t wave = threadIdx.x >> 6, second = lds + (wave >> 1) * (uint32_t)kQmmStageBytes + kQmmStageBytes / 2 + (wave & 1) * (uint32_t)kQmmWBytes;
+            wbuf_sum = wbuf + second;
+            wread_sum = 2 * wread + (second - wbuf);
+            qmm_w_copy(rows, min(1, last_pair), second);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * AC + (WB == 2 ? 4 : 0)) : "memory");
         __builtin_amdgcn_s_barrier();
         w[0][0] = lds_read16<0>(wread);
         w[0][1] = lds_read16<2048>(wread);
@@ -468,7 +483,11 @@ struct QmmLoop {
         else qmm_sb_read_tail<0>(sb, rows, 0, sbread);
         read_frags<0>(0, frag[0]);
         asm volatile("s_waitcnt lgkmcnt(%8)" : "+v"(w[0][0]), "+v"(w[0][1]), "+v"(w[1][0]), "+v"(w[1][1]), "+v"(sb.s[0]), "+v"(sb.s[1]), "+v"(sb.b[0]), "+v"(sb.b[1]) : "n"(RT) : "memory");
-        qmm_w_copy(rows, min(1, last_pair), wbuf);
+        qmm_w_copy(rows, min(WB, last_pair), wbuf);
+        if constexpr (WB == 2) {
+            wread = wread_sum - wread;
+            wbuf = wbuf_sum - wbuf;
+        }
         if constexpr (SD == 0) qmm_normalise_small_rows(rows, sb.s);
 #pragma unroll
         for (int j = 0; j < 2; ++j) scales_of(sb.s[j], sb.b[j], j, false, s2c[j], b2c[j]);
