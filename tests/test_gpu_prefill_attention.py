@@ -140,3 +140,39 @@ def test_contract():
     assert run(fx, q_token_stride_elements=255)[0] == bad and run(fx, o_token_stride_elements=255)[0] == bad   # :127-130
     assert run(fx, kv_token_stride_elements=127)[0] == bad                                      # :131-132
     assert run(fx, kv_valid_count=6)[0] == bad                                                  # :133-134
+
+
+@pytest.mark.parametrize("start,count,window,hq,hkv,ring,scale", [
+    (2000, 129, 0, 16, 16, 0, 512 ** -0.5),       # chunks; the second block of every head holds one column
+    (4000, 130, 2500, 32, 16, 2700, 0.4),         # a window in a ring, two heads a row; scores of +-40: the running maximum moves
+    (0, 400, 0, 64, 64, 0, 512 ** -0.5),          # one chunk: the kernel writes the rows itself
+    (1500, 500, 0, 16, 2, 0, 512 ** -0.5),        # a block of a global layer
+])
+def test_wide_columns_of_head_dim_512(start, count, window, hq, hkv, ring, scale):
+    # blocks of 128 columns (at least three quarters as many of them as compute units), against 64-bit arithmetic; the bound is the one
+    # the block attention is held to elsewhere in this file
+    import ctypes as C
+    import torch
+    hd, n = 512, start + count
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(start + count)
+    q, k, v = (torch.randn(rows, heads, hd, device="cuda", generator=gen).half() for rows, heads in ((count, hq), (n, hkv), (n, hkv)))
+    if ring:                                       # rows the window has left are overwritten by later positions
+        kr, vr = (torch.zeros(ring, hkv, hd, device="cuda", dtype=torch.float16) for _ in range(2))
+        at = torch.arange(n - ring, n, device="cuda")
+        kr[at % ring], vr[at % ring] = k[at], v[at]
+    else:
+        kr, vr = k, v
+    out = torch.full((count, hq, hd), float("nan"), device="cuda", dtype=torch.float16)
+    kk = ctx()
+    kk.reserve(max_q_heads=hq, max_attention_block_tokens=count)
+    p = tfk.PrefillAttentionParams(start, count, hd, hq, hkv, n, window, hkv * hd, hq * hd, hq * hd, scale)
+    kk.check(kk.lib.tf_prefill_attention_causal(kk.handle, None, q.data_ptr(), 0, kr.data_ptr(), 0, vr.data_ptr(), 0, out.data_ptr(), 0, C.byref(p), ring))
+    torch.cuda.synchronize()
+    pos, row = torch.arange(n, device="cuda")[None, :], torch.arange(start, n, device="cuda")[:, None]
+    hidden = (pos > row) | ((pos <= row - window) if window else torch.zeros_like(pos > row))
+    for h in range(hq):
+        g = h // (hq // hkv)
+        scores = (q[:, h].double() @ k[:, g].double().T.contiguous()) * scale
+        want = torch.softmax(scores.masked_fill(hidden, float("-inf")), 1) @ v[:, g].double()
+        assert torch.all((out[:, h].double() - want).abs() <= 2e-3 * want.abs().clamp(min=1.0)), h

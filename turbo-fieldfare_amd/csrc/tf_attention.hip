@@ -617,6 +617,241 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
     }
 }
 
+// The same for head_dim 512 with 128 columns a block.  In the kernel above every wave reads the whole K and the whole V tile and turns
+// the whole V tile into operands with byte permutes, for 16 columns: one wave a SIMD, 5000 cycles a tile against 1024 of matrix
+// work, and 16 column blocks fetch every cache row from L2 (128 queries over 32768 keys: 325 us, 422 TFLOP/s).  Here eight waves, two a
+// SIMD, take the scores of 16 columns each as above and leave the probabilities in LDS as the operands they are; for the values a
+// wave owns 64 of the 512 output elements of ALL 128 columns, so a V tile is read and permuted once a block instead of once a wave, and
+// twice the columns share each tile's trip into LDS.
+constexpr int kWideWaves = 8, kWideCols = kWideWaves * kTileHeads;
+__global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_kernel(const half_t *Q, const half_t *K, const half_t *V, half_t *O, float *m_part,
+                                                                                    float *d_part, float *o_part, PrefillShape s, uint32_t group_shift,
+                                                                                    uint32_t col_blocks, uint32_t num_chunks) {
+    constexpr int HD = 512, KS = HD / 32, BLK = 1040, TILEB = kPrefillKeys * BLK;      // a tile row: 1024 bytes and 16 of padding (see above)
+    constexpr int CPW = kPrefillKeys / kWideWaves;                                     // rows a wave copies per tile and matrix
+    __shared__ __align__(16) uint8_t k_lds[2][TILEB];
+    __shared__ __align__(16) uint8_t v_lds[2][TILEB];
+    __shared__ __align__(16) uint8_t p_lds[kWideWaves * 1024];                         // wave w's probabilities: 16 bytes a lane
+    __shared__ __align__(16) float col_lds[kWideCols];                                 // a column's rescale factor; at the end its denominator
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, quad = lane >> 4;
+
+    const uint32_t groups = s.num_kv_heads * num_chunks;
+    uint32_t grp, col_block;
+    if (groups % kXcds == 0u) {
+        const uint32_t xcd = blockIdx.x % kXcds, slot = blockIdx.x / kXcds;
+        grp = xcd + kXcds * (slot / col_blocks);
+        col_block = slot % col_blocks;
+    } else {
+        grp = blockIdx.x / col_blocks;
+        col_block = blockIdx.x % col_blocks;
+    }
+    const uint32_t kv_head = grp / num_chunks, chunk = grp % num_chunks;
+    const uint32_t group = 1u << group_shift, pairs = s.count << group_shift;
+
+    const uint32_t col0 = col_block * kWideCols;
+    const uint32_t t_lo = min(col0 >> group_shift, s.count - 1u), t_hi = min((col0 + kWideCols - 1u) >> group_shift, s.count - 1u);
+    uint32_t p_lo, p_hi, unused;
+    visible_keys(s, t_lo, p_lo, unused);
+    visible_keys(s, t_hi, unused, p_hi);
+    const uint32_t span = p_hi > p_lo ? p_hi - p_lo : 0u;
+    const uint32_t chunk_len = ((span + num_chunks - 1u) / num_chunks + kPrefillKeys - 1u) / kPrefillKeys * kPrefillKeys;
+    const uint32_t c_lo = p_lo + chunk * chunk_len, c_hi = min(p_hi, c_lo + chunk_len);
+
+    // the lane's column as a producer of probabilities
+    const uint32_t pair = col0 + (uint32_t)(wave * kTileHeads + col);
+    const bool col_live = pair < pairs;
+    const uint32_t t_col = col_live ? pair >> group_shift : 0u, q_head = kv_head * group + (pair & (group - 1u));
+    uint32_t first_col = 0u, last_col = 0u;
+    if (col_live) visible_keys(s, t_col, first_col, last_col);
+
+    half8_t qf[KS];
+#pragma unroll
+    for (int d = 0; d < KS; ++d) {
+        u32x4 raw = {0u, 0u, 0u, 0u};
+        if (col_live) raw = load16(Q + (size_t)t_col * s.q_stride + (size_t)q_head * HD + 32 * d + 8 * quad);
+        qf[d] = __builtin_bit_cast(half8_t, raw);
+    }
+    float4_t o[kWideWaves][4];      // o[c][t][r]: element 64 wave + 4 (4 quad + r) + t of column 16 c + col
+#pragma unroll
+    for (int c = 0; c < kWideWaves; ++c)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) o[c][t] = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    float m_run = -INFINITY, d_run = 0.0f;
+
+    const attn_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(K + (size_t)kv_head * HD), 0, (int)0xFFFFFFFFu, 0x00020000);
+    const attn_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(V + (size_t)kv_head * HD), 0, (int)0xFFFFFFFFu, 0x00020000);
+    const uint32_t row_bytes = s.kv_stride * 2u;
+    auto copy_tile = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0, uint32_t lane16) {
+#pragma unroll
+        for (int q = 0; q < CPW; ++q) {
+            const uint32_t n = (uint32_t)wave + (uint32_t)(kWideWaves * q);
+            const uint32_t p = min(t0 + n, c_hi - 1u);
+            attn_lds_copy16(rsrc, tile + n * BLK, prefill_row(s, p) * row_bytes + lane16);
+        }
+    };
+    const uint32_t k_tile = (uint32_t)(uintptr_t)k_lds[0], v_tile = (uint32_t)(uintptr_t)v_lds[0];      // buffer b: + b TILEB
+    const uint32_t p_base = (uint32_t)(uintptr_t)p_lds, p_tile = p_base + (uint32_t)lane * 16u, f_base = (uint32_t)(uintptr_t)col_lds;
+    // operand pieces inside a tile: K row `col` (and 16 + col), 16 bytes `quad` of every step; V rows 4 quad + 0 .. 3 (and 16 more), the
+    // four elements 4 col .. of the wave's 64
+    const uint32_t k_lane = (uint32_t)(col * BLK + quad * 16), v_lane = (uint32_t)(4 * quad * BLK + wave * 128 + col * 8);
+
+    auto scores = [&](uint32_t tile, float4_t &acc0, float4_t &acc1) {
+        const uint32_t at = tile + k_lane;
+        acc0 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        acc1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        u32x4 kf[2][4];                     // two steps of two row groups each, two deep
+        auto issue = [&](u32x4 (&f)[4], int b) {
+            const uint32_t from = at + (uint32_t)(b * 128);
+            f[0] = attn_lds_read16<0>(from);
+            f[1] = attn_lds_read16<16 * BLK>(from);
+            f[2] = attn_lds_read16<64>(from);
+            f[3] = attn_lds_read16<16 * BLK + 64>(from);
+        };
+        issue(kf[0], 0);
+#pragma unroll
+        for (int b = 0; b < KS / 2; ++b) {
+            u32x4 (&f)[4] = kf[b & 1];
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(f[3]));
+            if (b + 1 < KS / 2) issue(kf[(b + 1) & 1], b + 1);
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, f[2 * d]), qf[2 * b + d], acc0, 0, 0, 0);
+                acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, f[2 * d + 1]), qf[2 * b + d], acc1, 0, 0, 0);
+            }
+        }
+    };
+
+    if (c_lo < c_hi) {
+        const uint32_t n_tiles = (c_hi - c_lo + kPrefillKeys - 1u) / kPrefillKeys;
+        copy_tile(k_rsrc, k_tile, c_lo, (uint32_t)lane * 16u);
+        copy_tile(v_rsrc, v_tile, c_lo, (uint32_t)lane * 16u);
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        constexpr float kMaxSlack = 8.0f;      // as above: the reference maximum moves when a score exceeds it by more
+        for (uint32_t i = 0; i < n_tiles; ++i) {
+            // K and V tile i are in LDS and nobody reads the other two buffers any more (past the chunk: repeated rows, never used)
+            const uint32_t t0 = c_lo + i * kPrefillKeys, cur = (i & 1u) * TILEB, other = TILEB - cur;
+            uint32_t lane16 = p_tile - p_base;         // made anew in every step, here and below: there are no registers to keep it in
+            asm volatile("" : "+v"(lane16));
+            copy_tile(k_rsrc, k_tile + other, t0 + kPrefillKeys, lane16);
+            copy_tile(v_rsrc, v_tile + other, t0 + kPrefillKeys, lane16);
+            float4_t acc0, acc1;
+            scores(k_tile + cur, acc0, acc1);
+            float sc[8], tile_max = -INFINITY;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t p = t0 + (uint32_t)(16 * (e >> 2) + 4 * quad + (e & 3));
+                const float raw = e < 4 ? acc0[e & 3] : acc1[e & 3];
+                sc[e] = (p >= first_col && p < last_col) ? raw * s.scale : -INFINITY;
+                tile_max = fmaxf(tile_max, sc[e]);
+            }
+            tile_max = column_reduce(tile_max, [](float a, float b) { return fmaxf(a, b); });
+            const bool fresh = m_run == -INFINITY;
+            const float m_new = (fresh || tile_max > m_run + kMaxSlack) ? fmaxf(m_run, tile_max) : m_run;
+            const float alpha = fresh ? 1.0f : __expf(m_run - m_new);
+            float sum = 0.0f;
+            half8_t p8;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const float pe = exp_weight(sc[e], m_new);
+                p8[e] = (half_t)pe;
+                sum += pe;
+            }
+            sum = column_reduce(sum, [](float a, float b) { return a + b; });
+            d_run = d_run * alpha + sum;
+            m_run = m_new;
+            asm volatile("ds_write_b128 %0, %1" ::"v"(p_tile + (uint32_t)wave * 1024u), "v"(p8) : "memory");
+            lane16 = p_tile - p_base;
+            asm volatile("" : "+v"(lane16));
+            if (lane16 < 16u * kTileHeads) asm volatile("ds_write_b32 %0, %1" ::"v"(f_base + (uint32_t)wave * (kTileHeads * 4u) + (lane16 >> 2)), "v"(alpha) : "memory");
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+
+            // values: slot e of a lane's 8 keys is row 16 (e / 4) + 4 quad + e % 4 of the tile
+            float f0, f1;
+            u32x2 in[8];
+            lane16 = p_tile - p_base;
+            asm volatile("" : "+v"(lane16));
+            const uint32_t va = v_tile + cur + v_lane, fa = f_base + (lane16 >> 2);
+            asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:256" : "=&v"(f0), "=&v"(f1) : "v"(fa));
+#define TF_READ_V(E) asm volatile("ds_read_b64 %0, %1 offset:%2" : "=v"(in[E]) : "v"(va), "n"(((E) >> 2) * 16 * BLK + ((E) & 3) * BLK))
+            TF_READ_V(0); TF_READ_V(1); TF_READ_V(2); TF_READ_V(3); TF_READ_V(4); TF_READ_V(5); TF_READ_V(6); TF_READ_V(7);
+#undef TF_READ_V
+            u32x4 pf[2];
+            pf[0] = attn_lds_read16<0>(p_tile);
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f0), "+v"(f1), "+v"(in[0]), "+v"(in[1]), "+v"(in[2]), "+v"(in[3]), "+v"(in[4]), "+v"(in[5]), "+v"(in[6]), "+v"(in[7]), "+v"(pf[0]));
+            if (__builtin_expect(__any(f0 != 1.0f || f1 != 1.0f), 0)) {
+#pragma unroll
+                for (int c = 0; c < kWideWaves; ++c) {
+                    float f;
+                    lane16 = p_tile - p_base;
+                    asm volatile("" : "+v"(lane16));
+                    asm volatile("ds_read_b32 %0, %1\n\ts_waitcnt lgkmcnt(0)" : "=v"(f) : "v"(f_base + (uint32_t)(kTileHeads * c) * 4u + ((lane16 >> 2) & (kTileHeads * 4u - 4u))));
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) o[c][t] *= f;
+                }
+            }
+            u32x4 a[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;
+#pragma unroll
+                for (int kp = 0; kp < 4; ++kp) a[t][kp] = __builtin_amdgcn_perm(in[2 * kp + 1][t >> 1], in[2 * kp][t >> 1], sel);
+            }
+#define TF_VALUES(C)                                                                                                                     \
+            {                                                                                                                            \
+                if constexpr ((C) + 1 < kWideWaves) pf[((C) + 1) & 1] = attn_lds_read16<(((C) + 1) % kWideWaves) * 1024>(p_tile);             \
+                _Pragma("unroll") for (int t = 0; t < 4; ++t)                                                                            \
+                    o[C][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, a[t]), __builtin_bit_cast(half8_t, pf[(C) & 1]), o[C][t], 0, 0, 0); \
+                if constexpr ((C) + 1 < kWideWaves) asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(pf[((C) + 1) & 1]));                        \
+            }
+            TF_VALUES(0) TF_VALUES(1) TF_VALUES(2) TF_VALUES(3) TF_VALUES(4) TF_VALUES(5) TF_VALUES(6) TF_VALUES(7)
+#undef TF_VALUES
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // this wave's copies have landed
+            __builtin_amdgcn_s_barrier();
+        }
+    }
+
+    // the columns' denominators (or the states' m and d) from the waves that kept them; a wave's elements of all columns from itself
+    __syncthreads();
+    if (quad == 0) {
+        if (num_chunks == 1u) {
+            col_lds[wave * kTileHeads + col] = d_run > 0.0f ? 1.0f / d_run : 0.0f;      // zero where the column saw no key
+        } else if (col_live) {
+            const size_t state = ((size_t)t_col * s.num_q_heads + q_head) * num_chunks + chunk;
+            m_part[state] = m_run;
+            d_part[state] = d_run;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < kWideWaves; ++c) {
+        const uint32_t pc = col0 + (uint32_t)(kTileHeads * c + col);
+        if (pc >= pairs) continue;
+        const uint32_t tc = pc >> group_shift, hc = kv_head * group + (pc & (group - 1u));
+        const uint32_t e0 = (uint32_t)(64 * wave + 16 * quad);           // + 4 r + t
+        if (num_chunks == 1u) {
+            const float inv = col_lds[kTileHeads * c + col];
+            half_t *dst = O + (size_t)tc * s.o_stride + (size_t)hc * HD + e0;
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                u32x4 packed;
+#pragma unroll
+                for (int w = 0; w < 4; ++w) {
+                    const int r = 2 * h + (w >> 1), t = 2 * (w & 1);
+                    packed[w] = as_u32(half2_t{(half_t)(o[c][t][r] * inv), (half_t)(o[c][t + 1][r] * inv)});
+                }
+                *reinterpret_cast<u32x4 *>(dst + 8 * h) = packed;
+            }
+        } else {
+            float *dst = o_part + (((size_t)tc * s.num_q_heads + hc) * num_chunks + chunk) * HD + e0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) *reinterpret_cast<float4_t *>(dst + 4 * r) = float4_t{o[c][0][r], o[c][1][r], o[c][2][r], o[c][3][r]};
+        }
+    }
+}
+
 // merge of the chunks' partial states of one (query, head) column: out = sum_c w_c o_c / sum_c w_c d_c, w_c = exp(m_c - max m);
 // chunks are added in ascending order; a chunk that saw no key has weight zero and its o is not read
 __global__ __launch_bounds__(128) void attention_prefill_combine_kernel(const float *m_part, const float *d_part, const float *o_part, half_t *O,
@@ -852,7 +1087,7 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
                       aligned16(kp) && aligned16(vp) && aligned16(op) && s.q_stride % 8 == 0 && s.kv_stride % 8 == 0 && s.o_stride % 8 == 0 &&
                       cache_bytes < (1ull << 32);   // the copies address cache rows with 32-bit byte offsets
     if (mfma) {
-        const uint32_t col_blocks = (s.count * group + kPrefillCols - 1) / kPrefillCols, base = col_blocks * s.num_kv_heads;
+        uint32_t col_blocks = (s.count * group + kPrefillCols - 1) / kPrefillCols, base = col_blocks * s.num_kv_heads;
         // enough chunks to give every CU a block (two where two fit), none shorter than kMinChunkKeys
         const uint32_t abs_first = s.start, abs_last = s.start + s.count - 1u;
         const uint32_t lo_first = (s.window != 0u && abs_first + 1u > s.window) ? abs_first + 1u - s.window : 0u;
@@ -860,15 +1095,47 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
         const uint32_t span = hi_last > lo_first ? hi_last - lo_first : 0u;
         const uint32_t target = (uint32_t)ctx->num_cus * (hd > 256 ? 1u : 2u);
         uint32_t chunks = std::max(1u, std::min({(target + base - 1) / base, span / kMinChunkKeys, kMaxPrefillChunks}));
-        float *m = nullptr, *d = nullptr, *o = nullptr;
+        auto states_of = [&](uint32_t c) { return (size_t)s.count * s.num_q_heads * c; };
+        float *m = nullptr, *d = nullptr, *o = nullptr, *scratch = nullptr;
         if (chunks > 1) {
-            const size_t states = (size_t)s.count * s.num_q_heads * chunks;
-            float *scratch = nullptr;
-            const int32_t rc = attention_scratch(ctx, states * (2 + (size_t)hd), scratch);
+            const int32_t rc = attention_scratch(ctx, states_of(chunks) * (2 + (size_t)hd), scratch);
             if (rc != TF_OK) return rc;
+        }
+        // head_dim 512: the wide kernel where the model below prices it lower.  Both kernels have one block on a compute unit; a block takes
+        // about 0.092 us a key here and 0.1 us in the wide kernel, for 64 and 128 columns.  So the wide kernel wins wherever its
+        // blocks, half as many a chunk, still fill the chip: 128 queries over 32768 keys (256 blocks either way) 310 -> 218 us, 500 over
+        // 2000 120 -> 81, 160 over 24160 493 -> 205; but 77 over 3077 (120 blocks for 240) 44 -> 48 and 128 over 768 (48 for 96) 37 -> 43.
+        bool wide = false;
+        if (hd == 512) {
+            const uint32_t wide_blocks = (s.count * group + kWideCols - 1) / kWideCols, wide_base = wide_blocks * s.num_kv_heads, cus = (uint32_t)ctx->num_cus;
+            // in keys: the longest compute unit's blocks, one at a time (20 blocks a chunk: 12 chunks in one go, not 13 in two), and the
+            // merge, where a chunk's partial states of 195 columns cost as much as a key of a block (4 KB a column written and read
+            // back at 8 TB/s).  Chunks only as far as the scratch reaches (a reserved context's always does).
+            auto price = [&](uint32_t blocks, uint32_t c, float key) {
+                return (float)((blocks * c + cus - 1) / cus) * (float)span / (float)c * key + (c > 1 ? (float)s.count * (float)s.num_q_heads * (float)c / 195.0f : 0.0f);
+            };
+            uint32_t best = 1;
+            for (uint32_t c = 2; c <= std::min(span / kMinChunkKeys, kMaxPrefillChunks) && states_of(c) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes; ++c)
+                if (price(wide_base, c, 1.0f) < price(wide_base, best, 1.0f)) best = c;
+            wide = price(wide_base, best, 1.0f) < price(base, chunks, 0.92f);
+            if (wide) {
+                col_blocks = wide_blocks;
+                base = wide_base;
+                chunks = best;
+                scratch = static_cast<float *>(ctx->attn_scratch);
+            }
+        }
+        if (chunks > 1) {
             m = scratch;
-            d = scratch + states;
-            o = scratch + 2 * states;
+            d = scratch + states_of(chunks);
+            o = scratch + 2 * states_of(chunks);
+        }
+        if (wide) {
+            hipLaunchKernelGGL(attention_prefill_wide_kernel, dim3(base * chunks), dim3(64 * kWideWaves), 0, st, qp, kp, vp, op, m, d, o, s, shift, col_blocks, chunks);
+            if (chunks > 1)
+                hipLaunchKernelGGL(attention_prefill_combine_kernel, dim3(s.count * s.num_q_heads), dim3(128), 0, st, m, d, o, op, hd, chunks, s.num_q_heads,
+                                   s.o_stride);
+            return check_launch(ctx, "prefill_attention");
         }
         const dim3 grid(base * chunks);
         switch (hd) {
