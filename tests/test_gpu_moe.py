@@ -475,6 +475,29 @@ def test_prefill_shared_expert_block_with_gate_and_up_scales_far_apart_takes_the
     del arena
 
 
+@pytest.mark.parametrize("rows,d,f,far,y_pad", [(2, 1152, 1088, False, 0), (7, 2816, 2112, False, 1), (9, 1152, 1088, True, 3), (25, 2816, 2112, True, 0),
+                                                (11, 4096, 1536, True, 8)])
+def test_prefill_shared_expert_rows_of_the_single_row_chain_in_two_launches(rows, d, f, far, y_pad):
+    # few rows, or gate and up scales out of one descriptor's reach: the chain's own bits, in one, two and four passes over a row
+    c = _shared_block_case(rows, d, f, 0x4A0 + rows)
+    k = ctx()
+    t = {n: [dev(a) for a in c[n]] for n in ("gate", "up", "down")}
+    pg, pu = _proj(*t["gate"], f, d), _proj(*t["up"], f, d)
+    if far:
+        at = (1 << 31) + (1 << 20)
+        arena = torch.empty(at + (1 << 20), dtype=torch.uint8, device="cuda")
+        for p, bits, offset in ((pg, c["gate"][1], 0), (pu, c["up"][1], at)):
+            arena[offset:offset + bits.nbytes] = torch.from_numpy(np.ascontiguousarray(bits).view(np.uint8).ravel()).cuda()
+            p.scales, p.scales_offset = arena.data_ptr(), offset
+    x, y = dev(c["x_bits"]), dev(np.full((rows, d + y_pad), SENTINEL, np.uint16))
+    sg, su, sa = zeros_bytes(f * 2), zeros_bytes(f * 2), zeros_bytes(f * 2)
+    rc = k.prefill_shared_expert_block(x, pg, pu, _proj(*t["down"], d, f), y, sg, su, sa, rows, d, f, y_stride=d + y_pad, raise_on_error=False)
+    assert rc == tfk.TF_OK, k.last_error()
+    got = host(y, np.uint16).reshape(rows, d + y_pad)
+    assert np.array_equal(got[:, :d], _repeated_rows(c, rows))
+    assert np.all(got[:, d:] == SENTINEL)
+
+
 def test_prefill_shared_expert_block_contract():
     c = _shared_block_case(4, 128, 64, 7)
     assert run_shared_block(c, 0, 128, 128)[0] == tfk.TF_OK                       # queryCount 0: nothing to do

@@ -523,6 +523,59 @@ __global__ __launch_bounds__(256) void shared_gate_up_long_kernel(SharedGateUpAr
     shared_gate_up_long_body<RT, NP, SD>(a, blockIdx.x, xa, xsum);
 }
 
+// The single-row chain for a block of rows, bit for bit: a block takes its four tiles' weights once and up to kRowsPerBlock activation
+// rows one after the other.  Row by row in launches of their own 512 rows of d 2816, f 2112 took 4.4 ms, most of it launches and weights fetched
+// anew; so 0.72 ms.  GEGLU: two matrices, half(gelu_tanh(half(gate)) * half(up)); otherwise one.
+constexpr int kRowsPerBlock = 8;
+struct SharedRowsArgs {
+    const uint8_t *W[2], *S[2], *B[2];
+    const half_t *x;
+    long ldx;
+    half_t *y;
+    long ldy;
+    uint32_t rows, m;
+    int k;
+};
+template <int RT, int NP, int SD, bool GEGLU>
+__global__ __launch_bounds__(256) void shared_rows_kernel(SharedRowsArgs a) {
+    __shared__ __align__(16) u32x4 xa[XStage::kMaxK / 8];
+    __shared__ float xsum[XStage::kMaxK / 32];
+    const int lane = threadIdx.x & 63;
+    const uint32_t row0 = uniform_u32((blockIdx.x * blockDim.x + threadIdx.x) >> 6) * RT;
+    const uint32_t first = blockIdx.y * kRowsPerBlock, last = min(first + (uint32_t)kRowsPerBlock, a.rows);
+    const bool live = row0 < a.m;
+    XStage stage;
+    stage.request(a.x + (size_t)first * a.ldx, a.k);
+    RowStream<RT, NP> rs;
+    typename RowStream<RT, NP>::Tile t0, t1;
+    rs.init_map(a.k, lane);
+    if (live) {
+        const size_t w_byte = (size_t)row0 * (a.k >> 1), sb_byte = (size_t)row0 * (a.k >> 6) * 2;
+        rs.load(t0, a.W[0] + w_byte, a.S[0] + sb_byte, a.B[0] + sb_byte, a.m - row0);
+        if constexpr (GEGLU) rs.load(t1, a.W[1] + w_byte, a.S[1] + sb_byte, a.B[1] + sb_byte, a.m - row0);
+    }
+    for (uint32_t row = first; row < last; ++row) {
+        stage.publish(a.k, xa, xsum);                     // ends with a barrier
+        if (row + 1 < last) stage.request(a.x + (size_t)(row + 1) * a.ldx, a.k);
+        if (live) {
+            rs.init_x_lds(xa, xsum, a.k);
+            float v[RT], up[RT];
+            rs.template reduce<SD>(t0, v);
+            if constexpr (GEGLU) rs.template reduce<SD>(t1, up);
+            if (lane == 0) {
+#pragma unroll
+                for (int r = 0; r < RT; ++r) {
+                    if (row0 + r >= a.m) continue;
+                    half_t out = (half_t)v[r];
+                    if constexpr (GEGLU) out = (half_t)(gelu_tanh((float)out) * (float)(half_t)up[r]);
+                    a.y[(size_t)row * a.ldy + row0 + r] = out;
+                }
+            }
+        }
+        __syncthreads();                                  // the row in LDS has been read
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ two stages, one launch
 // The shared expert does not depend on the router or the routed experts (the reference commits it on a command buffer of its
 // own).  In a chain of launches on one stream it can ride along: its gate / up rows as extra blocks of the router launch, its
@@ -1237,6 +1290,41 @@ int32_t shared8_block(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, co
 #undef TF_GEMV8_ROWS
 #undef TF_SH8_ROWS
     return check_launch(ctx, "int8 gemv rows");
+}
+
+// TF_ERR_UNAVAILABLE: the single-row chain would take other kernels than the long-row ones; the caller goes row by row
+int32_t shared4_rows(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const void *x,
+                     uint32_t x_stride_elements, void *y, uint32_t y_stride_elements, uint32_t rows, void *acts, tf_dtype scale_dtype) {
+    const uint32_t f = gate->rows, d = gate->cols;
+    const uint8_t *gw = at(gate->weights, gate->weights_offset), *uw = at(up->weights, up->weights_offset);
+    const uint8_t *dw = at(down->weights, down->weights_offset);
+    const LongPlan plan_d = plan_long_rows((int)d), plan_f = plan_long_rows((int)f);
+    const bool ok = projection_ok(gate) && projection_ok(up) && projection_ok(down) && aligned16(gw) && aligned16(uw) && aligned16(dw) && aligned16(x) &&
+                    aligned16(acts) && x_stride_elements % 8 == 0 && d > 1024 && f > 1024 && plan_d.rt > 0 && plan_f.rt > 0 &&
+                    rows <= 65535u * (uint32_t)kRowsPerBlock && (scale_dtype == TF_BF16 || scale_dtype == TF_FP16);
+    if (!ok) return TF_ERR_UNAVAILABLE;
+    half_t *ap = static_cast<half_t *>(acts);
+    const SharedRowsArgs a1 = {{gw, uw}, {at(gate->scales, gate->scales_offset), at(up->scales, up->scales_offset)},
+                               {at(gate->biases, gate->biases_offset), at(up->biases, up->biases_offset)}, static_cast<const half_t *>(x),
+                               (long)x_stride_elements, ap, (long)f, rows, f, (int)d};
+    const uint8_t *ds = at(down->scales, down->scales_offset), *db = at(down->biases, down->biases_offset);
+    const SharedRowsArgs a2 = {{dw, dw}, {ds, ds}, {db, db}, ap, (long)f, static_cast<half_t *>(y), (long)y_stride_elements, rows, d, (int)f};
+    auto launch = [&](const SharedRowsArgs &a, const LongPlan &plan, auto geglu) {
+        const dim3 grid(((a.m + plan.rt - 1) / plan.rt + 3) / 4, (rows + kRowsPerBlock - 1) / kRowsPerBlock);
+#define TF_SH_ROWS(RT_, NP_)                                                                                                              \
+    if (plan.rt == RT_ && plan.np == NP_) {                                                                                               \
+        if (scale_dtype == TF_BF16) hipLaunchKernelGGL((shared_rows_kernel<RT_, NP_, 0, decltype(geglu)::value>), grid, dim3(256), 0, st, a); \
+        else hipLaunchKernelGGL((shared_rows_kernel<RT_, NP_, 1, decltype(geglu)::value>), grid, dim3(256), 0, st, a);                        \
+        return check_launch(ctx, "shared expert rows");                                                                                   \
+    }
+        TF_SH_ROWS(1, 1) TF_SH_ROWS(1, 2) TF_SH_ROWS(1, 3) TF_SH_ROWS(1, 4)
+        TF_SH_ROWS(2, 1) TF_SH_ROWS(2, 2) TF_SH_ROWS(2, 3) TF_SH_ROWS(2, 4)
+        TF_SH_ROWS(4, 1) TF_SH_ROWS(4, 2) TF_SH_ROWS(4, 3) TF_SH_ROWS(4, 4)
+#undef TF_SH_ROWS
+        return (int32_t)TF_ERR_UNAVAILABLE;
+    };
+    const int32_t rc = launch(a1, plan_d, std::true_type{});
+    return rc != TF_OK ? rc : launch(a2, plan_f, std::false_type{});
 }
 
 }  // namespace tfk

@@ -788,6 +788,17 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
         rc8 = shared8_block(ctx, st, gate, up, down, xp, x_stride_elements, yp, y_stride_elements, query_count, acts8, scale_dtype);
         if (rc8 != TF_ERR_UNAVAILABLE) return rc8;
     }
+    // The single-row chain over many rows (fewer than kSharedBlockMinRows, or gate and up arrays out of each other's reach) in two launches, with the
+    // same bits, where every row would take the chain's vector kernels and the context holds the activations: 7 / 53 / 512 rows of d 2816,
+    // f 2112 64 / 423 / 4370 -> 26 / 84 / 723 us
+    const uint64_t one_row = (uint64_t)intermediate * 2;
+    if (!block_path && weight_bits == 4 && pointers && even && query_count >= 2 && (uint64_t)query_count * one_row <= ctx->shared_block_acts_bytes &&
+        intermediate % TF_GROUP_SIZE == 0 && d % TF_GROUP_SIZE == 0 && scratch_gate_offset + one_row <= scratch_gate_length &&
+        scratch_up_offset + one_row <= scratch_up_length && scratch_act_offset + one_row <= scratch_act_length && scratch_gate_offset % 2 == 0 &&
+        scratch_up_offset % 2 == 0 && aligned16(at(scratch_act, scratch_act_offset))) {
+        const int32_t rc4 = shared4_rows(ctx, st, gate, up, down, xp, x_stride_elements, yp, y_stride_elements, query_count, ctx->shared_block_acts, scale_dtype);
+        if (rc4 != TF_ERR_UNAVAILABLE) return rc4;
+    }
     if (!block_path) {
         // PrefillSharedExpert.encodeBlock itself: the single-row chain once per row, every row through the same scratch
         for (uint32_t row = 0; row < query_count; ++row) {
