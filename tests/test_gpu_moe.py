@@ -361,6 +361,13 @@ def test_prefill_shared_expert_block_with_8_bit_weights_is_the_row_chain(d, f, r
 
 
 
+@pytest.mark.parametrize("d,f,rows,pad", [(64, 64, 16, 0), (1088, 1984, 33, 0),           # fewer groups than waves; odd numbers of groups
+                                          (2816, 2112, 97, 8),                          # two row tiles of 64 a gate / up tile, 64 x 64 down tiles
+                                          (4096, 4096, 40, 0), (4160, 64, 20, 0)])       # the widest rows the split kernels take; wider
+def test_8_bit_block_tile_edges(d, f, rows, pad):
+    test_prefill_shared_expert_block_with_8_bit_weights_is_the_row_chain(d, f, rows, pad)
+
+
 def test_8_bit_block_on_matrix_cores_with_small_scales():
     # From 16 rows on the 8-bit block rounds every weight to fp16 (half(q s + b), the reference's staged-affine rounding point,
     # tensorops.metal:57-94) while the row chain keeps q s + b in fp32.  Weights of magnitude 1e-3 and less have scales near
@@ -475,10 +482,10 @@ def test_prefill_shared_expert_block_with_gate_and_up_scales_far_apart_takes_the
     del arena
 
 
-@pytest.mark.parametrize("rows,d,f,far,y_pad", [(2, 1152, 1088, False, 0), (7, 2816, 2112, False, 1), (9, 1152, 1088, True, 3), (25, 2816, 2112, True, 0),
+@pytest.mark.parametrize("rows,d,f,far,y_pad", [(7, 1152, 1088, False, 1), (8, 1152, 1088, True, 0), (9, 1152, 1088, True, 3), (25, 2816, 2112, True, 0),
                                                 (11, 4096, 1536, True, 8)])
-def test_prefill_shared_expert_rows_of_the_single_row_chain_in_two_launches(rows, d, f, far, y_pad):
-    # few rows, or gate and up scales out of one descriptor's reach: the chain's own bits, in one, two and four passes over a row
+def test_prefill_shared_expert_block_far_apart_in_two_launches(rows, d, f, far, y_pad):
+    # gate and up scales out of one descriptor's reach (and seven rows, which go one by one): the chain's own bits, in two to four passes over a row
     c = _shared_block_case(rows, d, f, 0x4A0 + rows)
     k = ctx()
     t = {n: [dev(a) for a in c[n]] for n in ("gate", "up", "down")}

@@ -90,4 +90,8 @@ bool geglu_split_ok(const tf_projection *gate, long ldx);
 int32_t launch_geglu_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const half_t *x, long ldx, half_t *a_out,
                            long lda, int m, tf_dtype sd);
 
+bool shared8_split_ok(const tf_projection *gate, long ldx);
+int32_t launch_shared8_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const half_t *x,
+                             long ldx, half_t *acts, half_t *y, long ldy, int m, tf_dtype sd);
+
 }  // namespace tfk

@@ -682,6 +682,7 @@ int32_t shared8_block_mfma(tf_ctx *ctx, hipStream_t st, const tf_projection *gat
     if (!(aligned16(w[0]) && aligned16(w[1]) && aligned16(w[2]) && aligned16(x) && x_stride % 8 == 0 && d % 64 == 0 && f % 64 == 0 &&
           (sd == TF_BF16 || sd == TF_FP16) && rows <= 65535u * 32u))
         return TF_ERR_UNAVAILABLE;
+    if (shared8_split_ok(gate, (long)x_stride)) return launch_shared8_split(ctx, st, gate, up, down, x, (long)x_stride, acts, y, (long)y_stride, (int)rows, sd);
     const uint8_t *sc[3], *bi[3];
     const tf_projection *proj[3] = {gate, up, down};
     for (int p = 0; p < 3; ++p) {
@@ -788,11 +789,11 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
         rc8 = shared8_block(ctx, st, gate, up, down, xp, x_stride_elements, yp, y_stride_elements, query_count, acts8, scale_dtype);
         if (rc8 != TF_ERR_UNAVAILABLE) return rc8;
     }
-    // The single-row chain over many rows (fewer than kSharedBlockMinRows, or gate and up arrays out of each other's reach) in two launches, with the
-    // same bits, where every row would take the chain's vector kernels and the context holds the activations: 7 / 53 / 512 rows of d 2816,
-    // f 2112 64 / 423 / 4370 -> 26 / 84 / 723 us
+    // The single-row chain over a block of rows whose gate and up arrays lie out of each other's reach, in two launches and with the same
+    // bits, where every row would take the chain's vector kernels and the context holds the activations, as it does for a block whose
+    // arrays are near: 53 / 512 rows of d 2816, f 2112 423 / 4370 -> 84 / 723 us.  Fewer rows than a block stay in the caller's scratch.
     const uint64_t one_row = (uint64_t)intermediate * 2;
-    if (!block_path && weight_bits == 4 && pointers && even && query_count >= 2 && (uint64_t)query_count * one_row <= ctx->shared_block_acts_bytes &&
+    if (!block_path && weight_bits == 4 && pointers && even && query_count >= kSharedBlockMinRows && (uint64_t)query_count * one_row <= ctx->shared_block_acts_bytes &&
         intermediate % TF_GROUP_SIZE == 0 && d % TF_GROUP_SIZE == 0 && scratch_gate_offset + one_row <= scratch_gate_length &&
         scratch_up_offset + one_row <= scratch_up_length && scratch_act_offset + one_row <= scratch_act_length && scratch_gate_offset % 2 == 0 &&
         scratch_up_offset % 2 == 0 && aligned16(at(scratch_act, scratch_act_offset))) {

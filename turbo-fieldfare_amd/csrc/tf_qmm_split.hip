@@ -33,10 +33,12 @@ struct SplitArgs {
 __device__ __forceinline__ void lds_write4(uint32_t addr, uint32_t v) { asm volatile("ds_write_b32 %0, %1" ::"v"(addr), "v"(v) : "memory"); }
 
 // GP: most pairs of groups a wave may be given
-template <int MT, int NJ, int NW, int GP>
+template <int BITS, int MT, int NJ, int NW, int GP>
 struct SplitGeom {
-    static constexpr int kStage = MT * 4096 + NJ * 1024;
-    static constexpr int kCopies = MT * 4 + NJ;
+    static constexpr int kWRow = 8 * BITS;                    // bytes of a weight row per step
+    static constexpr int kWCopies = NJ * BITS / 4;
+    static constexpr int kStage = MT * 4096 + NJ * 32 * kWRow;
+    static constexpr int kCopies = MT * 4 + kWCopies;
     static constexpr int kSB = GP * 2 * 64 * 4;               // [group][row]: half(s) | half(b) << 16
     static constexpr int kWave = 3 * kStage + kSB;
     static constexpr int kSumRow = 32 * NJ + 4;                    // floats per row of a wave's sums
@@ -44,9 +46,9 @@ struct SplitGeom {
     static constexpr int kLds = NW * (kWave > kSums ? kWave : kSums);
 };
 
-template <int SD, int MT, int NJ, int NW, int GP, bool GEGLU>
+template <int BITS, int SD, int MT, int NJ, int NW, int GP, bool GEGLU>
 __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
-    typedef SplitGeom<MT, NJ, NW, GP> G;
+    typedef SplitGeom<BITS, MT, NJ, NW, GP> G;
     __shared__ __align__(128) uint8_t lds[G::kLds];
     static_assert(!GEGLU || NJ == 2, "a gate tile and an up tile");
     constexpr int kCols = GEGLU ? 32 : 32 * NJ;
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
     const int groups = a.K >> 6, pairs = (groups + 1) >> 1;
     const int g0 = 2 * (pairs * wave / NW), g1 = min(groups, 2 * (pairs * (wave + 1) / NW)), steps = g1 - g0;
     const uint32_t base = (uint32_t)(uintptr_t)lds + (uint32_t)(wave * G::kWave), sb_area = base + 3 * G::kStage;
-    const uint32_t row_bytes = (uint32_t)a.K >> 1;
+    const uint32_t row_bytes = (uint32_t)a.K * BITS / 8u;
 
     float16_t acc[MT][NJ];
 #pragma unroll
@@ -100,25 +102,26 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
             }
         }
         // copies: activation rows 8 q + lane / 8, chunk (lane & 7) ^ ((row / 2) & 7); weight rows 32 q + lane / 2, 16-byte half
-        // (lane & 1) ^ ((row / 4) & 1).  Rows past the matrix repeat its last row; what they produce is not stored.
+        // (lane & 1) ^ ((row / 4) & 1), or with 8 bits rows 16 q + lane / 4, piece (lane & 3) ^ ((row / 4) & 3).  Rows past the matrix repeat its last row; what they produce is not stored.
         qmm_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(a.X + (size_t)m0 * a.ldx), 0, (int)0xFFFFFFFFu, 0x00020000);
         qmm_rsrc_t wr[2];
         wr[0] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.W[0] + (size_t)n0 * row_bytes), 0, (int)0xFFFFFFFFu, 0x00020000);
         wr[1] = GEGLU ? __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t *>(a.W[1] + (size_t)n0 * row_bytes), 0, (int)0xFFFFFFFFu, 0x00020000) : wr[0];
-        uint32_t xoff[MT * 4], woff[NJ];
+        uint32_t xoff[MT * 4], woff[G::kWCopies];
 #pragma unroll
         for (int q = 0; q < MT * 4; ++q) {
             const int r = 8 * q + (lane >> 3);
             xoff[q] = (uint32_t)(min(m0 + r, a.M - 1) - m0) * (uint32_t)(a.ldx * 2) + (uint32_t)(((lane & 7) ^ ((r >> 1) & 7)) * 16);
         }
 #pragma unroll
-        for (int q = 0; q < NJ; ++q) {
-            const int r = 32 * q + (lane >> 1);
-            woff[q] = (uint32_t)(min(n0 + (GEGLU ? (r & 31) : r), a.N - 1) - n0) * row_bytes + (uint32_t)(((lane & 1) ^ ((r >> 2) & 1)) * 16);
+        for (int q = 0; q < G::kWCopies; ++q) {
+            constexpr int kPieces = BITS / 2;      // 16-byte pieces of a row per step
+            const int r = (64 / kPieces) * q + lane / kPieces;
+            woff[q] = (uint32_t)(min(n0 + (GEGLU ? (r & 31) : r), a.N - 1) - n0) * row_bytes + (uint32_t)(((lane % kPieces) ^ ((r >> 2) % kPieces)) * 16);
         }
         auto copy = [&](int g, uint32_t stage) {
 #pragma unroll
-            for (int q = 0; q < NJ; ++q) lds_copy16(wr[q], stage + MT * 4096 + q * 1024, woff[q], g * 32);
+            for (int q = 0; q < G::kWCopies; ++q) lds_copy16(wr[q * NJ / G::kWCopies], stage + MT * 4096 + q * 1024, woff[q], g * G::kWRow);
 #pragma unroll
             for (int q = 0; q < MT * 4; ++q) lds_copy16(xr, stage + q * 1024, xoff[q], g * 128);
         };
@@ -129,7 +132,7 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
         uint32_t shift = 0;
         if constexpr (SD == 0) {
             // the power of two of the lane's row over the wave's run: every |s| < 2^(es - 126), every |b| < 2^(eb - 126), and
-            // 2^(140 - max(es + 4, eb)) brings 15 |s| + |b| below 2^15
+            // 2^(140 - max(es + BITS, eb)) brings q |s| + |b| below 2^15
             u16x2 es = {0, 0}, eb = {0, 0};
             bool small = false;
 #pragma unroll
@@ -140,8 +143,8 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
                 small = small || (lo != 0u && lo < 113u) || (hi != 0u && hi < 113u);      // 2^-14 = fp16's smallest normal number
             }
             if (__builtin_amdgcn_ballot_w64(small) != 0ull) {
-                const uint32_t top = max(((uint32_t)max(es[0], es[1]) >> 7) + 4u, (uint32_t)max(eb[0], eb[1]) >> 7);
-                const int e = top == 4u ? 0 : min(max(140 - (int)top, -100), 100);
+                const uint32_t top = max(((uint32_t)max(es[0], es[1]) >> 7) + (uint32_t)BITS, (uint32_t)max(eb[0], eb[1]) >> 7);
+                const int e = top == (uint32_t)BITS ? 0 : min(max(140 - (int)top, -100), 100);
                 shift = (uint32_t)e << 23;
                 const float p = __uint_as_float((uint32_t)(127 - e) << 23);
                 post[0] = __shfl(p, i, kWave);
@@ -159,16 +162,20 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
         }
 
         struct Frags {
-            u32x4 x[MT][4], w[NJ];
+            u32x4 x[MT][4], w[NJ][BITS / 4];
             uint32_t sb[NJ];
         };
         const uint32_t x0 = (uint32_t)i * 128u + ((((uint32_t)kb * 4u) ^ (uint32_t)((i >> 1) & 7)) << 4);
-        const uint32_t w0 = MT * 4096 + (uint32_t)i * 32u + ((uint32_t)(kb ^ ((i >> 2) & 1)) << 4);
+        const uint32_t w0 = MT * 4096 + (uint32_t)i * (uint32_t)G::kWRow + (BITS == 4 ? (uint32_t)(kb ^ ((i >> 2) & 1)) << 4 : (uint32_t)((2 * kb) ^ ((i >> 2) & 3)) << 4);
         const uint32_t sb0 = sb_area + (uint32_t)i * 4u;
         auto read = [&](Frags &f, uint32_t stage, int t) {
             const uint32_t xa = stage + x0, wa = stage + w0, sa = sb0 + (uint32_t)t * 256u;
-            f.w[0] = lds_read16<0>(wa);
-            if constexpr (NJ > 1) f.w[1] = lds_read16<1024>(wa);
+            f.w[0][0] = lds_read16<0>(wa);
+            if constexpr (NJ > 1) f.w[NJ - 1][0] = lds_read16<32 * G::kWRow>(wa);
+            if constexpr (BITS == 8) {                 // the other half of the lane's 32 bytes: the piece beside it
+                f.w[0][BITS / 4 - 1] = lds_read16<0>(wa ^ 16u);
+                if constexpr (NJ > 1) f.w[NJ - 1][BITS / 4 - 1] = lds_read16<32 * G::kWRow>(wa ^ 16u);
+            }
             f.sb[0] = lds_read4<0>(sa);
             if constexpr (NJ > 1) f.sb[1] = lds_read4<128>(sa);
 #pragma unroll
@@ -179,8 +186,10 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
         };
         // all reads of f have landed; also keeps the copies that follow behind them
         auto landed = [&](Frags &f) {
-            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.w[0]), "+v"(f.sb[0]), "+v"(f.x[0][0]), "+v"(f.x[0][1]), "+v"(f.x[0][2]), "+v"(f.x[0][3]) : : "memory");
-            if constexpr (NJ > 1) asm volatile("" : "+v"(f.w[1]), "+v"(f.sb[1]));
+            asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(f.w[0][0]), "+v"(f.sb[0]), "+v"(f.x[0][0]), "+v"(f.x[0][1]), "+v"(f.x[0][2]), "+v"(f.x[0][3]) : : "memory");
+            if constexpr (NJ > 1) asm volatile("" : "+v"(f.w[NJ - 1][0]), "+v"(f.sb[NJ - 1]));
+            if constexpr (BITS == 8) asm volatile("" : "+v"(f.w[0][BITS / 4 - 1]));
+            if constexpr (BITS == 8 && NJ > 1) asm volatile("" : "+v"(f.w[NJ - 1][BITS / 4 - 1]));
             if constexpr (MT > 1) asm volatile("" : "+v"(f.x[1][0]), "+v"(f.x[1][1]), "+v"(f.x[1][2]), "+v"(f.x[1][3]));
         };
         uint32_t mask = 0x00F0000Fu;
@@ -191,12 +200,17 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
 #pragma unroll
                 for (int j = 0; j < NJ; ++j) {
                     const half2_t sb = as_half2(f.sb[j]), s2 = {sb[0], sb[0]}, b2 = {sb[1], sb[1]};
-                    const half2_t off = {(half_t)-1024.0f, (half_t)-64.0f};
+                    const half2_t off = {(half_t)-1024.0f, (half_t)(BITS == 4 ? -64.0f : -1024.0f)};
                     u32x4 o;
 #pragma unroll
                     for (int p = 0; p < 4; ++p) {
-                        const uint32_t both = __builtin_amdgcn_perm(0u, f.w[j][d], 0x0c000c00u | ((uint32_t)p << 16) | (uint32_t)p);
-                        const half2_t q = as_half2((both & mask) | 0x54006400u) + off;          // 1024 + q, 64 + q: exact
+                        half2_t q;                                       // 1024 + q and 64 + q, or 1024 + q twice: exact
+                        if constexpr (BITS == 4) {
+                            const uint32_t both = __builtin_amdgcn_perm(0u, f.w[j][0][d], 0x0c000c00u | ((uint32_t)p << 16) | (uint32_t)p);
+                            q = as_half2((both & mask) | 0x54006400u) + off;
+                        } else {
+                            q = as_half2(__builtin_amdgcn_perm(0x64646464u, f.w[j][(d >> 1) % (BITS / 4)][2 * (d & 1) + (p >> 1)], (p & 1) ? 0x04030402u : 0x04010400u)) + off;
+                        }
                         o[p] = as_u32(__builtin_elementwise_fma(q, s2, b2));
                     }
                     wf[j] = __builtin_bit_cast(half8_t, o);
@@ -264,7 +278,7 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
         if constexpr (GEGLU) {
             const f32x4 up = total(32 + col);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = gelu_tanh_fast((float)(half_t)v[e]) * (float)(half_t)up[e];
+            for (int e = 0; e < 4; ++e) v[e] = (BITS == 4 ? gelu_tanh_fast((float)(half_t)v[e]) : gelu_tanh((float)(half_t)v[e])) * (float)(half_t)up[e];
         }
         half_t *y = a.Y + (size_t)m * a.ldy + n;
         if (a.vec) {
@@ -277,12 +291,12 @@ __global__ __launch_bounds__(64 * NW) void qmm_split_kernel(SplitArgs a) {
     }
 }
 
-template <int MT, int NJ, int NW, int GP, bool GEGLU>
+template <int BITS, int MT, int NJ, int NW, int GP, bool GEGLU>
 void launch_split(hipStream_t st, const SplitArgs &a, tf_dtype sd) {
     constexpr int cols = GEGLU ? 32 : 32 * NJ;
     const dim3 grid((uint32_t)((a.N + cols - 1) / cols) * (uint32_t)((a.M + 32 * MT - 1) / (32 * MT)));
-    if (sd == TF_BF16) hipLaunchKernelGGL((qmm_split_kernel<0, MT, NJ, NW, GP, GEGLU>), grid, dim3(64 * NW), 0, st, a);
-    else hipLaunchKernelGGL((qmm_split_kernel<1, MT, NJ, NW, GP, GEGLU>), grid, dim3(64 * NW), 0, st, a);
+    if (sd == TF_BF16) hipLaunchKernelGGL((qmm_split_kernel<BITS, 0, MT, NJ, NW, GP, GEGLU>), grid, dim3(64 * NW), 0, st, a);
+    else hipLaunchKernelGGL((qmm_split_kernel<BITS, 1, MT, NJ, NW, GP, GEGLU>), grid, dim3(64 * NW), 0, st, a);
 }
 
 }  // namespace
@@ -315,14 +329,14 @@ int32_t launch_qmm_split(tf_ctx *ctx, hipStream_t st, int variant, const uint8_t
     const SplitArgs a = {{w, w}, {s, s}, {b, b}, x, ldx, y, ldy, m, n, k, aligned(y, 8) && n % 4 == 0 && ldy % 4 == 0};
     const bool wide = k > 4096;       // twice the scales to keep
     if (variant == kSplit32x32) {
-        if (wide) launch_split<1, 1, 8, 8, false>(st, a, sd);
-        else launch_split<1, 1, 8, 4, false>(st, a, sd);
+        if (wide) launch_split<4, 1, 1, 8, 8, false>(st, a, sd);
+        else launch_split<4, 1, 1, 8, 4, false>(st, a, sd);
     } else if (variant == kSplit64x32) {
-        if (wide) launch_split<2, 1, 4, 16, false>(st, a, sd);
-        else launch_split<2, 1, 4, 8, false>(st, a, sd);
+        if (wide) launch_split<4, 2, 1, 4, 16, false>(st, a, sd);
+        else launch_split<4, 2, 1, 4, 8, false>(st, a, sd);
     } else {
-        if (wide) launch_split<2, 2, 4, 16, false>(st, a, sd);
-        else launch_split<2, 2, 4, 8, false>(st, a, sd);
+        if (wide) launch_split<4, 2, 2, 4, 16, false>(st, a, sd);
+        else launch_split<4, 2, 2, 4, 8, false>(st, a, sd);
     }
     return check_launch(ctx, "int4_qmm");
 }
@@ -336,9 +350,30 @@ int32_t launch_geglu_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gat
                          {at(gate->scales, gate->scales_offset), at(up->scales, up->scales_offset)},
                          {at(gate->biases, gate->biases_offset), at(up->biases, up->biases_offset)},
                          x, ldx, a_out, lda, m, f, d, aligned(a_out, 8) && f % 4 == 0 && lda % 4 == 0};
-    if (d > 4096) launch_split<1, 2, 4, 16, true>(st, a, sd);
-    else launch_split<1, 2, 8, 4, true>(st, a, sd);
+    if (d > 4096) launch_split<4, 1, 2, 4, 16, true>(st, a, sd);
+    else launch_split<4, 1, 2, 8, 4, true>(st, a, sd);
     return check_launch(ctx, "prefill_shared_expert gate/up");
+}
+
+// The 8-bit shared expert of a block of rows (what a wave keeps of scales ends at 4096 columns).
+bool shared8_split_ok(const tf_projection *gate, long ldx) { return gate->cols <= 4096 && gate->rows <= 4096 && ldx <= (1l << 24); }
+
+int32_t launch_shared8_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const half_t *x,
+                             long ldx, half_t *acts, half_t *y, long ldy, int m, tf_dtype sd) {
+    const int f = (int)gate->rows, d = (int)gate->cols;
+    auto blocks = [&](int n, int rows, int cols) { return (int64_t)((m + (int64_t)rows - 1) / rows) * ((n + (int64_t)cols - 1) / cols); };
+    const SplitArgs a1 = {{at(gate->weights, gate->weights_offset), at(up->weights, up->weights_offset)},
+                          {at(gate->scales, gate->scales_offset), at(up->scales, up->scales_offset)},
+                          {at(gate->biases, gate->biases_offset), at(up->biases, up->biases_offset)},
+                          x, ldx, acts, (long)f, m, f, d, aligned(acts, 8) && f % 4 == 0};
+    if (blocks(f, 32, 32) <= 256) launch_split<8, 1, 2, 4, 8, true>(st, a1, sd);
+    else launch_split<8, 2, 2, 4, 8, true>(st, a1, sd);
+    const uint8_t *w = at(down->weights, down->weights_offset), *s = at(down->scales, down->scales_offset), *b = at(down->biases, down->biases_offset);
+    const SplitArgs a2 = {{w, w}, {s, s}, {b, b}, acts, (long)f, y, ldy, m, d, f, aligned(y, 8) && d % 4 == 0 && ldy % 4 == 0};
+    if (blocks(d, 32, 32) <= 256) launch_split<8, 1, 1, 8, 4, false>(st, a2, sd);
+    else if (blocks(d, 64, 32) <= 256) launch_split<8, 2, 1, 4, 8, false>(st, a2, sd);
+    else launch_split<8, 2, 2, 4, 8, false>(st, a2, sd);
+    return check_launch(ctx, "shared expert 8-bit block");
 }
 
 }  // namespace tfk
