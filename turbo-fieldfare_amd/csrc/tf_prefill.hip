@@ -91,8 +91,17 @@ __global__ __launch_bounds__(64) void prefill_select_kernel(float *logits, const
     float *row = logits + (size_t)t * num_experts;
     if (planes > 0) {
         for (uint32_t e = threadIdx.x; e < num_experts; e += 64) {
+            // sixteen planes at a time, all requested before the first is added (one by one, eight planes of two entries a lane were
+            // sixteen trips to memory: 9.0 us for 128 tokens)
             float v = 0.0f;
-            for (uint32_t p = 1; p <= planes; ++p) v += row[p * plane_stride + e];
+            for (uint32_t p0 = 1; p0 <= planes; p0 += 16) {
+                float part[16];
+#pragma unroll
+                for (uint32_t i = 0; i < 16; ++i) part[i] = row[min(p0 + i, planes) * plane_stride + e];
+#pragma unroll
+                for (uint32_t i = 0; i < 16; ++i)
+                    if (p0 + i <= planes) v += part[i];
+            }
             row[e] = v;
         }
     }
