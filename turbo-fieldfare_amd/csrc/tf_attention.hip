@@ -332,7 +332,7 @@ __device__ __forceinline__ void visible_keys(const PrefillShape &s, uint32_t t, 
 // With several chunks the block leaves an unnormalised partial state (m, d, o) per column for the merge kernel; with one
 // it writes the rows itself.  HD in {64, 128, 256, 512}, G in {1, 2, 4, 8, 16}, rows 16-byte aligned.
 constexpr int kPrefillKeys = 32, kPrefillCols = 64;
-constexpr uint32_t kMaxPrefillChunks = 16, kMinChunkKeys = 256;
+constexpr uint32_t kMaxPrefillChunks = 16, kMinChunkKeys = 256, kShortChunkKeys = 128;
 constexpr uint32_t kXcds = 8;
 
 typedef __amdgpu_buffer_rsrc_t attn_rsrc_t;
@@ -1096,6 +1096,12 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
         const uint32_t target = (uint32_t)ctx->num_cus * (hd > 256 ? 1u : 2u);
         uint32_t chunks = std::max(1u, std::min({(target + base - 1) / base, span / kMinChunkKeys, kMaxPrefillChunks}));
         auto states_of = [&](uint32_t c) { return (size_t)s.count * s.num_q_heads * c; };
+        // blocks for less than three eighths of the compute units: shorter chunks (33 queries over 1033 keys of a sliding window 22.4 -> 19.2 us,
+        // 53 over 1076 23.1 -> 20.4; with more blocks the merge takes what the shorter walk gives, 200 over 1200 29.7 -> 32.9)
+        if (base * chunks * 8u <= (uint32_t)ctx->num_cus * 3u) {
+            const uint32_t more = std::min({(target + base - 1) / base, span / kShortChunkKeys, kMaxPrefillChunks});
+            if (more > chunks && states_of(more) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes) chunks = more;
+        }
         float *m = nullptr, *d = nullptr, *o = nullptr, *scratch = nullptr;
         if (chunks > 1) {
             const int32_t rc = attention_scratch(ctx, states_of(chunks) * (2 + (size_t)hd), scratch);
