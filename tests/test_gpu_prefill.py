@@ -667,6 +667,7 @@ def test_int4_qmm_on_matrix_cores_with_scales_below_fp16_normal_range(m, n, k, l
     (53, 2816, 2112, True, 0), (31, 40, 4160, False, 2), (40, 33, 8192, True, 0),    # an odd number of groups over eight waves; more than 4096; rows stored value by value
     (70, 2752, 1024, False, 0), (130, 2720, 4160, True, 0),                          # 64 x 32 tiles (258 and 425 tiles of 32 x 32)
     (65, 4130, 1088, False, 0), (129, 4100, 4224, False, 2),                         # 64 x 64 tiles (258 and 387 tiles of 64 x 32), and with wide scale areas
+    (700, 4090, 1024, False, 0), (513, 8192, 1088, True, 0), (200, 250, 832, False, 2),   # the tile kernel's tiles of 64 rows, their remainders in rows and columns
 ])
 def test_int4_qmm_with_the_contraction_split_between_waves(m, n, k, fp16_scales, shift):
     # against 64-bit sums of the exact weights; the bound at the end is what rounding weights and outputs to fp16 amounts to
