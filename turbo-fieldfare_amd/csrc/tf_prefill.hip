@@ -815,10 +815,11 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     const bool p1_fast = blobs16 && hidden16 && off.gate_W_off % 16 == 0 && off.up_W_off % 16 == 0;
     const bool dn_fast = blobs16 && acts16 && off.down_W_off % 16 == 0;
     int32_t rc;
-    // Fewer than five pairs per expert on average: the quad kernels serve the call (chunks longer than their LDS image, if any,
-    // in batches).  From there on so few chunks are short that the matrix-core tile kernels are faster (128 experts: 64 tokens
-    // 151 us on the quad kernels against 164 us on the tiles; 80 tokens 178 against 173 us; 96 tokens 187 against 173 us; running
-    // both families in one call, each on its chunks, was never better than the better of the two).
+    // Fewer than five pairs per expert on average: the quad kernels serve the call (chunks longer than their LDS image in batches).
+    // From there on so few chunks are short that the matrix-core tile kernels are faster (top 8 of 128 experts, rows with a common
+    // direction, quad against tiles: 48 tokens 86 / 87 us, 64: 109 / 94, 72: 118 / 124, 80: 126 / 114, 96: 134 / 110, 128: 163 / 111; below
+    // the line the quad kernels also keep q s + b in 32 bits where the tiles round a weight to fp16.  Running both families in one
+    // call, each on its chunks, was never better than the better of the two).
     const int p1_passes = ((g.d >> 5) + 15) / 16, dn_passes = ((g.f >> 5) + 7) / 8;
     const bool quad_ok = p1_fast && dn_fast && acts16 && g.d <= kQuadMaxD && p1_passes <= 6 && g.f <= kQuadMaxF && dn_passes <= 4 && g.d % 8 == 0 &&
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;
