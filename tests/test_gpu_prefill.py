@@ -393,10 +393,22 @@ def test_quad_kernels_long_chunks_and_row_widths(T, E, d, f):
     check_against_oracle(r, T, d, f, top_k, abs_tol=1e-3 * max(1.0, scale))
 
 
+def run_quad_work_list(r, chunks, T, E, d, f, top_k):
+    n = T * top_k
+    k = ctx()
+    koff = tfk.ExpertOffsets(*r["off"].as_tuple())
+    d_pool, d_hidden, d_pairs, d_chunks, d_n = dev(r["pool"]), dev(r["hidden"]), dev(r["sorted_pairs"].view(np.uint32)), dev(np.array(chunks, np.uint32)), dev(np.array([len(chunks)], np.uint32))
+    acts, partials = zeros_bytes(n * f * 2), zeros_bytes(n * d * 2)
+    k.check(k.lib.tf_prefill_grouped_routed_moe_resident(k.handle, None, d_hidden.data_ptr(), 0, d, d_pairs.data_ptr(), d_chunks.data_ptr(), d_n.data_ptr(),
+                                                         len(chunks), n, d_pool.data_ptr(), r["stride"], E, C.byref(koff), acts.data_ptr(),
+                                                         partials.data_ptr(), d, f, top_k, tfk.TF_BF16))
+    return host(partials, np.uint16, n * d)
+
+
 @pytest.mark.parametrize("T,E,run", [(75, 128, 1), (40, 128, 3), (31, 128, 128), (20, 40, 9)])
 def test_quad_kernels_share_out_any_work_list(T, E, run):
-    # The blocks share out batches of up to eight pairs (more than 512 chunks, or more batches than blocks: whole chunks).  A pair's sums do
-    # not depend on whom it shares a batch with, so however the runs are cut the outputs are those of the device grouping's list.
+    # The blocks share out batches of up to eight pairs (more than 512 chunks: whole chunks).  A pair's sums do not depend on whom it
+    # shares a batch with, so however the runs are cut the outputs are those of the device grouping's list.
     d, f, top_k = 128, 64, 8
     r = resident_pipeline(T, E, d, f, top_k, 0x4A00 + T + run, zipf=True, from_router=False)
     n = T * top_k
@@ -410,14 +422,36 @@ def test_quad_kernels_share_out_any_work_list(T, E, run):
         chunks.append((int(pairs["expert"][at]), at, end - at))
         at = end
     assert (len(chunks) > 512) == (run == 1)
-    k = ctx()
-    koff = tfk.ExpertOffsets(*r["off"].as_tuple())
-    d_pool, d_hidden, d_pairs, d_chunks, d_n = dev(r["pool"]), dev(r["hidden"]), dev(pairs.view(np.uint32)), dev(np.array(chunks, np.uint32)), dev(np.array([len(chunks)], np.uint32))
-    acts, partials = zeros_bytes(n * f * 2), zeros_bytes(n * d * 2)
-    k.check(k.lib.tf_prefill_grouped_routed_moe_resident(k.handle, None, d_hidden.data_ptr(), 0, d, d_pairs.data_ptr(), d_chunks.data_ptr(), d_n.data_ptr(),
-                                                         len(chunks), n, d_pool.data_ptr(), r["stride"], E, C.byref(koff), acts.data_ptr(),
-                                                         partials.data_ptr(), d, f, top_k, tfk.TF_BF16))
-    assert np.array_equal(host(partials, np.uint16, n * d), r["partials"])
+    assert np.array_equal(run_quad_work_list(r, chunks, T, E, d, f, top_k), r["partials"])
+
+
+@pytest.mark.parametrize("T,E,run,singles,blocks_per_cu", [(375, 640, 9, 200, 3), (1400, 2300, 24, 0, 5)])
+def test_quad_kernels_given_more_batches_than_blocks(T, E, run, singles, blocks_per_cu):
+    # At most 512 chunks whose batches of eight pairs outnumber the blocks of the launch (three a compute unit for gate / up, five for
+    # down): a block's share is cut in whole chunks, whose batches it takes one after the other.
+    import torch
+    d, f, top_k = 128, 64, 8
+    n = T * top_k
+    counts = [run] * ((n - singles) // run) + [1] * singles
+    counts += [n - sum(counts)] if sum(counts) < n else []
+    assert len(counts) <= 512 and n < 5 * E
+    assert sum((c + 7) // 8 for c in counts) > blocks_per_cu * torch.cuda.get_device_properties(0).multi_processor_count
+    base = resident_pipeline(16, 128, d, f, top_k, 0x4B00 + T, from_router=False)
+    pairs = np.zeros(n, tfo.PAIR_DTYPE)
+    rng = np.random.default_rng(0x4B10 + T)
+    order = rng.permutation(n)
+    pairs["token"], pairs["rank"], pairs["expert"] = order // top_k, order % top_k, np.repeat(np.arange(len(counts)), counts)
+    hidden = rng.standard_normal((T, d)).astype(np.float16).view(np.uint16)
+    r = dict(off=base["off"], stride=base["stride"], pool=np.resize(base["pool"].reshape(128, base["stride"]), (E, base["stride"])).ravel(),   # 128 blobs in turn
+             hidden=hidden, sorted_pairs=pairs)
+    starts = np.cumsum(counts) - counts
+    whole = [(e, int(at), int(c)) for e, (at, c) in enumerate(zip(starts, counts))]
+    cut = [(e, p, min(4, at + c - p)) for e, at, c in whole for p in range(at, at + c, 4)]      # more than 512 chunks: no batches are counted
+    assert len(cut) > 512
+    got = run_quad_work_list(r, whole, T, E, d, f, top_k)
+    assert np.array_equal(got, run_quad_work_list(r, cut, T, E, d, f, top_k))
+    want = tfo.from_f16_bits(tfo.prefill_route_partials(pairs, T, hidden.ravel(), d, r["pool"], r["stride"], r["off"], top_k, d, f, fill_bits=0, threads=8))
+    assert within_north_star(tfo.from_f16_bits(got), want, abs_=1e-3 * max(1.0, float(np.max(np.abs(want)))))
 
 
 @pytest.mark.parametrize("T,E,d,f,fp16_scales,pad", [(3, 16, 1536, 128, False, 0), (5, 64, 2048, 256, True, 8), (2, 32, 4096, 64, False, 0),

@@ -93,7 +93,7 @@ struct QuadSpan {
     tf_prefill_group run[2];          // the pairs of unit0 and of the unit after it
     bool units;                       // false: too many chunks or units for this scheme, a "unit" is a whole chunk (batches in the block's own loop)
 };
-// scratch: 64 bytes of LDS that nothing else uses until the block's next barrier; 256 threads, all call
+// scratch: 64 bytes of LDS that nothing else uses until the block's next barrier, and free again when this returns; 256 threads, all call
 __device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_chunks, uint32_t max_pairs, uint32_t tiles_per_unit, uint32_t *scratch) {
     QuadSpan sp;
     uint32_t units = n_chunks;
@@ -122,7 +122,10 @@ __device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_ch
         first = before + sum - batches[0] - batches[1];
         units = uniform_u32(total);
         sp.units = units <= gridDim.x;
-        if (!sp.units) units = n_chunks;
+        if (!sp.units) {
+            units = n_chunks;
+            __syncthreads();          // every wave has read the sums: the caller may write over them (the other way out ends with a barrier too)
+        }
     }
     const uint32_t per_unit = units ? gridDim.x / units : 0u;
     if (per_unit >= kQuadMinBlocksPerUnit) {
