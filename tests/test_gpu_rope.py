@@ -66,6 +66,22 @@ def test_fused_qkv_epilogue(d, nq, nkv, pairs, position, theta):
         same_up_to_rounding(got, w, ulps=2, share=0.05)
 
 
+@pytest.mark.parametrize("d,nq", [(256, 3), (512, 1), (64, 6), (128, 4)])
+def test_fused_qkv_epilogue_of_query_heads_alone(d, nq):
+    # no k and v heads: their arguments and the k weight are placeholders, the query heads come out as beside k and v heads
+    k = ctx()
+    q, kk, v = (tfo.to_f16_bits(rand(n * d, s)) for n, s in ((nq, 21), (2, 22), (2, 23)))
+    wq, wk = tfo.bf16_bits_array(1.0 + 0.1 * rand(d, 24)), tfo.bf16_bits_array(1.0 + 0.1 * rand(d, 25))
+    t = dict(q=dev(q), k=dev(kk), v=dev(v), wq=dev(wq), wk=dev(wk))
+    k.check(k.lib.tf_fused_qkv_epilogue(k.handle, None, t["q"].data_ptr(), 0, t["k"].data_ptr(), 0, t["v"].data_ptr(), 0, t["wq"].data_ptr(), 0,
+                                        t["wk"].data_ptr(), 0, d, nq, 2, 77, 1e4, d // 4, 1e-6))
+    alone, nothing = dev(q), dev(np.full(1, 0x7FC0, np.uint16))
+    k.check(k.lib.tf_fused_qkv_epilogue(k.handle, None, alone.data_ptr(), 0, nothing.data_ptr(), 0, nothing.data_ptr(), 0, t["wq"].data_ptr(), 0,
+                                        nothing.data_ptr(), 0, d, nq, 0, 77, 1e4, d // 4, 1e-6))
+    assert np.array_equal(host(alone, np.uint16), host(t["q"], np.uint16))
+    assert host(nothing, np.uint16)[0] == 0x7FC0
+
+
 def test_contract():
     k = ctx()
     data = dev(np.zeros(512, np.uint16))

@@ -21,3 +21,11 @@ def test_host_mirror_compiles_and_groups(tmp_path):
     subprocess.run(cmd, check=True, cwd=ROOT)
     out = subprocess.run([str(exe)], check=True, capture_output=True, text=True)
     assert "host mirror ok" in out.stdout
+
+
+@pytest.mark.skipif(shutil.which("g++") is None, reason="needs g++")
+def test_norm_rope_waves_read_only_heads_and_weights_that_exist(tmp_path):
+    exe = tmp_path / "epilogue_heads_check"
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-Werror", "-o", str(exe), str(ROOT / "tests" / "epilogue_heads_check.cpp")], check=True, cwd=ROOT)
+    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    assert out.returncode == 0 and "epilogue heads ok" in out.stdout, out.stdout

@@ -6,6 +6,7 @@
 
 #include "tf_common.hpp"
 #include "tf_context.hpp"
+#include "tf_epilogue_heads.hpp"
 
 using namespace tfk;
 
@@ -60,14 +61,15 @@ __global__ __launch_bounds__(256) void qkv_epilogue_wave_kernel(half_t *q, half_
     typedef half_t piece_t __attribute__((ext_vector_type(EPL)));
     __shared__ float cosine[kHalfDim], sine[kHalfDim];
     const uint32_t t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t heads = num_q_heads + 2 * num_kv_heads, head0 = blockIdx.x * 4 * heads_per_wave + wave;
+    const EpilogueHeads kinds = {num_q_heads, num_kv_heads};
+    const uint32_t heads = kinds.count(), head0 = blockIdx.x * 4 * heads_per_wave + wave;
     auto head_at = [&](uint32_t h) {
         return h < num_q_heads ? q + (size_t)t * q_token_stride + (size_t)h * kHeadDim
                : h < num_q_heads + num_kv_heads ? k + (size_t)t * kv_token_stride + (size_t)(h - num_q_heads) * kHeadDim
                                                 : v + (size_t)t * kv_token_stride + (size_t)(h - num_q_heads - num_kv_heads) * kHeadDim;
     };
     auto load = [&](uint32_t h, float x[EPL]) {
-        const half_t *src = head_at(min(h, heads - 1)) + lane * EPL;
+        const half_t *src = head_at(kinds.read(h)) + lane * EPL;
         if constexpr (VEC) {
             const piece_t p = *reinterpret_cast<const piece_t *>(src);
 #pragma unroll
@@ -78,7 +80,7 @@ __global__ __launch_bounds__(256) void qkv_epilogue_wave_kernel(half_t *q, half_
         }
     };
     auto load_weight = [&](uint32_t h, float wv[EPL]) {
-        const uint16_t *w = (h < num_q_heads ? q_weight : k_weight) + lane * EPL;
+        const uint16_t *w = (kinds.takes_q_weight(h) ? q_weight : k_weight) + lane * EPL;
 #pragma unroll
         for (int j = 0; j < EPL; ++j) wv[j] = bf16_to_f32(w[j]);
     };
