@@ -128,10 +128,10 @@ struct DenseArgs {
     long ldy;
     int M, N, K;
     bool rows_vectorizable;   // Y 16-byte aligned, N % 8 == 0, ldy % 8 == 0: whole 16-byte pieces of output rows
-    int bm;                   // rows of a block's tile: kQmmBM, or half of it (the same sums)
 };
-// VEC: a.rows_vectorizable holds and the tile leaves through LDS as row pieces
-template <int SD, bool VEC>
+// VEC: a.rows_vectorizable holds and the tile leaves through LDS as row pieces.  BM: rows of a block's tile, kQmmBM or half of it (the same
+// sums); known when compiling, because as an argument it cost the variant without row pieces 13 spilled registers.
+template <int SD, bool VEC, int BM = kQmmBM>
 __device__ __forceinline__ void qmm_dense_body(const DenseArgs &a, uint32_t id, uint8_t *lds) {
     const uint8_t *W = a.W, *S = a.S, *B = a.B;
     const half_t *X = a.X;
@@ -140,8 +140,8 @@ __device__ __forceinline__ void qmm_dense_body(const DenseArgs &a, uint32_t id, 
     const int M = a.M, N = a.N, K = a.K;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     uint32_t row_tile, col_tile;
-    if (!dense_tile(id, (uint32_t)(M + a.bm - 1) / (uint32_t)a.bm, (uint32_t)(N + kQmmBN - 1) / kQmmBN, row_tile, col_tile)) return;
-    const int n0 = (int)col_tile * kQmmBN + wave * kQmmWaveN, m0 = (int)row_tile * a.bm;
+    if (!dense_tile(id, (uint32_t)(M + BM - 1) / BM, (uint32_t)(N + kQmmBN - 1) / kQmmBN, row_tile, col_tile)) return;
+    const int n0 = (int)col_tile * kQmmBN + wave * kQmmWaveN, m0 = (int)row_tile * BM;
     QmmARows<4> arow;
     arow.rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(X), 0, (int)0xFFFFFFFFu, 0x00020000);
 #pragma unroll
@@ -149,7 +149,7 @@ __device__ __forceinline__ void qmm_dense_body(const DenseArgs &a, uint32_t id, 
     const uint8_t *w[2] = {W, W}, *s[2] = {S, S}, *b[2] = {B, B};
     const int row0[2] = {n0, n0 + 32}, limit[2] = {N, N};
     QmmBRows rows = make_b_rows<SD>(w, s, b, row0, limit, K >> 1, K >> 6, lane);
-    const int row_tiles = min(a.bm >> 5, (M - m0 + 31) >> 5);
+    const int row_tiles = min(BM / 32, (M - m0 + 31) >> 5);
     float16_t acc[4][2];
     zero_acc(acc);
     qmm_k_loop<SD, 4>(K >> 6, arow, rows, (uint32_t)(uintptr_t)lds, lane, row_tiles, acc);
@@ -158,31 +158,31 @@ __device__ __forceinline__ void qmm_dense_body(const DenseArgs &a, uint32_t id, 
 #pragma unroll
         for (int j = 0; j < 2; ++j)
 #pragma unroll
-            for (int mt = 0; mt < 4; ++mt)
+            for (int mt = 0; mt < BM / 32; ++mt)
 #pragma unroll
                 for (int r = 0; r < 16; ++r)
                     out_tile_put<kQmmBN>(lds, mt * 32 + acc_row(r, lane), wave * kQmmWaveN + j * 32 + acc_col(lane), acc[mt][j][r] * rows.post[j]);
         const int nb = (int)col_tile * kQmmBN;
-        out_tile_store<kQmmBN>(lds, min(a.bm, M - m0), min(kQmmBN, N - nb), [&](int row) { return Y + (size_t)(m0 + row) * ldy + nb; });
+        out_tile_store<kQmmBN>(lds, min(BM, M - m0), min(kQmmBN, N - nb), [&](int row) { return Y + (size_t)(m0 + row) * ldy + nb; });
         return;
     }
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int n = n0 + j * 32 + acc_col(lane);
 #pragma unroll
-        for (int mt = 0; mt < 4; ++mt)
+        for (int mt = 0; mt < BM / 32; ++mt)
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const int m = m0 + mt * 32 + acc_row(r, lane);
-                if (m < min(M, m0 + a.bm) && n < N) Y[(size_t)m * ldy + n] = (half_t)(acc[mt][j][r] * rows.post[j]);
+                if (m < M && n < N) Y[(size_t)m * ldy + n] = (half_t)(acc[mt][j][r] * rows.post[j]);
             }
     }
 }
 
-template <int SD, bool VEC>
+template <int SD, bool VEC, int BM>
 __global__ __launch_bounds__(256, 2) void qmm_dense_kernel(DenseArgs a) {
     __shared__ __align__(128) uint8_t lds[block_lds_bytes<4, kQmmBN>()];
-    qmm_dense_body<SD, VEC>(a, blockIdx.x, lds);
+    qmm_dense_body<SD, VEC, BM>(a, blockIdx.x, lds);
 }
 
 // Shared-expert gate and up projections of a block of rows in one pass: a wave's first column tile is 32 rows of the gate
@@ -437,7 +437,7 @@ __global__ __launch_bounds__(64 * kGroupedWaves, 8 / kGroupedWaves) void grouped
 
 DenseArgs dense_args(const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx, half_t *y, long ldy, int m, int n, int k) {
     const bool rows_vec = aligned16(y) && n % 8 == 0 && ldy % 8 == 0;   // whole 16-byte pieces of output rows
-    return DenseArgs{w, s, b, x, ldx, y, ldy, m, n, k, rows_vec, kQmmBM};
+    return DenseArgs{w, s, b, x, ldx, y, ldy, m, n, k, rows_vec};
 }
 DenseGegluArgs dense_geglu_args(const tf_projection *gate, const tf_projection *up, const half_t *x, long ldx, half_t *a, long lda, int m) {
     return DenseGegluArgs{at(gate->weights, gate->weights_offset), at(gate->scales, gate->scales_offset), at(gate->biases, gate->biases_offset),
@@ -524,20 +524,24 @@ int32_t launch_qmm_dense(tf_ctx *ctx, hipStream_t st, const uint8_t *w, const ui
         if (variant != kSplitNone) return launch_qmm_split(ctx, st, variant, w, s, b, x, ldx, y, ldy, m, n, k, sd);
     }
     const uint32_t col_tiles = (uint32_t)(n + kQmmBN - 1) / kQmmBN;
-    DenseArgs a = dense_args(w, s, b, x, ldx, y, ldy, m, n, k);
+    const DenseArgs a = dense_args(w, s, b, x, ldx, y, ldy, m, n, k);
     // Tiles of 64 rows, the same sums, where all of them get a compute unit of their own at once (dense_grid() counts the XCD with the most
     // row tiles for all eight): such a tile takes 0.8 to 0.9 of the time of one of 128 rows, and those would leave half of the units without a
     // block.  2048 x 2048 x 2816 40.6 -> 36.9 us, 1024 x 2816 x 8192 94.6 -> 79.9, 320 x 8192 x 2816 37.1 -> 31.0; but 1200 x 2816 x 2112, three
     // row tiles of 11 on some XCDs, 32.7 -> 39.2.
-    if (dense_grid((uint32_t)(m + kQmmBM / 2 - 1) / (kQmmBM / 2), col_tiles) <= (uint32_t)ctx->num_cus) a.bm = kQmmBM / 2;
-    const dim3 grid(dense_grid((uint32_t)(m + a.bm - 1) / (uint32_t)a.bm, col_tiles));
-    if (a.rows_vectorizable) {
-        if (sd == TF_BF16) hipLaunchKernelGGL((qmm_dense_kernel<0, true>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((qmm_dense_kernel<1, true>), grid, dim3(256), 0, st, a);
-    } else {
-        if (sd == TF_BF16) hipLaunchKernelGGL((qmm_dense_kernel<0, false>), grid, dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((qmm_dense_kernel<1, false>), grid, dim3(256), 0, st, a);
-    }
+    auto launch = [&](auto bm) {
+        constexpr int BM = decltype(bm)::value;
+        const dim3 grid(dense_grid((uint32_t)(m + BM - 1) / BM, col_tiles));
+        if (a.rows_vectorizable) {
+            if (sd == TF_BF16) hipLaunchKernelGGL((qmm_dense_kernel<0, true, BM>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((qmm_dense_kernel<1, true, BM>), grid, dim3(256), 0, st, a);
+        } else {
+            if (sd == TF_BF16) hipLaunchKernelGGL((qmm_dense_kernel<0, false, BM>), grid, dim3(256), 0, st, a);
+            else hipLaunchKernelGGL((qmm_dense_kernel<1, false, BM>), grid, dim3(256), 0, st, a);
+        }
+    };
+    if (dense_grid((uint32_t)(m + kQmmBM / 2 - 1) / (kQmmBM / 2), col_tiles) <= (uint32_t)ctx->num_cus) launch(std::integral_constant<int, kQmmBM / 2>{});
+    else launch(std::integral_constant<int, kQmmBM>{});
     return check_launch(ctx, "int4_qmm");
 }
 
