@@ -612,6 +612,34 @@ def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, sh
     assert not host(partials, np.uint16, n * d).any()
 
 
+@pytest.mark.parametrize("T,E", [(53, 128), (53, 16), (96, 16)])     # the shared expert in launches of its own, few and many pairs an expert; in the routed launches
+def test_refused_shared_expert_leaves_the_routed_stages_unlaunched(T, E):
+    d, f, shared_f, top_k = 128, 64, 192, 8
+    r = resident_pipeline(T, E, d, f, top_k, 0x6A00 + T, from_router=False)
+    k, n = tfk.Context(0), T * top_k             # a context of its own: with the limits it was created with
+    g = device_grouping(r["idx"], r["w_bits"], T, top_k, E)
+    koff = tfk.ExpertOffsets(*r["off"].as_tuple())
+    d_pool, d_hidden = dev(r["pool"]), dev(r["hidden"])
+    mats = [[dev(a) for a in refcases.synthetic_int4(rows, cols, 0x7B, name)] for name, rows, cols in (("g", shared_f, d), ("u", shared_f, d), ("d", d, shared_f))]
+    gate, up, down = (tfk.projection(*m, rows, cols) for m, rows, cols in zip(mats, (shared_f, shared_f, d), (d, d, shared_f)))
+    acts, partials, y, scratch = zeros_bytes(n * f * 2), zeros_bytes(n * d * 2), zeros_bytes(T * d * 2), zeros_bytes(shared_f * 2)
+
+    def call(shared, rows=shared_f, projections=(gate, up, down), last_length=shared_f * 2):
+        return k.lib.tf_prefill_grouped_routed_moe_resident_shared(
+            k.handle, None, d_hidden.data_ptr(), 0, d, g["sorted_pairs"].data_ptr(), g["chunks"].data_ptr(), g["n_chunks"].data_ptr(), g["cap"], n,
+            d_pool.data_ptr(), r["stride"], E, C.byref(koff), acts.data_ptr(), partials.data_ptr(), d, f, top_k, tfk.TF_BF16, d_hidden.data_ptr(), 0, shared, 0,
+            *(C.byref(p) for p in projections), *(v for length in (rows * 2, rows * 2, last_length) for v in (scratch.data_ptr(), 0, length)), T, rows, d, d, 4)
+
+    assert call(y.data_ptr(), last_length=shared_f * 2 - 2) == tfk.TF_ERR_SCRATCH_TOO_SMALL          # the caller's scratch holds less than a row
+    wide = 2048 * 2112 // T // 64 * 64 + 64                                                          # activations beyond the context's reserved buffer
+    big = (tfk.projection(*mats[0], wide, d), tfk.projection(*mats[1], wide, d), tfk.projection(*mats[2], d, wide))
+    assert call(y.data_ptr(), rows=wide, projections=big, last_length=wide * 2) == tfk.TF_ERR_SCRATCH_TOO_SMALL
+    assert not host(partials, np.uint16, n * d).any() and not host(acts, np.uint16, n * f).any() and not host(y, np.uint16, T * d).any()
+    assert call(y.data_ptr()) == tfk.TF_OK
+    assert np.array_equal(host(partials, np.uint16, n * d), r["partials"]) and host(y, np.uint16, T * d).any()
+    k.close()
+
+
 def test_token_major_reduce_matches_cpu_reference():
     # PrefillMoETests.swift:11-44
     rows, top_k, d = 3, 8, 64

@@ -780,7 +780,7 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
                             intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX &&
                             geglu_arrays_near(gate, up);
     const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);
-    if (plan && (!block_path || split)) return TF_OK;
+    if (plan && !block_path) return TF_OK;
     if (weight_bits == 8 && pointers && even && query_count >= 2) {
         // 8-bit projections.  Up to kShared8MfmaMinRows - 1 rows: rows in groups against each weight row, bit-identical to the
         // rows one by one.  From there on the matrix cores: every weight is rounded to fp16 as half(q s + b) first (the
@@ -832,7 +832,7 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
     int32_t rc = shared_block_acts(ctx, (size_t)query_count * intermediate, acts);
     if (rc != TF_OK) return rc;
     if (plan) {
-        *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count};
+        if (!split) *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count};
         return TF_OK;
     }
     rc = split ? launch_geglu_split(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype)
