@@ -751,8 +751,9 @@ int32_t tf_prefill_grouped_routed_moe_resident(tf_ctx *ctx, tf_stream stream,
 /* tf_prefill_grouped_routed_moe_resident and tf_prefill_shared_expert_int4_block of the same token rows as one call
  * (the reference encodes them back to back in one command buffer: the routed stages of PrefillGroupedRoutedMoE.swift:386-461,
  * then PrefillSharedExpert.encodeBlock, PrefillSharedExpert.swift:12-67).  Neither reads what the other writes, so the
- * shared expert's matrix-core tiles are placed ahead of the routed tiles in the same two launches (gate / up / GeGLU, then
- * down) instead of under-filling the chip in launches of their own; results are bit-identical to the two calls.
+ * shared expert's matrix-core tiles (up to 79 rows its split contractions) are placed ahead of the routed tiles in the same two
+ * launches (gate / up / GeGLU, then down) instead of under-filling the chip in launches of their own; results are bit-identical to
+ * the two calls.
  * Applies when the routed pairs go to the matrix-core tile kernels and the shared expert is 4-bit with at least 8 rows and
  * 16-byte aligned operands; otherwise the two calls are made one after the other.  Arguments: those of the routed call, then
  * those of the shared call (its d is the routed d, its scale dtype the routed one; query_count token rows). */

@@ -552,13 +552,21 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
 
 
 @pytest.mark.parametrize("T,E,d,f,shared_f,y_stride,bits", [
-    (64, 16, 2816, 704, 2112, 2816, 4),    # production row widths; routed tiles and shared tiles in the same two launches
+    # up to 79 rows the shared expert's split kernels, their runs shared out over the waves of the routed tiles' blocks
+    (64, 16, 2816, 704, 2112, 2816, 4),    # production row widths; eight runs in both stages
+    (72, 16, 2816, 704, 2112, 2824, 4),    # down in four runs, padded output rows
+    (8, 8, 512, 128, 192, 512, 4),         # runs without a group; down, a short contraction, as a dense tile
+    (40, 16, 192, 64, 1088, 192, 4),       # odd numbers of groups in both stages
+    # dense tiles
+    (96, 16, 2816, 704, 2112, 2816, 4),    # production row widths
+    (97, 16, 2816, 704, 2112, 2816, -4),   # the same bits read as fp16 scales and biases (other numbers, the same equality)
     (200, 16, 256, 192, 128, 264, 4),      # two row tiles of the shared expert, padded output rows
     (1100, 8, 128, 64, 64, 128, 4),        # nine shared row tiles: the shared tiles numbered by XCD
     (96, 8, 512, 128, 192, 515, 4),        # output rows that cannot leave as 16-byte pieces: the two calls one after the other
     (6, 32, 2816, 704, 2112, 2816, 4),     # quad kernels serve the routed pairs: likewise
     (64, 16, 512, 128, 192, 512, 8),       # 8-bit shared expert: likewise
-    (65, 16, 2816, 704, 2112, 2816, -4),   # the first case with the same bits read as fp16 scales and biases (other numbers, the same equality)
+    (65, 16, 2816, 704, 2112, 2816, -4),   # the split kernels (down in four runs) with the same bits read as fp16 scales and biases
+    (33, 16, 2816, 704, 2112, 2816, -4),   # and with down in eight
 ])
 def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, shared_f, y_stride, bits):
     top_k = 8
@@ -610,6 +618,40 @@ def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, sh
         d, y_stride, bits)
     assert rc == tfk.TF_ERR_DIMENSION_MISMATCH
     assert not host(partials, np.uint16, n * d).any()
+
+
+def launches_of(k, call):
+    """Kernels that a call enqueues: the nodes of a graph it is recorded into."""
+    import torch
+    stream = torch.cuda.Stream()
+    graph, nodes = C.c_void_p(), C.c_size_t()
+    assert k.lib.hipStreamBeginCapture(C.c_void_p(stream.cuda_stream), 2) == 0      # hipStreamCaptureModeRelaxed
+    rc = call(stream.cuda_stream)
+    assert k.lib.hipStreamEndCapture(C.c_void_p(stream.cuda_stream), C.byref(graph)) == 0
+    k.check(rc)
+    assert k.lib.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and k.lib.hipGraphDestroy(graph) == 0
+    return nodes.value
+
+
+@pytest.mark.parametrize("T,E,shared_f,launches", [(8, 8, 192, 2), (53, 16, 192, 2), (79, 64, 1088, 2), (96, 16, 192, 2),      # routed tiles: the shared expert rides
+                                                   (53, 128, 192, 4), (7, 8, 192, None)])                                    # quad kernels; a block that is done row by row
+def test_shared_expert_rides_wherever_the_routed_pairs_go_to_the_tiles(T, E, shared_f, launches):
+    d, f, top_k = 128, 64, 8
+    k, n = ctx(), T * top_k
+    pool, hidden = zeros_bytes(E * 65536), zeros_bytes(T * d * 2)
+    off = tfk.ExpertOffsets(*(4096 * i for i in range(9)))
+    pairs, chunks, count, cap = zeros_bytes(n * 16), zeros_bytes((E + n // 64 + 1) * 12), zeros_bytes(4), E + n // 64 + 1      # never run
+    acts, partials, y, scratch, w = zeros_bytes(n * f * 2), zeros_bytes(n * d * 2), zeros_bytes(T * d * 2), zeros_bytes(shared_f * 2), zeros_bytes(d * shared_f)
+    gate, up, down = tfk.projection(w, w, w, shared_f, d), tfk.projection(w, w, w, shared_f, d), tfk.projection(w, w, w, d, shared_f)
+
+    def call(stream):
+        return k.lib.tf_prefill_grouped_routed_moe_resident_shared(
+            k.handle, stream, hidden.data_ptr(), 0, d, pairs.data_ptr(), chunks.data_ptr(), count.data_ptr(), cap, n, pool.data_ptr(), 65536, E, C.byref(off),
+            acts.data_ptr(), partials.data_ptr(), d, f, top_k, tfk.TF_BF16, hidden.data_ptr(), 0, y.data_ptr(), 0, C.byref(gate), C.byref(up), C.byref(down),
+            *(v for _ in range(3) for v in (scratch.data_ptr(), 0, shared_f * 2)), T, shared_f, d, d, 4)
+
+    got = launches_of(k, call)
+    assert got == launches if launches else got > 4
 
 
 @pytest.mark.parametrize("T,E", [(53, 128), (53, 16), (96, 16)])     # the shared expert in launches of its own, few and many pairs an expert; in the routed launches

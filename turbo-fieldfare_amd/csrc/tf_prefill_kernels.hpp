@@ -60,6 +60,7 @@ struct DenseRide {
     half_t *y;            // [rows, down->rows], row stride ldy halves
     long ldy;
     int rows;
+    bool split;           // gate / up as launch_geglu_split computes them, down as qmm_split_variant says; else the dense tiles
 };
 
 // Operands of the grouped expert stages, as the launch helpers pass them on.
@@ -85,7 +86,7 @@ enum { kSplitNone = 0, kSplit32x32, kSplit64x32, kSplit64x64 };
 int qmm_split_variant(int m, int n, int k, long ldx);
 int32_t launch_qmm_split(tf_ctx *ctx, hipStream_t st, int variant, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
                          half_t *y, long ldy, int m, int n, int k, tf_dtype sd);
-// the same for a gate and an up matrix with GeGLU
+// the same for a gate and an up matrix with GeGLU (rows of up to 4096 columns either way, so that the result can also be had inside a grouped launch)
 bool geglu_split_ok(const tf_projection *gate, long ldx);
 int32_t launch_geglu_split(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const half_t *x, long ldx, half_t *a_out,
                            long lda, int m, tf_dtype sd);

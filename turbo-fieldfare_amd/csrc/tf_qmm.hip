@@ -1,6 +1,7 @@
 // Matrix-core (MFMA) kernels: dense int4 QMM, and the grouped expert GEMMs of batched prefill
 // (gate/up + GeGLU, then down) driven by a work list of (expert, pair range) chunks.
 #include "tf_prefill_kernels.hpp"
+#include "tf_qmm_split.hpp"
 #include "tf_rowdot.hpp"
 
 using namespace tfk;
@@ -351,6 +352,22 @@ __global__ __launch_bounds__(64 * kGroupedWaves, 8 / kGroupedWaves) void grouped
     else grouped_phase1_body<SD>(a, blockIdx.x - dense_blocks, lds);
 }
 
+// The same launch with the gate / up / GeGLU tiles of a small block's shared expert: the split kernel's tiles and its eight runs, two to each of
+// the four waves, in the half of a compute unit's LDS that a block of this launch has.
+constexpr size_t kRideLds = 81920;
+template <int NW, int COLS, int SPLIT_LDS>
+constexpr int ride_lds_bytes() {
+    constexpr int tiles = block_lds_bytes<NW, COLS>();
+    static_assert(SPLIT_LDS <= (int)kRideLds && tiles <= (int)kRideLds, "two blocks on a compute unit");
+    return tiles > SPLIT_LDS ? tiles : SPLIT_LDS;
+}
+template <int SD>
+__global__ __launch_bounds__(64 * kGroupedWaves, 8 / kGroupedWaves) void grouped_phase1_and_split_geglu_kernel(GroupedP1Args a, uint32_t split_blocks, SplitArgs split) {
+    __shared__ __align__(128) uint8_t lds[ride_lds_bytes<kGroupedWaves, kP1BN, SplitGeom<4, 1, 2, kGroupedWaves, 4, 8>::kLds>()];
+    if (blockIdx.x < split_blocks) qmm_split_body<4, SD, 1, 2, kGroupedWaves, 4, true, 8>(split, blockIdx.x, lds);
+    else grouped_phase1_body<SD>(a, blockIdx.x - split_blocks, lds);
+}
+
 // ------------------------------------------------------------------------------------------------ grouped down
 // Block = one chunk x 64 NW output columns: X rows are the chunk's activation rows, Y rows scatter to
 // route_partials[(token * top_k + rank) * D + c].
@@ -435,6 +452,16 @@ __global__ __launch_bounds__(64 * kGroupedWaves, 8 / kGroupedWaves) void grouped
     else grouped_down_body<SD>(a, blockIdx.x - dense_blocks, lds);
 }
 
+// the same launch with a small block's down product as the split kernels compute it: eight runs of up to four pairs of groups, or four of up to
+// eight (the sums of the 64 x 32 tiles; here 32 x 32, a row's sums are the same)
+template <int SD, int RUNS>
+__global__ __launch_bounds__(64 * kGroupedWaves, 8 / kGroupedWaves) void grouped_down_and_split_kernel(GroupedDownArgs a, uint32_t split_blocks, SplitArgs split) {
+    constexpr int GP = 32 / RUNS;
+    __shared__ __align__(128) uint8_t lds[ride_lds_bytes<kGroupedWaves, kDownBN, SplitGeom<4, 1, 1, kGroupedWaves, GP, RUNS>::kLds>()];
+    if (blockIdx.x < split_blocks) qmm_split_body<4, SD, 1, 1, kGroupedWaves, GP, false, RUNS>(split, blockIdx.x, lds);
+    else grouped_down_body<SD>(a, blockIdx.x - split_blocks, lds);
+}
+
 DenseArgs dense_args(const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx, half_t *y, long ldy, int m, int n, int k) {
     const bool rows_vec = aligned16(y) && n % 8 == 0 && ldy % 8 == 0;   // whole 16-byte pieces of output rows
     return DenseArgs{w, s, b, x, ldx, y, ldy, m, n, k, rows_vec};
@@ -476,6 +503,13 @@ int32_t launch_grouped_phase1_mfma(tf_ctx *ctx, hipStream_t st, const ExpertTabl
                                    tf_dtype sd, const DenseRide *ride) {
     const uint32_t grouped = (uint32_t)((f + kP1BN - 1) / kP1BN) * ((n_chunks_upper + kChunkRun - 1) / kChunkRun * kChunkRun);
     const GroupedP1Args a = {tab, off, cl, pairs, hidden, hidden_stride, acts, acts_pair_base, d, f};
+    if (ride && ride->split) {
+        const SplitArgs split = geglu_split_args(ride->gate, ride->up, ride->x, ride->ldx, ride->acts, (long)ride->gate->rows, ride->rows);
+        const uint32_t blocks = (uint32_t)((ride->rows + 31) / 32) * (uint32_t)((split.N + 31) / 32), extra = (blocks + kXcds - 1) / kXcds * kXcds;
+        if (sd == TF_BF16) hipLaunchKernelGGL(grouped_phase1_and_split_geglu_kernel<0>, dim3(grouped + extra), dim3(64 * kGroupedWaves), 0, st, a, extra, split);
+        else hipLaunchKernelGGL(grouped_phase1_and_split_geglu_kernel<1>, dim3(grouped + extra), dim3(64 * kGroupedWaves), 0, st, a, extra, split);
+        return check_launch(ctx, "grouped_phase1_mfma + shared gate/up");
+    }
     if (ride) {
         // the shared expert's gate / up / GeGLU tiles ahead of the grouped tiles (the full-height, longest tiles first), padded
         // to a multiple of 8 blocks so that both kinds keep their XCDs
@@ -497,6 +531,16 @@ int32_t launch_grouped_down_mfma(tf_ctx *ctx, hipStream_t st, const ExpertTable 
     const GroupedDownArgs a = {tab, off, cl, pairs, acts, acts_pair_base, route_partials, d, f, top_k};
     if (ride) {
         const tf_projection *dn = ride->down;   // ride->y: 16-byte aligned rows of whole 16-byte pieces (dense_ride_ok)
+        const int variant = ride->split ? qmm_split_variant(ride->rows, (int)dn->rows, (int)dn->cols, (long)dn->cols) : kSplitNone;
+        if (variant != kSplitNone) {      // the kernel that the product has in a launch of its own
+            const SplitArgs split = qmm_split_args(at(dn->weights, dn->weights_offset), at(dn->scales, dn->scales_offset), at(dn->biases, dn->biases_offset),
+                                                   ride->acts, (long)dn->cols, ride->y, ride->ldy, ride->rows, (int)dn->rows, (int)dn->cols);
+            const uint32_t blocks = (uint32_t)((ride->rows + 31) / 32) * (uint32_t)((split.N + 31) / 32), extra = (blocks + kXcds - 1) / kXcds * kXcds;
+            auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(grouped + extra), dim3(64 * kGroupedWaves), 0, st, a, extra, split); };
+            if (variant == kSplit32x32) sd == TF_BF16 ? launch(grouped_down_and_split_kernel<0, 8>) : launch(grouped_down_and_split_kernel<1, 8>);
+            else sd == TF_BF16 ? launch(grouped_down_and_split_kernel<0, 4>) : launch(grouped_down_and_split_kernel<1, 4>);
+            return check_launch(ctx, "grouped_down_mfma + shared down");
+        }
         const DenseArgs dense = dense_args(at(dn->weights, dn->weights_offset), at(dn->scales, dn->scales_offset), at(dn->biases, dn->biases_offset),
                                            ride->acts, (long)dn->cols, ride->y, ride->ldy, ride->rows, (int)dn->rows, (int)dn->cols);
         const uint32_t extra = (dense_grid((uint32_t)(ride->rows + kQmmBM - 1) / kQmmBM, (uint32_t)((int)dn->rows + kQmmBN - 1) / kQmmBN) + kXcds - 1) / kXcds * kXcds;
@@ -568,8 +612,11 @@ int32_t shared_block_acts(tf_ctx *ctx, size_t halves, half_t *&out) {
 }
 
 constexpr uint32_t kSharedBlockMinRows = 8;   // fewer rows go through the single-row chain, bit-identical to decode
-// Up to here the shared expert's gate / up and down go to the split kernels (53 rows of 2112 x 2816: 11 + 8 us against 27 + 22 us in
-// launches of their own); from five pairs an expert on (80 tokens of top 8 among 128) its tiles ride in the grouped launches.
+// Up to here the shared expert's gate / up and down are computed as the split kernels do: in launches of their own beside the quad kernels (53
+// rows of 2112 x 2816: 20 us for both against 50 on the dense tiles), or riding in the routed tiles' launches (the one call, 53 rows, 16 experts
+// of 704 x 2816: 47 us against 56 with dense tiles riding; 32 experts 57 against 58, 64 experts 71 against 75).  The rule asks for the rows
+// alone, never for the experts: the shared expert by itself and the one call give the same bits.  From 80 rows on, where top 8 of 128
+// experts leave the quad kernels, the dense tiles ride; the split kernels have not been measured against them there.
 constexpr uint32_t kSharedSplitMaxRows = 79;
 
 // ---- 8-bit projections over a block of rows ----------------------------------------------------------------------
@@ -779,7 +826,7 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
                             qmm_operands_ok(gw, xp, x_stride_elements, (int)d) && aligned16(uw) && aligned16(dw) &&
                             intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX &&
                             geglu_arrays_near(gate, up);
-    const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);
+    const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);      // one choice for the call alone and for a ride
     if (plan && !block_path) return TF_OK;
     if (weight_bits == 8 && pointers && even && query_count >= 2) {
         // 8-bit projections.  Up to kShared8MfmaMinRows - 1 rows: rows in groups against each weight row, bit-identical to the
@@ -832,13 +879,13 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
     int32_t rc = shared_block_acts(ctx, (size_t)query_count * intermediate, acts);
     if (rc != TF_OK) return rc;
     if (plan) {
-        if (!split) *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count};
+        *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count, split};
         return TF_OK;
     }
     rc = split ? launch_geglu_split(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype)
                : launch_qmm_dense_geglu(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype);
     if (rc != TF_OK) return rc;
-    // a block that may ride in the grouped launches takes the tiles here too: the same bits either way
+    // more rows: gate / up took the dense tiles, and so does down, as in a ride
     return launch_qmm_dense(ctx, st, dw, at(down->scales, down->scales_offset), at(down->biases, down->biases_offset), acts, (long)intermediate,
                             yp, (long)y_stride_elements, (int)query_count, (int)d, (int)intermediate, scale_dtype, !split);
 }
