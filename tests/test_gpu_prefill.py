@@ -407,7 +407,7 @@ def run_quad_work_list(r, chunks, T, E, d, f, top_k):
 
 @pytest.mark.parametrize("T,E,run", [(75, 128, 1), (40, 128, 3), (31, 128, 128), (20, 40, 9)])
 def test_quad_kernels_share_out_any_work_list(T, E, run):
-    # The blocks share out batches of up to eight pairs (more than 512 chunks: whole chunks).  A pair's sums do not depend on whom it
+    # The blocks share out batches of up to eight pairs (more than 320 chunks: whole chunks).  A pair's sums do not depend on whom it
     # shares a batch with, so however the runs are cut the outputs are those of the device grouping's list.
     d, f, top_k = 128, 64, 8
     r = resident_pipeline(T, E, d, f, top_k, 0x4A00 + T + run, zipf=True, from_router=False)
@@ -425,16 +425,16 @@ def test_quad_kernels_share_out_any_work_list(T, E, run):
     assert np.array_equal(run_quad_work_list(r, chunks, T, E, d, f, top_k), r["partials"])
 
 
-@pytest.mark.parametrize("T,E,run,singles,blocks_per_cu", [(375, 640, 9, 200, 3), (1400, 2300, 24, 0, 5)])
+@pytest.mark.parametrize("T,E,run,singles,blocks_per_cu", [(750, 1250, 20, 20, 3), (1350, 2200, 36, 0, 5)])
 def test_quad_kernels_given_more_batches_than_blocks(T, E, run, singles, blocks_per_cu):
-    # At most 512 chunks whose batches of eight pairs outnumber the blocks of the launch (three a compute unit for gate / up, five for
+    # At most 320 chunks whose batches of eight pairs outnumber the blocks of the launch (three a compute unit for gate / up, five for
     # down): a block's share is cut in whole chunks, whose batches it takes one after the other.
     import torch
     d, f, top_k = 128, 64, 8
     n = T * top_k
     counts = [run] * ((n - singles) // run) + [1] * singles
     counts += [n - sum(counts)] if sum(counts) < n else []
-    assert len(counts) <= 512 and n < 5 * E
+    assert len(counts) <= 320 and n < 5 * E
     assert sum((c + 7) // 8 for c in counts) > blocks_per_cu * torch.cuda.get_device_properties(0).multi_processor_count
     base = resident_pipeline(16, 128, d, f, top_k, 0x4B00 + T, from_router=False)
     pairs = np.zeros(n, tfo.PAIR_DTYPE)
@@ -446,8 +446,8 @@ def test_quad_kernels_given_more_batches_than_blocks(T, E, run, singles, blocks_
              hidden=hidden, sorted_pairs=pairs)
     starts = np.cumsum(counts) - counts
     whole = [(e, int(at), int(c)) for e, (at, c) in enumerate(zip(starts, counts))]
-    cut = [(e, p, min(4, at + c - p)) for e, at, c in whole for p in range(at, at + c, 4)]      # more than 512 chunks: no batches are counted
-    assert len(cut) > 512
+    cut = [(e, p, min(4, at + c - p)) for e, at, c in whole for p in range(at, at + c, 4)]      # more than 320 chunks: no batches are counted
+    assert len(cut) > 320
     got = run_quad_work_list(r, whole, T, E, d, f, top_k)
     assert np.array_equal(got, run_quad_work_list(r, cut, T, E, d, f, top_k))
     want = tfo.from_f16_bits(tfo.prefill_route_partials(pairs, T, hidden.ravel(), d, r["pool"], r["stride"], r["off"], top_k, d, f, fill_bits=0, threads=8))

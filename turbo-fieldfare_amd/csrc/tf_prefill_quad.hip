@@ -73,11 +73,6 @@ struct QuadMap {
     __device__ __forceinline__ uint32_t sboff(int p) const { return p < NPASS - 1 ? sboff0 + (uint32_t)(QC * p / 2) * 2u : sboff_last; }
 };
 
-// chunks of the call, as every thread of a launch sees it
-__device__ __forceinline__ uint32_t quad_chunk_count(const ChunkList &cl, uint32_t n_chunks_upper) {
-    return uniform_u32(min(cl.dev ? *cl.dev_n : cl.n, n_chunks_upper));
-}
-
 // The work of a call is cut into units: a unit is one batch of a chunk, up to max_pairs of its pairs (what the LDS image holds)
 // against all of its expert's tiles.  A popular expert's chunk is many units: given the same number of blocks as every other chunk, as
 // it once was, its blocks went over the expert's weights once per batch one after the other and set the launch's time (16 tokens: gate / up
@@ -93,40 +88,46 @@ struct QuadSpan {
     tf_prefill_group run[2];          // the pairs of unit0 and of the unit after it
     bool units;                       // false: too many chunks or units for this scheme, a "unit" is a whole chunk (batches in the block's own loop)
 };
-// scratch: 64 bytes of LDS that nothing else uses until the block's next barrier, and free again when this returns; 256 threads, all call
-__device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_chunks, uint32_t max_pairs, uint32_t tiles_per_unit, uint32_t *scratch) {
+// lane l: the sum of v over lanes 0 .. l
+__device__ __forceinline__ uint32_t wave_running_sum(uint32_t v) {
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false);      // one, two, four, eight lanes down inside each row of 16
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false);
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false);      // the last lane of rows 0 and 2 into the row after
+    v += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false);      // lane 31 into the upper half
+    return v;
+}
+
+// Every wave works its block's share out by itself, up to five times 64 chunks (the device grouping of up to 256 experts with fewer than five
+// pairs each makes at most 276), so that nothing passes through LDS and no barrier stands before the first weight row.  The list has
+// room for n_chunks_upper chunks: they are asked for beside their number, not after it.  Both launches for 6 tokens x 8 of 128 experts, d 512,
+// f 128: 11.3 us with equal shares by chunk, 13.5 with a scan over the block's threads through LDS
+// behind two trips to memory, 12.6 so; at d 2816, f 704 33.6, 35.0 and 33.7, and 39.4, 30.6 and 29.4 where a few experts are popular.
+__device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_chunks_upper, uint32_t max_pairs, uint32_t tiles_per_unit) {
+    constexpr uint32_t K = 5;
     QuadSpan sp;
-    uint32_t units = n_chunks;
-    sp.units = n_chunks <= 512u;
-    tf_prefill_group mine[2] = {{0u, 0u, 0u}, {0u, 0u, 0u}};      // thread t: chunks 2 t and 2 t + 1
-    uint32_t batches[2] = {0u, 0u}, first = 0u;
-    if (sp.units) {
+    const uint32_t lane = threadIdx.x & 63u;
+    tf_prefill_group mine[K];                  // chunk 64 i + lane
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            if (2u * threadIdx.x + i < n_chunks && get_chunk(cl, 2u * threadIdx.x + i, mine[i])) batches[i] = (mine[i].pair_count + max_pairs - 1) / max_pairs;
-        uint32_t sum = batches[0] + batches[1];                       // inclusive scan over the wave, then over the four waves
+    for (uint32_t i = 0; i < K; ++i) {
+        mine[i] = {0u, 0u, 0u};
+        if (kWave * i < n_chunks_upper) mine[i] = cl.dev[min(kWave * i + lane, n_chunks_upper - 1u)];
+    }
+    const uint32_t n_chunks = uniform_u32(min(*cl.dev_n, n_chunks_upper));
+    uint32_t batches[K], first[K], units = 0u;
 #pragma unroll
-        for (int step = 1; step < 64; step <<= 1) {
-            const uint32_t below = (uint32_t)__shfl_up((int)sum, step, kWave);
-            if ((int)(threadIdx.x & 63) >= step) sum += below;
-        }
-        if ((threadIdx.x & 63) == 63) scratch[threadIdx.x >> 6] = sum;
-        __syncthreads();
-        uint32_t before = 0u, total = 0u;
-#pragma unroll
-        for (uint32_t w = 0; w < 4; ++w) {
-            const uint32_t t = scratch[w];
-            before += w < (threadIdx.x >> 6) ? t : 0u;
-            total += t;
-        }
-        first = before + sum - batches[0] - batches[1];
-        units = uniform_u32(total);
-        sp.units = units <= gridDim.x;
-        if (!sp.units) {
-            units = n_chunks;
-            __syncthreads();          // every wave has read the sums: the caller may write over them (the other way out ends with a barrier too)
+    for (uint32_t i = 0; i < K; ++i) {
+        batches[i] = first[i] = 0u;
+        if (kWave * i < n_chunks) {
+            batches[i] = kWave * i + lane < n_chunks ? (mine[i].pair_count + max_pairs - 1) / max_pairs : 0u;
+            const uint32_t through = wave_running_sum(batches[i]);
+            first[i] = units + through - batches[i];
+            units += (uint32_t)__builtin_amdgcn_readlane((int)through, 63);
         }
     }
+    sp.units = n_chunks <= K * kWave && units <= gridDim.x;
+    if (!sp.units) units = n_chunks;
     const uint32_t per_unit = units ? gridDim.x / units : 0u;
     if (per_unit >= kQuadMinBlocksPerUnit) {
         const uint32_t unit = blockIdx.x / per_unit, part = blockIdx.x - unit * per_unit;
@@ -140,25 +141,24 @@ __device__ __forceinline__ QuadSpan quad_span(const ChunkList &cl, uint32_t n_ch
     }
     sp.unit0 = sp.lo / tiles_per_unit;
     if (sp.units) {
-        // the owners of the two units' chunks tell the block
+        // the lane whose chunk a unit belongs to tells the wave
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
+        for (uint32_t u = 0; u < 2; ++u) {
+            tf_prefill_group run = {0u, 0u, 0u};
+            bool own = false;
 #pragma unroll
-            for (uint32_t u = 0; u < 2; ++u) {
-                const uint32_t batch = sp.unit0 + u - first;          // wraps far beyond `batches` for a unit of an earlier chunk
+            for (uint32_t i = 0; i < K; ++i) {
+                const uint32_t batch = sp.unit0 + u - first[i];          // wraps far beyond `batches` for a unit of an earlier chunk
                 if (batch < batches[i]) {
-                    scratch[4 + 3 * u] = mine[i].expert;
-                    scratch[5 + 3 * u] = mine[i].pair_start + batch * max_pairs;
-                    scratch[6 + 3 * u] = min(max_pairs, mine[i].pair_count - batch * max_pairs);
+                    own = true;
+                    run = {mine[i].expert, mine[i].pair_start + batch * max_pairs, min(max_pairs, mine[i].pair_count - batch * max_pairs)};
                 }
             }
-            first += batches[i];
+            const uint64_t owners = __ballot(own);
+            const int owner = owners != 0ull ? (int)__builtin_ctzll(owners) : 0;       // none: past the last unit, and not asked for
+            sp.run[u] = {(uint32_t)__builtin_amdgcn_readlane((int)run.expert, owner), (uint32_t)__builtin_amdgcn_readlane((int)run.pair_start, owner),
+                         (uint32_t)__builtin_amdgcn_readlane((int)run.pair_count, owner)};
         }
-        __syncthreads();
-#pragma unroll
-        for (uint32_t u = 0; u < 2; ++u)
-            sp.run[u] = tf_prefill_group{uniform_u32(scratch[4 + 3 * u]), uniform_u32(scratch[5 + 3 * u]), uniform_u32(scratch[6 + 3 * u])};
-        __syncthreads();
     }
     return sp;
 }
@@ -328,7 +328,7 @@ __global__ __launch_bounds__(256, 3) void grouped_phase1_quad_kernel(ExpertTable
     QuadPass t[NPASS];
     // the block's share of the tiles of all units
     const uint32_t tpe = (uint32_t)f / Map::kRows;
-    const QuadSpan span = quad_span(cl, quad_chunk_count(cl, n_chunks_upper), (uint32_t)MAXP, tpe, reinterpret_cast<uint32_t *>(quad_lds));
+    const QuadSpan span = quad_span(cl, n_chunks_upper, (uint32_t)MAXP, tpe);
     for (uint32_t pos = span.lo; pos < span.hi;) {
     const uint32_t unit = pos / tpe;
     const int t_lo = (int)(pos - unit * tpe), t_hi = (int)min(tpe, (uint32_t)t_lo + (span.hi - pos));
@@ -428,7 +428,7 @@ __global__ __launch_bounds__(256, 5) void grouped_down_quad_kernel(ExpertTable t
     tsb.init(lane, (uint32_t)Map::kRows * ((uint32_t)f >> 6) * 2u);
     // the block's share of the tiles of all units (see the gate / up kernel)
     const uint32_t tiles = (uint32_t)d / Map::kRows;
-    const QuadSpan span = quad_span(cl, quad_chunk_count(cl, n_chunks_upper), kQuadMaxPairs, tiles, reinterpret_cast<uint32_t *>(quad_lds));
+    const QuadSpan span = quad_span(cl, n_chunks_upper, kQuadMaxPairs, tiles);
     for (uint32_t pos = span.lo; pos < span.hi;) {
     const uint32_t unit = pos / tiles;
     const int t_lo = (int)(pos - unit * tiles), t_hi = (int)min(tiles, (uint32_t)t_lo + (span.hi - pos));
