@@ -200,3 +200,24 @@ def test_graph_of_a_short_context_survives_a_longer_eager_call():
     torch.cuda.synchronize()
     assert np.array_equal(host(out, np.uint16), first)
     k.close()
+
+
+def test_block_attention_does_not_depend_on_how_much_is_reserved():
+    # 376 queries of 16 heads over 32000 keys of head_dim 512: the same chunks, so the same bits, in a context that is reserved for the call
+    # and in one that is reserved for sixteen times as many tokens
+    import ctypes as C
+    import torch
+    T, rows, nq, nkv, hd = 376, 32000, 16, 2, 512
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(0x7A3)
+    q, kc, vc = (torch.randn(n, generator=gen, device="cuda").to(torch.float16) for n in (T * nq * hd, rows * nkv * hd, rows * nkv * hd))
+    params = tfk.PrefillAttentionParams(rows - T, T, hd, nq, nkv, rows, 0, nkv * hd, nq * hd, nq * hd, hd ** -0.5)
+    outs = []
+    for reserved in (T, 16 * T):
+        k = tfk.Context(0)
+        k.reserve(max_attention_block_tokens=reserved)
+        out = zeros_bytes(T * nq * hd * 2)
+        k.check(k.lib.tf_prefill_attention_causal(k.handle, None, q.data_ptr(), 0, kc.data_ptr(), 0, vc.data_ptr(), 0, out.data_ptr(), 0, C.byref(params), 0))
+        outs.append(host(out, np.uint16))
+        k.close()
+    assert np.array_equal(*outs)

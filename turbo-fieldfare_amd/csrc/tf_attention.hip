@@ -624,6 +624,7 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
 // wave owns 64 of the 512 output elements of ALL 128 columns, so a V tile is read and permuted once a block instead of once a wave, and
 // twice the columns share each tile's trip into LDS.
 constexpr int kWideWaves = 8, kWideCols = kWideWaves * kTileHeads;
+constexpr uint32_t kWideGoes = 2;            // chunks only as far as the blocks fill the compute units this often
 __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_kernel(const half_t *Q, const half_t *K, const half_t *V, half_t *O, float *m_part,
                                                                                     float *d_part, float *o_part, PrefillShape s, uint32_t group_shift,
                                                                                     uint32_t col_blocks, uint32_t num_chunks) {
@@ -1005,16 +1006,19 @@ namespace tfk {
 
 // Upper bound of the partial states (m, d and head_dim values of o each) any call within the limits asks for.
 // Decode: q_heads x chunks with at most kMaxDeviceChunks chunks.  Block attention: n = queries x q_heads columns make at
-// least ceil(n / 64) blocks per chunk, and chunks stop at two blocks per compute unit or kMaxPrefillChunks.
+// least ceil(n / 64) blocks per chunk, and chunks stop at two blocks per compute unit or kMaxPrefillChunks; the wide kernel's n columns make
+// at least ceil(n / 128), and its chunks stop where they fill the compute units kWideGoes times.
 size_t attention_scratch_floats_for(int num_cus, uint32_t q_heads, uint32_t head_dim, uint32_t block_tokens) {
     size_t states = (size_t)q_heads * kMaxDeviceChunks;
-    const size_t target = (size_t)(num_cus > 0 ? num_cus : 256) * 2;
+    const size_t cus = (size_t)(num_cus > 0 ? num_cus : 256), target = cus * 2;
     const size_t max_n = (size_t)block_tokens * q_heads;
     for (size_t n = 1; n <= max_n; ++n) {
         const size_t base = (n + kPrefillCols - 1) / kPrefillCols;
         const size_t chunks = std::min<size_t>(kMaxPrefillChunks, (target + base - 1) / base);
         states = std::max(states, n * chunks);
     }
+    if (head_dim >= 512)
+        for (size_t c = 1; c <= kMaxPrefillChunks; ++c) states = std::max(states, c * std::min(max_n, kWideGoes * cus / c * (size_t)kWideCols));
     return states * (2 + (size_t)head_dim);
 }
 
@@ -1116,12 +1120,14 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
             const uint32_t wide_blocks = (s.count * group + kWideCols - 1) / kWideCols, wide_base = wide_blocks * s.num_kv_heads, cus = (uint32_t)ctx->num_cus;
             // in keys: the longest compute unit's blocks, one at a time (20 blocks a chunk: 12 chunks in one go, not 13 in two), and the
             // merge, where a chunk's partial states of 195 columns cost as much as a key of a block (4 KB a column written and read
-            // back at 8 TB/s).  Chunks only as far as the scratch reaches (a reserved context's always does).
+            // back at 8 TB/s).  How many chunks depends on the shape and the device alone where the context is reserved for the call; one that
+            // takes it beyond its limits may hold the states of fewer.
             auto price = [&](uint32_t blocks, uint32_t c, float key) {
                 return (float)((blocks * c + cus - 1) / cus) * (float)span / (float)c * key + (c > 1 ? (float)s.count * (float)s.num_q_heads * (float)c / 195.0f : 0.0f);
             };
             uint32_t best = 1;
-            for (uint32_t c = 2; c <= std::min(span / kMinChunkKeys, kMaxPrefillChunks) && states_of(c) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes; ++c)
+            const uint32_t most = std::min({span / kMinChunkKeys, kMaxPrefillChunks, kWideGoes * cus / wide_base});
+            for (uint32_t c = 2; c <= most && states_of(c) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes; ++c)
                 if (price(wide_base, c, 1.0f) < price(wide_base, best, 1.0f)) best = c;
             wide = price(wide_base, best, 1.0f) < price(base, chunks, 0.92f);
             if (wide) {
