@@ -56,3 +56,17 @@ def device_view(ptr: int, count: int, typestr: str):
     import torch
     torch.cuda.synchronize()
     return torch.as_tensor(_RawDeviceArray(ptr, count, typestr), device="cuda").cpu().numpy().copy()
+
+
+def launches_of(k, call):
+    """Kernels that a call enqueues: the nodes of a graph it is recorded into."""
+    import ctypes as C
+    import torch
+    stream = torch.cuda.Stream()
+    graph, nodes = C.c_void_p(), C.c_size_t()
+    assert k.lib.hipStreamBeginCapture(C.c_void_p(stream.cuda_stream), 2) == 0      # hipStreamCaptureModeRelaxed
+    rc = call(stream.cuda_stream)
+    assert k.lib.hipStreamEndCapture(C.c_void_p(stream.cuda_stream), C.byref(graph)) == 0
+    k.check(rc)
+    assert k.lib.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and k.lib.hipGraphDestroy(graph) == 0
+    return nodes.value

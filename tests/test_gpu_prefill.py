@@ -8,7 +8,7 @@ import pytest
 import torch
 
 import refcases
-from gpu_helpers import device_view, ctx, dev, host, tfk, within_north_star, zeros_bytes
+from gpu_helpers import ctx, dev, device_view, host, launches_of, tfk, within_north_star, zeros_bytes
 from oracle import tfo
 
 pytestmark = pytest.mark.gpu
@@ -618,19 +618,6 @@ def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, sh
         d, y_stride, bits)
     assert rc == tfk.TF_ERR_DIMENSION_MISMATCH
     assert not host(partials, np.uint16, n * d).any()
-
-
-def launches_of(k, call):
-    """Kernels that a call enqueues: the nodes of a graph it is recorded into."""
-    import torch
-    stream = torch.cuda.Stream()
-    graph, nodes = C.c_void_p(), C.c_size_t()
-    assert k.lib.hipStreamBeginCapture(C.c_void_p(stream.cuda_stream), 2) == 0      # hipStreamCaptureModeRelaxed
-    rc = call(stream.cuda_stream)
-    assert k.lib.hipStreamEndCapture(C.c_void_p(stream.cuda_stream), C.byref(graph)) == 0
-    k.check(rc)
-    assert k.lib.hipGraphGetNodes(graph, None, C.byref(nodes)) == 0 and k.lib.hipGraphDestroy(graph) == 0
-    return nodes.value
 
 
 @pytest.mark.parametrize("T,E,shared_f,launches", [(8, 8, 192, 2), (53, 16, 192, 2), (79, 64, 1088, 2), (96, 16, 192, 2),      # routed tiles: the shared expert rides

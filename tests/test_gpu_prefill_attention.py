@@ -4,7 +4,7 @@ the contract (PrefillAttentionTests.swift)."""
 import numpy as np
 import pytest
 
-from gpu_helpers import ctx, dev, host, tfk
+from gpu_helpers import ctx, dev, host, launches_of, tfk
 from oracle import tfo
 from test_oracle_prefill_attention import CASES, kernel_order, make_fixture, reference
 
@@ -176,3 +176,20 @@ def test_wide_columns_of_head_dim_512(start, count, window, hq, hkv, ring, scale
         scores = (q[:, h].double() @ k[:, g].double().T.contiguous()) * scale
         want = torch.softmax(scores.masked_fill(hidden, float("-inf")), 1) @ v[:, g].double()
         assert torch.all((out[:, h].double() - want).abs() <= 2e-3 * want.abs().clamp(min=1.0)), h
+
+
+@pytest.mark.parametrize("start,count,hd,hq,hkv,launches", [
+    (0, 256, 256, 16, 8, 1), (0, 384, 256, 16, 8, 1), (0, 376, 128, 16, 2, 1), (60, 200, 64, 16, 8, 1), (0, 300, 512, 16, 2, 1),      # a prompt's first block: one walk, no merge
+    (1023, 53, 256, 16, 8, 2), (400, 64, 128, 16, 2, 2), (300, 33, 512, 16, 2, 2), (300, 128, 256, 16, 8, 2),                       # few queries over more keys: shorter walks and a merge
+])
+def test_keys_are_cut_into_chunks_where_the_merge_is_worth_it(start, count, hd, hq, hkv, launches):
+    import ctypes as C
+    import torch
+    rows = start + count
+    q, k, v, out = (torch.zeros(n, heads * hd, dtype=torch.float16, device="cuda") for n, heads in ((count, hq), (rows, hkv), (rows, hkv), (count, hq)))
+    kk = tfk.Context(0)
+    kk.reserve(max_attention_block_tokens=count)
+    p = tfk.PrefillAttentionParams(start, count, hd, hq, hkv, rows, 0, hkv * hd, hq * hd, hq * hd, hd ** -0.5)
+    assert launches_of(kk, lambda stream: kk.lib.tf_prefill_attention_causal(kk.handle, stream, q.data_ptr(), 0, k.data_ptr(), 0, v.data_ptr(), 0, out.data_ptr(),
+                                                                             0, C.byref(p), 0)) == launches
+    kk.close()

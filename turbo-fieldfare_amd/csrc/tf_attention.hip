@@ -853,6 +853,19 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
     }
 }
 
+// What a block attention call takes, in microseconds, fitted to 16 / 8, 16 / 2, 16 / 1, 8 / 8, 8 / 1 and 4 / 4 heads, 1 to 2048 queries over 256
+// to 18000 keys (7 % off on average): start-up, 32 keys of the longest walk, the merge's launch, and a thousand partial states written and merged.
+struct AttnCost {
+    float start, tile, merge, thousand_states;
+};
+constexpr AttnCost kAttnCost[4] = {{0.0f, 0.55f, 2.4f, 0.36f}, {0.0f, 0.77f, 3.1f, 0.48f}, {0.0f, 1.13f, 3.1f, 0.68f}, {8.3f, 2.0f, 5.4f, 0.85f}};   // head_dim 64, 128, 256, 512
+constexpr AttnCost kWideCost = {9.0f, 2.5f, 8.0f, 0.67f};
+// blocks a chunk, in as many goes as `slots` blocks at once make of them
+inline float attn_us(const AttnCost &c, uint32_t blocks, uint32_t chunks, uint32_t span, size_t states, uint32_t slots) {
+    const uint32_t goes = (blocks * chunks + slots - 1) / slots, tiles = ((span + chunks - 1) / chunks + kPrefillKeys - 1) / kPrefillKeys;
+    return c.start + c.tile * (float)(goes * tiles) + (chunks > 1 ? c.merge + c.thousand_states * 1e-3f * (float)states : 0.0f);
+}
+
 // merge of the chunks' partial states of one (query, head) column: out = sum_c w_c o_c / sum_c w_c d_c, w_c = exp(m_c - max m);
 // chunks are added in ascending order; a chunk that saw no key has weight zero and its o is not read
 __global__ __launch_bounds__(128) void attention_prefill_combine_kernel(const float *m_part, const float *d_part, const float *o_part, half_t *O,
@@ -1100,36 +1113,34 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
         const uint32_t target = (uint32_t)ctx->num_cus * (hd > 256 ? 1u : 2u);
         uint32_t chunks = std::max(1u, std::min({(target + base - 1) / base, span / kMinChunkKeys, kMaxPrefillChunks}));
         auto states_of = [&](uint32_t c) { return (size_t)s.count * s.num_q_heads * c; };
-        // blocks for less than three eighths of the compute units: shorter chunks (33 queries over 1033 keys of a sliding window 22.4 -> 19.2 us,
-        // 53 over 1076 23.1 -> 20.4; with more blocks the merge takes what the shorter walk gives, 200 over 1200 29.7 -> 32.9)
+        // blocks for less than three eighths of the compute units: shorter chunks, where the shorter walk is worth the merge (16 / 8 heads of 256: 53
+        // queries over 1076 keys 23.1 -> 20.4 us, 128 over 428 22.4 -> 19.4; but a prompt's first 256 positions 14.8 -> 18.1, 384 19.9 -> 28.1)
+        const AttnCost &cost = kAttnCost[hd == 64 ? 0 : hd == 128 ? 1 : hd == 256 ? 2 : 3];
         if (base * chunks * 8u <= (uint32_t)ctx->num_cus * 3u) {
             const uint32_t more = std::min({(target + base - 1) / base, span / kShortChunkKeys, kMaxPrefillChunks});
-            if (more > chunks && states_of(more) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes) chunks = more;
+            if (more > chunks && attn_us(cost, base, more, span, states_of(more), target) < attn_us(cost, base, chunks, span, states_of(chunks), target) &&
+                states_of(more) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes)
+                chunks = more;
         }
         float *m = nullptr, *d = nullptr, *o = nullptr, *scratch = nullptr;
         if (chunks > 1) {
             const int32_t rc = attention_scratch(ctx, states_of(chunks) * (2 + (size_t)hd), scratch);
             if (rc != TF_OK) return rc;
         }
-        // head_dim 512: the wide kernel where the model below prices it lower.  Both kernels have one block on a compute unit; a block takes
-        // about 0.092 us a key here and 0.1 us in the wide kernel, for 64 and 128 columns.  So the wide kernel wins wherever its
-        // blocks, half as many a chunk, still fill the chip: 128 queries over 32768 keys (256 blocks either way) 310 -> 218 us, 500 over
+        // head_dim 512: the wide kernel where the model prices it lower.  Both kernels have one block on a compute unit, so the wide one wins wherever
+        // its blocks, half as many a chunk, still fill the chip: 128 queries over 32768 keys (256 blocks either way) 310 -> 218 us, 500 over
         // 2000 120 -> 81, 160 over 24160 493 -> 205; but 77 over 3077 (120 blocks for 240) 44 -> 48 and 128 over 768 (48 for 96) 37 -> 43.
         bool wide = false;
         if (hd == 512) {
             const uint32_t wide_blocks = (s.count * group + kWideCols - 1) / kWideCols, wide_base = wide_blocks * s.num_kv_heads, cus = (uint32_t)ctx->num_cus;
-            // in keys: the longest compute unit's blocks, one at a time (20 blocks a chunk: 12 chunks in one go, not 13 in two), and the
-            // merge, where a chunk's partial states of 195 columns cost as much as a key of a block (4 KB a column written and read
-            // back at 8 TB/s).  How many chunks depends on the shape and the device alone where the context is reserved for the call; one that
-            // takes it beyond its limits may hold the states of fewer.
-            auto price = [&](uint32_t blocks, uint32_t c, float key) {
-                return (float)((blocks * c + cus - 1) / cus) * (float)span / (float)c * key + (c > 1 ? (float)s.count * (float)s.num_q_heads * (float)c / 195.0f : 0.0f);
-            };
+            // How many chunks depends on the shape and the device alone where the context is reserved for the call; one that takes it beyond its
+            // limits may hold the states of fewer.
             uint32_t best = 1;
             const uint32_t most = std::min({span / kMinChunkKeys, kMaxPrefillChunks, kWideGoes * cus / wide_base});
+            auto us = [&](uint32_t c) { return attn_us(kWideCost, wide_base, c, span, states_of(c), cus); };
             for (uint32_t c = 2; c <= most && states_of(c) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes; ++c)
-                if (price(wide_base, c, 1.0f) < price(wide_base, best, 1.0f)) best = c;
-            wide = price(wide_base, best, 1.0f) < price(base, chunks, 0.92f);
+                if (us(c) < us(best)) best = c;
+            wide = us(best) < 0.97f * attn_us(cost, base, chunks, span, states_of(chunks), target);      // clearly: 1000 queries of 4 / 4 heads over 2000 keys 57 -> 60 at equal prices
             if (wide) {
                 col_blocks = wide_blocks;
                 base = wide_base;
