@@ -52,7 +52,7 @@ def test_calls_beyond_the_limits_are_refused_until_reserved():
     rc = k.lm_head_greedy(*t, tok, d, vocab, raise_on_error=False)
     assert rc == tfk.TF_ERR_SCRATCH_TOO_SMALL and "tf_ctx_reserve" in k.last_error()
     assert host(tok, np.uint32, 1)[0] == 0xEEEEEEEE                      # nothing was enqueued
-    # the truncating sampler keeps up to 256 candidates of every 1024-element tile in wrapper scratch
+    # the truncating sampler keeps the maximum of every 64 probabilities in wrapper scratch
     probs = dev(f16(np.full(vocab, 1.0 / vocab)))
     rc = k.lib.tf_sample(k.handle, None, probs.data_ptr(), tok.data_ptr(), vocab, 1.0, 200, 0.9, 7, 0)
     assert rc == tfk.TF_ERR_SCRATCH_TOO_SMALL and "tf_ctx_reserve" in k.last_error()
@@ -61,6 +61,25 @@ def test_calls_beyond_the_limits_are_refused_until_reserved():
     k.check(k.lm_head_greedy(*t, tok, d, vocab, raise_on_error=False))
     torch.cuda.synchronize()
     assert int(host(tok, np.uint32, 1)[0]) == tfo.lm_head_cpu_greedy(hidden, norm, W, S, B, threads=8)
+    k.close()
+
+
+def test_truncating_samplers_take_what_the_limit_says():
+    # the limit in whole 1024 elements, four times as many for k <= 64; neither one element more nor one fewer
+    import torch
+    k = tfk.Context(0)
+    probs = torch.full((4 * 300032 + 1,), 0.25, dtype=torch.float16, device="cuda")
+    tok = zeros_bytes(4, 0xEE)
+
+    def sample(v, top_k):
+        return k.lib.tf_sample(k.handle, None, probs.data_ptr(), tok.data_ptr(), v, 1.0, top_k, 0.9, 7, 0)
+
+    for admitted in (262144, 300032):
+        assert sample(admitted + 1, 200) == tfk.TF_ERR_SCRATCH_TOO_SMALL and "tf_ctx_reserve" in k.last_error()
+        assert sample(4 * admitted + 1, 64) == tfk.TF_ERR_SCRATCH_TOO_SMALL
+        assert sample(admitted, 200) == tfk.TF_OK and sample(4 * admitted, 64) == tfk.TF_OK
+        k.reserve(max_vocab=300000)
+    assert host(tok, np.uint32, 1)[0] < 64
     k.close()
 
 

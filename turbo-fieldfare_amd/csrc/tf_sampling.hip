@@ -545,6 +545,9 @@ constexpr size_t kPartialBytes = kSoftmaxMaxBlocks * 2 * sizeof(float);
 
 size_t sample_need(size_t elements) { return kCellBytes + kPartialBytes + (elements / kTopkChunk + 1) * sizeof(uint16_t); }
 
+// The truncating samplers take vocabularies up to the limit in whole 1024 elements, four times as many for k <= 64
+size_t topk_admitted(uint32_t max_vocab) { return ((size_t)max_vocab + 1023) / 1024 * 1024; }
+
 int32_t sample_scratch(tf_ctx *ctx, size_t elements, SampleScratch &out) {
     const size_t need = sample_need(elements);
     if (ctx->sample_scratch_bytes < need) return scratch_too_small(ctx, "sampler", need, ctx->sample_scratch_bytes);
@@ -572,8 +575,9 @@ int32_t launch_truncating_sampler(tf_ctx *ctx, hipStream_t st, const half_t *pro
     uint16_t *chunk_max = nullptr;
     if (v > most) {
         SampleScratch sc;
-        // the limits admit vocabularies up to max_vocab, four times that for k <= 64
-        const int32_t rc = sample_scratch(ctx, (k <= 64 ? 1u : kTopkVocabFactor) * (size_t)v, sc);
+        const size_t admitted = topk_admitted(ctx->limits.max_vocab) * (k <= 64 ? kTopkVocabFactor : 1u);
+        if (v > admitted) return scratch_too_small(ctx, "sampler", sample_need(v), sample_need(admitted));
+        const int32_t rc = sample_scratch(ctx, v, sc);
         if (rc != TF_OK) return rc;
         chunk_max = sc.chunk_max;
         const dim3 grid((v + 2047) / 2048);
@@ -589,7 +593,7 @@ int32_t launch_truncating_sampler(tf_ctx *ctx, hipStream_t st, const half_t *pro
 
 namespace tfk {
 
-size_t sample_scratch_bytes_for(uint32_t vocab) { return sample_need(kTopkVocabFactor * (size_t)vocab); }
+size_t sample_scratch_bytes_for(uint32_t vocab) { return sample_need(kTopkVocabFactor * topk_admitted(vocab)); }
 size_t sample_scratch_clear_bytes() { return kCellBytes; }
 
 }  // namespace tfk
