@@ -80,6 +80,23 @@ def test_softcap_softmax_matches_reference(v, dtype):
     assert int(np.argmax(got)) == int(np.argmax(ref)) or ref[int(np.argmax(got))] >= ref.max() * (1 - 2e-3)
 
 
+def test_softcap_softmax_of_the_longest_rows():
+    # every thread's walk ends although its last index is less than a stride from 2^32: the last element holds nearly all of the mass,
+    # e^30 against 2^32 others
+    import torch
+    k = ctx()
+    v = (1 << 32) - 3
+    logits, probs = (torch.zeros(v, dtype=torch.float16, device="cuda") for _ in range(2))
+    logits[-1] = 60000.0
+    probs[0] = 1.0
+    k.check(k.lib.tf_logit_softcap_softmax(k.handle, None, logits.data_ptr(), probs.data_ptr(), v, 30.0, tfk.TF_FP16))
+    torch.cuda.synchronize()
+    want = 1.0 / (1.0 + (v - 1) * np.exp(-30.0))
+    assert abs(float(probs[-1]) - want) < 2 ** -11 and int(torch.count_nonzero(probs)) == 1
+    del logits, probs
+    torch.cuda.empty_cache()
+
+
 def test_softcap_softmax_uniform_and_saturated_inputs():
     # LogitSoftcapSoftmaxTests.swift:56-89
     k = ctx()

@@ -81,14 +81,14 @@ constexpr uint32_t kSoftmaxRun = 4;
 // logits [i, i + 4) below v; missing ones are -inf.  VEC: the row is aligned to whole runs
 template <bool VEC, typename T>
 __device__ __forceinline__ void load_run(const T *logits, uint32_t i, uint32_t v, float z[kSoftmaxRun]) {
-    if (VEC && i + kSoftmaxRun <= v) {
+    if (VEC && i < v && v - i >= kSoftmaxRun) {
         typedef T run_t __attribute__((ext_vector_type(kSoftmaxRun)));
         const run_t x = *reinterpret_cast<const run_t *>(logits + i);
 #pragma unroll
         for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = (float)x[j];
     } else {
 #pragma unroll
-        for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = i + j < v ? (float)logits[i + j] : -INFINITY;
+        for (uint32_t j = 0; j < kSoftmaxRun; ++j) z[j] = i < v && j < v - i ? (float)logits[i + j] : -INFINITY;
     }
 }
 
@@ -96,18 +96,20 @@ template <bool VEC, typename T>
 __global__ __launch_bounds__(256) void softmax_partials_kernel(const T *logits, float *partials, uint32_t v, float softcap) {
     __shared__ float scratch[8];
     float m = -INFINITY, d = 0.0f;
-    for (uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) * kSoftmaxRun; i < v; i += gridDim.x * blockDim.x * kSoftmaxRun) {
+    // counted in runs: elements of a vocabulary near 2^32 would wrap and the loop never end
+    for (uint32_t run = blockIdx.x * blockDim.x + threadIdx.x; run <= (v - 1) / kSoftmaxRun; run += gridDim.x * blockDim.x) {
+        const uint32_t i = run * kSoftmaxRun;
         float z[kSoftmaxRun], mn = m;
         load_run<VEC>(logits, i, v, z);
 #pragma unroll
         for (uint32_t j = 0; j < kSoftmaxRun; ++j) {
-            z[j] = i + j < v ? softcapped(z[j], softcap) : -INFINITY;
+            z[j] = j < v - i ? softcapped(z[j], softcap) : -INFINITY;
             mn = fmaxf(mn, z[j]);
         }
         d = (m == -INFINITY) ? 0.0f : d * expf(m - mn);
 #pragma unroll
         for (uint32_t j = 0; j < kSoftmaxRun; ++j)
-            if (i + j < v) d += expf(z[j] - mn);
+            if (j < v - i) d += expf(z[j] - mn);
         m = mn;
     }
     block_merge_md(m, d, scratch);
@@ -137,19 +139,19 @@ __global__ __launch_bounds__(256) void softmax_normalize_kernel(const T *logits,
     half_t p[kSoftmaxRun];
 #pragma unroll
     for (uint32_t j = 0; j < kSoftmaxRun; ++j) p[j] = to_half_pinned(expf(z[j] - m) * inv_d);
-    if (VEC && i + kSoftmaxRun <= v) {
+    if (VEC && v - i >= kSoftmaxRun) {
         typedef half_t run_t __attribute__((ext_vector_type(kSoftmaxRun)));
         *reinterpret_cast<run_t *>(probs + i) = run_t{p[0], p[1], p[2], p[3]};
     } else {
 #pragma unroll
         for (uint32_t j = 0; j < kSoftmaxRun; ++j)
-            if (i + j < v) probs[i + j] = p[j];
+            if (j < v - i) probs[i + j] = p[j];
     }
 }
 
 template <typename T>
 void launch_softmax(hipStream_t st, const T *logits, float *partials, half_t *probs, uint32_t v, float softcap) {
-    const uint32_t runs = (v + 256 * kSoftmaxRun - 1) / (256 * kSoftmaxRun), blocks = runs < kSoftmaxMaxBlocks ? runs : kSoftmaxMaxBlocks;
+    const uint32_t runs = (v - 1) / (256 * kSoftmaxRun) + 1, blocks = runs < kSoftmaxMaxBlocks ? runs : kSoftmaxMaxBlocks;
     if (aligned16(logits) && aligned(probs, sizeof(half_t) * kSoftmaxRun)) {
         hipLaunchKernelGGL((softmax_partials_kernel<true, T>), dim3(blocks), dim3(256), 0, st, logits, partials, v, softcap);
         hipLaunchKernelGGL((softmax_normalize_kernel<true, T>), dim3(runs), dim3(256), 0, st, logits, partials, blocks, probs, v, softcap);
@@ -237,14 +239,14 @@ template <bool VEC>
 __global__ __launch_bounds__(256) void chunk_max_kernel(const uint16_t *probs, uint16_t *chunk_max, uint32_t v) {
     const uint32_t piece = blockIdx.x * 256 + threadIdx.x, first = piece * 8;
     uint32_t best = 0;
-    if (VEC && first + 8 <= v) {
+    if (VEC && first < v && v - first >= 8) {
         const u32x4 w = *reinterpret_cast<const u32x4 *>(probs + first);
 #pragma unroll
         for (int i = 0; i < 4; ++i) best = max(best, max(prob_key((uint16_t)w[i]), prob_key((uint16_t)(w[i] >> 16))));
     } else {
 #pragma unroll
         for (uint32_t i = 0; i < 8; ++i)
-            if (first + i < v) best = max(best, prob_key(probs[first + i]));
+            if (first < v && i < v - first) best = max(best, prob_key(probs[first + i]));
     }
 #pragma unroll
     for (int off = 1; off < 8; off <<= 1) best = max(best, (uint32_t)__shfl_xor((int)best, off, kWave));
@@ -402,7 +404,7 @@ __global__ __launch_bounds__(kTopkThreads) void topk_final_kernel(const uint16_t
         best[t] = 0;
     }
     if (chunk_max) {
-        const uint32_t chunks = (v + kTopkChunk - 1) / kTopkChunk, rounds = (chunks + kTopkThreads - 1) / kTopkThreads;
+        const uint32_t chunks = (v - 1) / kTopkChunk + 1, rounds = (chunks + kTopkThreads - 1) / kTopkThreads;
         auto maximum = [&](uint32_t r) { return r * kTopkThreads + t < chunks ? (uint32_t)chunk_max[r * kTopkThreads + t] : 0u; };
         uint32_t cached[kRounds];
 #pragma unroll
@@ -580,7 +582,7 @@ int32_t launch_truncating_sampler(tf_ctx *ctx, hipStream_t st, const half_t *pro
         const int32_t rc = sample_scratch(ctx, v, sc);
         if (rc != TF_OK) return rc;
         chunk_max = sc.chunk_max;
-        const dim3 grid((v + 2047) / 2048);
+        const dim3 grid((v - 1) / 2048 + 1);
         if (aligned16(probs)) hipLaunchKernelGGL(chunk_max_kernel<true>, grid, dim3(256), 0, st, bits, chunk_max, v);
         else hipLaunchKernelGGL(chunk_max_kernel<false>, grid, dim3(256), 0, st, bits, chunk_max, v);
     }
