@@ -1,5 +1,6 @@
-"""Register spills of the built kernels, from the metadata the compiler leaves in the library (no GPU needed).  A kernel that
-touches scratch memory is dispatched more slowly and waits for it in its loop."""
+"""What the built library says without a GPU: register spills of its kernels, from the metadata the compiler leaves in it (a kernel that
+touches scratch memory is dispatched more slowly and waits for it in its loop), and a rule that picks kernels by the device's size."""
+import ctypes
 import importlib
 import os
 import struct
@@ -47,3 +48,19 @@ def test_matrix_core_loops_keep_their_registers(name):
     found = {k[".name"]: k for k in kernels() if f"{len(name)}{name}" in k[".name"]}
     assert found
     assert not {n: k[".vgpr_spill_count"] for n, k in found.items() if k[".vgpr_spill_count"] or k[".private_segment_fixed_size"]}
+
+
+@pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
+def test_split_tiles_are_chosen_by_the_compute_units_there_are():
+    variant = getattr(ctypes.CDLL(LIB), "_ZN3tfk17qmm_split_variantEiiili")      # tfk::qmm_split_variant(m, n, k, ldx, num_cus)
+    variant.argtypes, variant.restype = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_long, ctypes.c_int], ctypes.c_int
+    none, t32x32, t64x32, t64x64 = range(4)
+    tiles = {t32x32: (32, 32), t64x32: (64, 32), t64x64: (64, 64)}
+    for cus in (32, 64, 128, 256, 304):
+        for m in (1, 32, 33, 64, 65, 128, 200, 500, 1000):
+            for n in (64, 2048, 2816, 8192):
+                short, got = variant(m, n, 1024, 1024, cus), variant(m, n, 2816, 2816, cus)
+                goes = {t: -(-m // rows) * -(-n // cols) / cus for t, (rows, cols) in tiles.items()}
+                first = next((t for t in tiles if goes[t] <= 1), t64x64 if m > 64 and goes[t64x64] <= 2 else none)
+                assert got == first and short == (none if goes[t64x64] > 1 else first), (cus, m, n)       # two goes only for longer contractions
+        assert variant(32, 64, 960, 960, cus) == none and variant(32, 64, 8256, 8256, cus) == none

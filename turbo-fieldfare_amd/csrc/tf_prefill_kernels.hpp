@@ -83,7 +83,7 @@ int32_t launch_grouped_quad(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab,
 // Dense products whose waves split the contraction (tf_qmm_split.hip).  qmm_split_variant: kSplitNone where the 128 x 256 tiles are the
 // better kernel, otherwise what launch_qmm_split is to be given; operands as qmm_operands_ok() demands.
 enum { kSplitNone = 0, kSplit32x32, kSplit64x32, kSplit64x64 };
-int qmm_split_variant(int m, int n, int k, long ldx);
+int qmm_split_variant(int m, int n, int k, long ldx, int num_cus);
 int32_t launch_qmm_split(tf_ctx *ctx, hipStream_t st, int variant, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
                          half_t *y, long ldy, int m, int n, int k, tf_dtype sd);
 // the same for a gate and an up matrix with GeGLU (rows of up to 4096 columns either way, so that the result can also be had inside a grouped launch)

@@ -531,7 +531,7 @@ int32_t launch_grouped_down_mfma(tf_ctx *ctx, hipStream_t st, const ExpertTable 
     const GroupedDownArgs a = {tab, off, cl, pairs, acts, acts_pair_base, route_partials, d, f, top_k};
     if (ride) {
         const tf_projection *dn = ride->down;   // ride->y: 16-byte aligned rows of whole 16-byte pieces (dense_ride_ok)
-        const int variant = ride->split ? qmm_split_variant(ride->rows, (int)dn->rows, (int)dn->cols, (long)dn->cols) : kSplitNone;
+        const int variant = ride->split ? qmm_split_variant(ride->rows, (int)dn->rows, (int)dn->cols, (long)dn->cols, ctx->num_cus) : kSplitNone;
         if (variant != kSplitNone) {      // the kernel that the product has in a launch of its own
             const SplitArgs split = qmm_split_args(at(dn->weights, dn->weights_offset), at(dn->scales, dn->scales_offset), at(dn->biases, dn->biases_offset),
                                                    ride->acts, (long)dn->cols, ride->y, ride->ldy, ride->rows, (int)dn->rows, (int)dn->cols);
@@ -564,7 +564,7 @@ namespace {
 int32_t launch_qmm_dense(tf_ctx *ctx, hipStream_t st, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
                          half_t *y, long ldy, int m, int n, int k, tf_dtype sd, bool tiles_only = false) {
     if (!tiles_only) {
-        const int variant = qmm_split_variant(m, n, k, ldx);
+        const int variant = qmm_split_variant(m, n, k, ldx, ctx->num_cus);
         if (variant != kSplitNone) return launch_qmm_split(ctx, st, variant, w, s, b, x, ldx, y, ldy, m, n, k, sd);
     }
     const uint32_t col_tiles = (uint32_t)(n + kQmmBN - 1) / kQmmBN;

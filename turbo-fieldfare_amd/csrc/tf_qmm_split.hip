@@ -24,7 +24,7 @@ void launch_split(hipStream_t st, const SplitArgs &a, tf_dtype sd) {
 namespace tfk {
 
 // Which kernel for M x N x K, in microseconds for the shapes below (K = 2816, weights from HBM; `tiles`: the 128 x 256 tile kernel; the
-// others by rows x columns of a block's tile).  A block has a CU to itself, so what counts is how often the 256 CUs are filled:
+// others by rows x columns of a block's tile).  A block has a CU to itself, so what counts is how often the device's CUs (here 256) are filled:
 //     rows x columns    32 x 32   64 x 32   64 x 64    tiles
 //        53 x 2048         8.0      10.2      14.1      26.9
 //       128 x 2048         8.7      10.4      14.4      33.9
@@ -33,14 +33,18 @@ namespace tfk {
 //       500 x 4096        53.9      37.2      28.6      35.5
 //       500 x 8192         107      72.6      53.4      37.2
 // So: the smallest tile that fits the chip in one go; 64 x 64 in two goes while the tile kernel would multiply full row tiles (up to
-// 64 rows it takes 27 - 29 us, no more than two goes do).  Contractions shorter than a pair of groups a wave, or longer than the waves'
+// 64 rows it takes 27 - 29 us, no more than two goes do).  Other contractions, 1 to 1200 rows of 64 to 8192 columns against the tile kernel alone:
+// K 8192 1.0 to 4 times as fast (53 x 2816 70.8 -> 17.6 us, 500 x 2816 in two goes 94.1 -> 63.6), K 1024 1.1 to 2.2 times in one go
+// but no gain in two (500 x 4096 16.8 -> 17.6 us; a thousand more of K are 6.3 us in two goes and 10.4 on the tiles).  Contractions shorter than a pair of groups a wave, or longer than the waves'
 // scale areas hold, stay with the tile kernel.
-int qmm_split_variant(int m, int n, int k, long ldx) {
+constexpr int kTwoGoesK = 1280;
+int qmm_split_variant(int m, int n, int k, long ldx, int num_cus) {
     if (k < 1024 || k > 8192 || ldx > (1l << 24)) return kSplitNone;
+    const int64_t cus = num_cus;
     auto blocks = [&](int rows, int cols) { return (int64_t)((m + (int64_t)rows - 1) / rows) * ((n + (int64_t)cols - 1) / cols); };
-    if (blocks(32, 32) <= 256) return kSplit32x32;
-    if (blocks(64, 32) <= 256) return kSplit64x32;
-    if (blocks(64, 64) <= (m > 64 ? 512 : 256)) return kSplit64x64;
+    if (blocks(32, 32) <= cus) return kSplit32x32;
+    if (blocks(64, 32) <= cus) return kSplit64x32;
+    if (blocks(64, 64) <= (m > 64 && k >= kTwoGoesK ? 2 * cus : cus)) return kSplit64x64;
     return kSplitNone;
 }
 
@@ -77,12 +81,12 @@ int32_t launch_shared8_split(tf_ctx *ctx, hipStream_t st, const tf_projection *g
     const int f = (int)gate->rows, d = (int)gate->cols;
     auto blocks = [&](int n, int rows, int cols) { return (int64_t)((m + (int64_t)rows - 1) / rows) * ((n + (int64_t)cols - 1) / cols); };
     const SplitArgs a1 = geglu_split_args(gate, up, x, ldx, acts, (long)f, m);
-    if (blocks(f, 32, 32) <= 256) launch_split<8, 1, 2, 4, 8, true>(st, a1, sd);
+    if (blocks(f, 32, 32) <= ctx->num_cus) launch_split<8, 1, 2, 4, 8, true>(st, a1, sd);
     else launch_split<8, 2, 2, 4, 8, true>(st, a1, sd);
     const uint8_t *w = at(down->weights, down->weights_offset), *s = at(down->scales, down->scales_offset), *b = at(down->biases, down->biases_offset);
     const SplitArgs a2 = qmm_split_args(w, s, b, acts, (long)f, y, ldy, m, d, f);
-    if (blocks(d, 32, 32) <= 256) launch_split<8, 1, 1, 8, 4, false>(st, a2, sd);
-    else if (blocks(d, 64, 32) <= 256) launch_split<8, 2, 1, 4, 8, false>(st, a2, sd);
+    if (blocks(d, 32, 32) <= ctx->num_cus) launch_split<8, 1, 1, 8, 4, false>(st, a2, sd);
+    else if (blocks(d, 64, 32) <= ctx->num_cus) launch_split<8, 2, 1, 4, 8, false>(st, a2, sd);
     else launch_split<8, 2, 2, 4, 8, false>(st, a2, sd);
     return check_launch(ctx, "shared expert 8-bit block");
 }
