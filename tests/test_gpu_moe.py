@@ -362,7 +362,7 @@ def test_prefill_shared_expert_block_with_8_bit_weights_is_the_row_chain(d, f, r
 
 
 @pytest.mark.parametrize("d,f,rows,pad", [(64, 64, 16, 0), (1088, 1984, 33, 0),           # fewer groups than waves; odd numbers of groups
-                                          (2816, 2112, 97, 8),                          # two row tiles of 64 a gate / up tile, 64 x 64 down tiles
+                                          (2816, 2112, 97, 8),                          # two row tiles of 64 a gate / up tile, 64 x 32 down tiles
                                           (4096, 4096, 40, 0), (4160, 64, 20, 0)])       # the widest rows the split kernels take; wider
 def test_8_bit_block_tile_edges(d, f, rows, pad):
     test_prefill_shared_expert_block_with_8_bit_weights_is_the_row_chain(d, f, rows, pad)
@@ -457,6 +457,66 @@ def test_prefill_shared_expert_block_on_matrix_cores(rows, d, f, x_stride, y_str
     chain = _repeated_rows(c, min(rows, 3))
     for r in range(min(rows, 3)):
         assert tfo.rel_error(tfo.from_f16_bits(y[r, :d]), tfo.from_f16_bits(chain[r])) < 6e-3
+
+
+def _random_affine(gen, rows, cols, bits, fp16, small):
+    """Codes, scales, biases (as bits) and the exact weights in 64 bits; small: "rows" makes every third row's scales about 1e-5 (below
+    fp16's normal range; weights of 1e-4), "groups" does so in every fifth group of every other row."""
+    W = torch.randint(0, 256, (rows, cols * bits // 8), dtype=torch.uint8, device="cuda", generator=gen)
+    lo, hi = (0.004, 0.02) if bits == 4 else (0.0003, 0.0012)
+    s = torch.rand((rows, cols // 64), device="cuda", generator=gen) * (hi - lo) + lo
+    if small == "rows":
+        s[::3] *= 1e-5 / hi
+    elif small == "groups":
+        s[::2, ::5] *= 1e-5 / hi
+    b = -(7.5 if bits == 4 else 127.5) * s * (torch.rand(s.shape, device="cuda", generator=gen) + 0.5)
+    dtype = torch.float16 if fp16 else torch.bfloat16
+    s, b = s.to(dtype), b.to(dtype)
+    q = W.double() if bits == 8 else torch.stack([W & 15, W >> 4], 2).reshape(rows, cols).double()
+    return (W, s, b), q * s.double().repeat_interleave(64, 1) + b.double().repeat_interleave(64, 1)
+
+
+@pytest.mark.parametrize("bits,rows,d,f,fp16,small", [
+    # 4 bits, split kernels (8 to 79 rows): eight runs, all of them busy; odd numbers of groups and rows; the widest rows; small scales of gate, up and down
+    (4, 53, 2816, 2112, False, None), (4, 79, 1088, 1984, True, None), (4, 40, 4096, 4096, True, None), (4, 33, 2816, 2112, False, "rows"),
+    (4, 65, 2816, 2112, False, "groups"),
+    # dense tiles: rows too wide for the split kernels, more rows
+    (4, 16, 4160, 64, False, None), (4, 80, 2816, 2112, True, None),
+    # 8 bits: 32 x 32, 64 x 32 and 64 x 64 down tiles, fp16 scales, small scales through each
+    (8, 16, 2816, 2112, True, "rows"), (8, 97, 2816, 2112, False, "groups"), (8, 129, 2816, 2112, False, None), (8, 200, 2816, 2112, True, None),
+    (8, 200, 2816, 2112, False, "rows"), (8, 33, 1088, 1984, True, None),
+])
+def test_shared_expert_block_against_64_bit_sums(bits, rows, d, f, fp16, small):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows * 7919 + d + f + bits)
+    mats = [_random_affine(gen, *shape, bits, fp16, small) for shape in ((f, d), (f, d), (d, f))]
+    (gate, wg), (up, wu), (down, wd) = mats
+    x = (torch.randn((rows, d), device="cuda", generator=gen) * 0.25).half()
+    y = torch.full((rows, d), float("nan"), dtype=torch.float16, device="cuda")
+    sg, su, sa = zeros_bytes(f * 2), zeros_bytes(f * 2), zeros_bytes(f * 2)
+    k = tfk.Context(0)
+    k.reserve(max_shared_intermediate=f)
+    rc = k.prefill_shared_expert_block(x, _proj(*gate, f, d), _proj(*up, f, d), _proj(*down, d, f), y, sg, su, sa, rows, d, f, weight_bits=bits,
+                                       scale_dtype=tfk.TF_FP16 if fp16 else tfk.TF_BF16, raise_on_error=False)
+    assert rc == tfk.TF_OK, k.last_error()
+    torch.cuda.synchronize()
+    k.close()
+    # Neighbouring fp16 numbers are at most 2^-10 of their size apart, so rounding a weight has a deviation of at most 2^-10 / sqrt(12) of it;
+    # roundings are independent, so a sum's deviation is that of sqrt(sum of (a w)^2).  Six deviations, and a fp16 rounding of every sum and
+    # activation (gelu's slope is below 1.13); a weight below fp16's normal range (beside ordinary groups of its row) is at most 2^-25 off.
+    def product(a, w, error):
+        half = 2.0 ** -11
+        spread = 6 * 2 * half / 12 ** 0.5 * ((a ** 2) @ (w ** 2).T.contiguous()).sqrt() + 2.0 ** -25 * a.norm(dim=1, keepdim=True)
+        v = a @ w.T.contiguous()
+        return v, spread + (0.0 if error is None else ((error ** 2) @ (w ** 2).T.contiguous()).sqrt()) + half * v.abs() + 2.0 ** -25
+    g, eg = product(x.double(), wg, None)
+    u, eu = product(x.double(), wu, None)
+    gelu = 0.5 * g * (1 + torch.tanh(0.7978845608028654 * (g + 0.044715 * g ** 3)))
+    act = gelu * u
+    want, bound = product(act, wd, 1.13 * eg * u.abs() + gelu.abs() * eu + 1.13 * eg * eu + 2.0 ** -11 * act.abs() + 2.0 ** -25)
+    off = (y.double() - want).abs()
+    assert torch.all(off <= bound), float((off / bound).max())
+    assert float(((y.double() - want).norm() / want.norm())) < (6e-3 if bits == 4 else tfo.Tolerance.quantInt8 * 4)
 
 
 def test_prefill_shared_expert_block_with_gate_and_up_scales_far_apart_takes_the_row_chain():
