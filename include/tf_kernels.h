@@ -335,8 +335,8 @@ int32_t tf_shared_expert_int8_down(tf_ctx *ctx, tf_stream stream, const tf_proje
  * query_count rows of x (row stride x_stride_elements halves) into query_count rows of y.  The reference runs the
  * single-row chain once per row through the same one-row scratch buffers; so does this entry for fewer than 8 rows and
  * for operands the matrix-core path cannot take (weights or x rows not 16-byte aligned, intermediate % 64 != 0, the scale
- * or the bias arrays of gate and up more than 2 GiB apart; with that last reason alone and rows of more than 1024 the chain's
- * bits come from two launches over all rows, activations in the buffer the context owns).
+ * or the bias arrays of gate and up more than 2 GiB apart; with that last reason alone, d and intermediate above 1024, the
+ * chain's bits come from two launches over all rows, activations in the buffer the context owns).
  * Otherwise the rows go through the matrix cores: gate and up in one pass with both sums rounded to fp16 before GeGLU
  * (the chain's stage boundary), activations in a buffer the context owns, then the down projection; weights are
  * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm, so results agree with the row chain within the shared

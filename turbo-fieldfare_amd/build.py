@@ -21,8 +21,11 @@ FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-Wall", "-Wno-u
 # does not preload).  The decode kernels are a launch and two or three memory round trips long, so that load is on the critical
 # path: 0.15 us of the three-launch decode step, 0.4 us of the eight-launch decoder layer.
 FLAGS += ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
-# tf_prefill_quad.hip: the scheduler's register-pressure trackers let the 8-pair gate / up quad kernel fit three blocks a CU (165
-# registers, no spill; without them 168 and one spill).  Only that file: the other kernels measured slightly slower with them.
+# Flags that single files measured faster with.
+#   tf_prefill_quad.hip: the scheduler's register-pressure trackers let the 8-pair gate / up quad kernel fit three blocks a CU (167 registers, no
+#     spill; without them 168 and six spills); the other kernels measured slightly slower with them.
+#   tf_qmm_split.hip: sums in ordinary registers instead of the second half of the register file: tiles of 64 rows take 178 registers instead of
+#     240 (8-bit shared expert of 200 / 500 / 2048 rows 41.4 / 71.1 / 213 -> 37.3 / 65.0 / 196 us; tiles of 32 rows the same either way).
 EXTRA_FLAGS: dict = {"tf_prefill_quad.hip": ["-mllvm", "-amdgpu-use-amdgpu-trackers=1"],
                      "tf_qmm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 

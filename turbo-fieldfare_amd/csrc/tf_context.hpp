@@ -84,11 +84,15 @@ size_t sample_scratch_clear_bytes();                                            
 size_t prefill_logits_floats_for(uint32_t tokens, uint32_t experts);                // tf_prefill.hip
 size_t attention_scratch_floats_for(int num_cus, uint32_t q_heads, uint32_t head_dim, uint32_t block_tokens);   // tf_attention.hip
 
+// The 4-bit shared expert's single-row chain over a block of rows (tf_moe.hip), for the block entry (tf_qmm.hip) where the gate and up arrays lie
+// out of each other's reach: two launches, every row bit-identical to the chain.  acts: [rows, intermediate] fp16 scratch, 16-byte aligned.
+// TF_ERR_UNAVAILABLE, with nothing enqueued, where the chain would not take the kernels for long aligned rows (d and intermediate above
+// 1024, weights, x rows and acts 16-byte aligned, bf16 or fp16 scales): the caller runs the rows one by one.
+int32_t shared4_rows(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const void *x,
+                     uint32_t x_stride_elements, void *y, uint32_t y_stride_elements, uint32_t rows, void *acts, tf_dtype scale_dtype);
 // The 8-bit shared expert over a block of rows (tf_moe.hip), for the block entry of the shared expert (tf_qmm.hip): two
 // launches, every row bit-identical to the single-row chain.  acts: [rows, intermediate] fp16 scratch.  TF_ERR_UNAVAILABLE when
 // the operands do not allow it (alignment, K > 4096): the caller runs the rows one by one.
-int32_t shared4_rows(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const void *x,
-                     uint32_t x_stride_elements, void *y, uint32_t y_stride_elements, uint32_t rows, void *acts, tf_dtype scale_dtype);
 int32_t shared8_block(tf_ctx *ctx, hipStream_t st, const tf_projection *gate, const tf_projection *up, const tf_projection *down, const void *x,
                       uint32_t x_stride_elements, void *y, uint32_t y_stride_elements, uint32_t rows, void *acts, tf_dtype scale_dtype);
 

@@ -815,11 +815,14 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     const bool p1_fast = blobs16 && hidden16 && off.gate_W_off % 16 == 0 && off.up_W_off % 16 == 0;
     const bool dn_fast = blobs16 && acts16 && off.down_W_off % 16 == 0;
     int32_t rc;
-    // Fewer than five pairs per expert on average: the quad kernels serve the call (chunks longer than their LDS image in batches).
-    // From there on so few chunks are short that the matrix-core tile kernels are faster (top 8 of 128 experts, rows with a common
-    // direction, quad against tiles: 48 tokens 86 / 87 us, 64: 109 / 94, 72: 118 / 124, 80: 126 / 114, 96: 134 / 110, 128: 163 / 111; below
-    // the line the quad kernels also keep q s + b in 32 bits where the tiles round a weight to fp16.  Running both families in one
-    // call, each on its chunks, was never better than the better of the two).
+    // Fewer than five pairs per expert on average: the quad kernels serve the call (chunks longer than their LDS image in batches); from
+    // there on the matrix-core tile kernels.  Top 8 of 128 experts, quad / tiles, both launches:
+    //     tokens                            32        53        64        72        79        96       128
+    //     experts about equally popular   93/133   103/135   115/136   126/137   124/137   130/134   162/134 us
+    //     rows with a common direction    70/78     91/87     96/75    112/88    110/110   127/92    152/115
+    // So the tiles would pay from about 50 tokens on where a few experts take most of the pairs, and from 100 on where none does.  The host
+    // does not know which, and below the line the quad kernels keep q s + b in 32 bits where the tiles round a weight to fp16: the
+    // line is not moved.  Running both families in one call, each on its chunks, was never better than the better of the two.
     const int p1_passes = ((g.d >> 5) + 15) / 16, dn_passes = ((g.f >> 5) + 7) / 8;
     const bool quad_ok = p1_fast && dn_fast && acts16 && g.d <= kQuadMaxD && p1_passes <= 6 && g.f <= kQuadMaxF && dn_passes <= 4 && g.d % 8 == 0 &&
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;

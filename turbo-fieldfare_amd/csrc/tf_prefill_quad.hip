@@ -301,11 +301,11 @@ __device__ __forceinline__ void quad_pass(const ChunkOperands &o, uint16_t s_bit
 }
 
 // Three blocks a CU is what this kernel is built around: with two, a SIMD's two waves wait for memory at the same time too often
-// (gate / up at 16 tokens: 45.8 us with two blocks, 40.4 us with three).  Registers: 165 a lane with the 8-pair image (this file is
-// compiled with the register-pressure trackers of the scheduler switched on: without them the allocator ends at 168 and one spill,
+// (gate / up at 16 tokens: 45.8 us with two blocks, 40.4 us with three).  Registers: 167 a lane with the 8-pair image (this file is
+// compiled with the register-pressure trackers of the scheduler switched on: without them the allocator ends at 168 and six spills,
 // and a kernel that touches scratch memory dispatches several times slower).  LDS: the image is sized for the rows in use, 52.6 KB at
 // 2816 columns; wider rows (up to kQuadMaxD) leave room for two blocks.
-// MAXP: pairs in the LDS image, 8 or 4.  With four the kernel needs 143 registers and 30 KB; chunks of more than four pairs then
+// MAXP: pairs in the LDS image, 8 or 4.  With four the kernel needs 149 registers and 30 KB; chunks of more than four pairs then
 // go through in two batches, which pays as long as they are rare (calls of up to 96 pairs: 8 / 12 tokens 55.4 / 59.8 -> 54.4 / 58.9 us).
 template <int NPASS, int SD, int MAXP>
 __global__ __launch_bounds__(256, 3) void grouped_phase1_quad_kernel(ExpertTable tab, tf_expert_offsets off, ChunkList cl, uint32_t n_chunks_upper,

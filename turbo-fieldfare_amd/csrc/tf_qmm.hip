@@ -558,9 +558,9 @@ int32_t launch_grouped_down_mfma(tf_ctx *ctx, hipStream_t st, const ExpertTable 
 namespace {
 
 // Y[m, n] = X[m, k] . W[n, k]^T on the matrix cores.  Operands as qmm_operands_ok() demands; ldx / ldy in halves.
-// Products that fill few compute units with 128-row tiles go to the split kernels (qmm_split_variant).  From there on 128-row
-// tiles even when they leave compute units idle (144 blocks at 2048 x 2112): 64-row blocks, twice as many, repeat each weight tile's
-// dequantisation and measured slower (0.18 ms against 0.155 ms for the three shared-expert GEMMs).
+// Products that fill few compute units with 128-row tiles go to the split kernels (qmm_split_variant).  From there on tiles of 128
+// rows, or of 64 where all of those run at once (below); where they do not, 64-row tiles only repeat each weight tile's expansion (the three
+// shared-expert products of 2048 rows: 0.18 ms against 0.155).
 int32_t launch_qmm_dense(tf_ctx *ctx, hipStream_t st, const uint8_t *w, const uint8_t *s, const uint8_t *b, const half_t *x, long ldx,
                          half_t *y, long ldy, int m, int n, int k, tf_dtype sd, bool tiles_only = false) {
     if (!tiles_only) {

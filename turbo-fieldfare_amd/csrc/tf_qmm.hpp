@@ -376,7 +376,8 @@ struct QmmLoop {
     //   second steps (HALF): the next pair's W words and scales are read from LDS, then W of the pair WB after it is requested
     //                        into the same buffer (4 copies);
     //   step (0,1):          also the next cycle's window of scales and biases (2 copies), read from step (2,1) on.
-    // What a step waits for was requested two steps earlier; the counts below are what may still be on its way at each wait.
+    // What a step waits for was requested two steps earlier (weights with two buffers: four); the counts below are what may still be on
+    // its way at each wait.
     template <int U3, int HALF>
     __device__ __forceinline__ void step(int kt, float16_t acc[4][2]) {
         constexpr int base = U3 * kQmmStageBytes;
