@@ -557,6 +557,7 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (72, 16, 2816, 704, 2112, 2824, 4),    # down in four runs, padded output rows
     (8, 8, 512, 128, 192, 512, 4),         # runs without a group; down, a short contraction, as a dense tile
     (40, 16, 192, 64, 1088, 192, 4),       # odd numbers of groups in both stages
+    (40, 16, 192, 64, 1088, 195, 4),       # output rows that cannot leave as 16-byte pieces: the two calls one after the other
     # dense tiles
     (96, 16, 2816, 704, 2112, 2816, 4),    # production row widths
     (97, 16, 2816, 704, 2112, 2816, -4),   # the same bits read as fp16 scales and biases (other numbers, the same equality)
@@ -789,6 +790,20 @@ def test_int4_qmm_with_the_contraction_split_between_waves(m, n, k, fp16_scales,
     # it; roundings are independent, so the sum's deviation is that of sqrt(sum of (x w)^2); six deviations and the output's own rounding
     bound = 6 * 2.0 ** -10 / np.sqrt(12) * np.sqrt((tfo.from_f16_bits(x).reshape(m, k).astype(np.float64) ** 2) @ (wf ** 2).T) + 2.0 ** -11 * np.abs(exact)
     assert np.all(np.abs(got - exact) <= bound), float(np.max(np.abs(got - exact) / bound))
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 96, 1152), (70, 2752, 1024), (65, 4130, 1088)])     # 32 x 32, 64 x 32 and 64 x 64 tiles
+@pytest.mark.parametrize("off_s,off_b", [(2, 0), (0, 2), (2, 6)])
+def test_split_kernels_read_scales_off_word_boundaries(m, n, k, off_s, off_b):
+    # scales and biases that are only 2-byte aligned are fetched one by one instead of in pairs: the same numbers, the same bits
+    W, S, B, x = mpp_inputs(m, n, k)
+    kk = ctx()
+    dW, dx, outs = dev(W), dev(x), []
+    for s_at, b_at in ((0, 0), (off_s, off_b)):
+        y, dS, dB = zeros_bytes(m * n * 2), dev(S, s_at), dev(B, b_at)
+        kk.check(kk.lib.tf_int4_qmm(kk.handle, None, dW.data_ptr(), 0, dS.data_ptr(), s_at, dB.data_ptr(), b_at, dx.data_ptr(), 0, y.data_ptr(), 0, m, n, k, tfk.TF_BF16))
+        outs.append(host(y, np.uint16))
+    assert np.array_equal(*outs) and outs[0].any()
 
 
 def test_int4_qmm_unavailable_and_exact_variant():
