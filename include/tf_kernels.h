@@ -339,8 +339,8 @@ int32_t tf_shared_expert_int8_down(tf_ctx *ctx, tf_stream stream, const tf_proje
  * chain's bits come from two launches over all rows, activations in the buffer the context owns).
  * Otherwise the rows go through the matrix cores: gate and up in one pass with both sums rounded to fp16 before GeGLU
  * (the chain's stage boundary), activations in a buffer the context owns, then the down projection; weights are
- * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm, so results agree with the row chain within the shared
- * expert's tolerance, not bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is
+ * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm (80 to 256 rows of 1280 to 3072 columns: q*s+b in 32 bits), so
+ * results agree with the row chain within the shared expert's tolerance, not bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is
  * left untouched.  weight_bits == 8 (PrefillSharedExpert's default): up to 15 rows in groups against each weight row,
  * bit-identical to repeated tf_shared_expert_int8; from 16 aligned rows on on the matrix cores with every weight
  * rounded to fp16 first, within the 8-bit shared expert's tolerance of the row chain (scales keep their precision
@@ -736,8 +736,9 @@ int32_t tf_prefill_routed_moe_few_tokens(tf_ctx *ctx, tf_stream stream,
                                          uint32_t f, tf_dtype scale_dtype);
 /* Resident-pool form of the same computation over ALL sorted pairs of a chunk of tokens in one go: experts are
  * pool + expert * pool_stride, the work list comes from tf_prefill_group_pairs_device, nothing is read by the host.  Groups
- * of a few pairs stream each expert row once and apply it to every routed token (weight-read bound, the small-M regime);
- * large groups run as a grouped GEMM on the matrix cores (weights expanded to fp16 in LDS, fp32 accumulation).
+ * of a few pairs stream each expert row once and apply it to every routed token (weight-read bound, the small-M regime), groups of a
+ * few dozen once for every 32 of them; large groups run as a grouped GEMM on the matrix cores (weights expanded to fp16 on the way,
+ * fp32 accumulation).
  * hidden holds pair_count / top_k token rows and every (token, rank) combination appears once among the pairs.
  * acts_scratch: pair_count * f halves.  max_chunks: capacity of `chunks`. */
 int32_t tf_prefill_grouped_routed_moe_resident(tf_ctx *ctx, tf_stream stream,
@@ -752,9 +753,9 @@ int32_t tf_prefill_grouped_routed_moe_resident(tf_ctx *ctx, tf_stream stream,
  * (the reference encodes them back to back in one command buffer: the routed stages of PrefillGroupedRoutedMoE.swift:386-461,
  * then PrefillSharedExpert.encodeBlock, PrefillSharedExpert.swift:12-67).  Neither reads what the other writes, so the
  * shared expert's matrix-core tiles (up to 79 rows its split contractions) are placed ahead of the routed tiles in the same two
- * launches (gate / up / GeGLU, then down) instead of under-filling the chip in launches of their own; results are bit-identical to
- * the two calls.
- * Applies when the routed pairs go to the matrix-core tile kernels and the shared expert is 4-bit with at least 8 rows and
+ * launches (gate / up / GeGLU, then down) instead of under-filling the chip in launches of their own, and from 80 to 256 rows some of
+ * the blocks of the routed launches take them; results are bit-identical to the two calls.
+ * Applies when the routed pairs go to the matrix-core tile or slice kernels and the shared expert is 4-bit with at least 8 rows and
  * 16-byte aligned operands; otherwise the two calls are made one after the other.  Arguments: those of the routed call, then
  * those of the shared call (its d is the routed d, its scale dtype the routed one; query_count token rows). */
 int32_t tf_prefill_grouped_routed_moe_resident_shared(tf_ctx *ctx, tf_stream stream,

@@ -454,6 +454,47 @@ def test_quad_kernels_given_more_batches_than_blocks(T, E, run, singles, blocks_
     assert within_north_star(tfo.from_f16_bits(got), want, abs_=1e-3 * max(1.0, float(np.max(np.abs(want)))))
 
 
+@pytest.mark.parametrize("T,E,d,f,fp16_scales", [
+    (24, 16, 1344, 320, False),     # last slices of one group; two slices of f: six groups of waves
+    (40, 32, 2816, 704, True),      # production widths, fp16 scales and biases
+    (100, 16, 1280, 256, False),    # whole slices; chunks of up to 100 pairs: batches of 32
+    (90, 12, 2880, 448, False),     # scales off word boundaries; twelve slices, the last of one group
+    (80, 8, 1536, 3072, True),      # the widest rows of the down product
+])
+def test_slice_kernels_match_oracle(T, E, d, f, fp16_scales):
+    # From three pairs per expert on: up to 8, 16 and 32 pairs a unit, units cut out of longer chunks, blocks whose share crosses into other units
+    top_k = 8
+    r = resident_pipeline(T, E, d, f, top_k, 0x5100 + T, zipf=True, from_router=False, fp16_scales=fp16_scales)
+    counts = np.bincount(r["idx"].ravel(), minlength=E)
+    assert T * top_k >= 3 * E and counts.max() > 16
+    blobs = [bf16_pool_matching(b, r["off"], d, f) for b in r["blobs"]] if fp16_scales else r["blobs"]      # the oracle reads bf16
+    pool = np.zeros((E, r["stride"]), np.uint8)
+    for e, b in enumerate(blobs):
+        pool[e, :b.size] = b
+    scale = float(np.max(np.abs(tfo.from_f16_bits(r["partials"]))))
+    check_against_oracle(dict(r, blobs=blobs, pool=pool.ravel()), T, d, f, top_k, abs_tol=1e-3 * max(1.0, scale))
+
+
+@pytest.mark.parametrize("run", [1, 3, 33, 128])
+def test_slice_kernels_share_out_any_work_list(run):
+    # A pair's sums do not depend on whom it shares a unit with, and chunks without pairs are passed over.
+    T, E, d, f, top_k = 24, 16, 1344, 320, 8
+    r = resident_pipeline(T, E, d, f, top_k, 0x5200, zipf=True, from_router=False)
+    pairs, n = r["sorted_pairs"], T * top_k
+    chunks, at = [(0, 0, 0)], 0
+    while at < n:
+        end = at
+        while end < n and end - at < run and pairs["expert"][end] == pairs["expert"][at]:
+            end += 1
+        chunks.append((int(pairs["expert"][at]), at, end - at))
+        at = end
+        if len(chunks) % 5 == 0:
+            chunks.append((3, at, 0))
+    chunks.append((1, 0, 0))
+    assert len(chunks) <= 256
+    assert np.array_equal(run_quad_work_list(r, chunks, T, E, d, f, top_k), r["partials"])
+
+
 @pytest.mark.parametrize("T,E,d,f,fp16_scales,pad", [(3, 16, 1536, 128, False, 0), (5, 64, 2048, 256, True, 8), (2, 32, 4096, 64, False, 0),
                                                      (7, 128, 2304, 192, True, 24), (4, 12, 2816, 1024, False, 16)])
 def test_few_tokens_in_one_call_other_row_widths_and_fp16_scales(T, E, d, f, fp16_scales, pad):
@@ -568,6 +609,9 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (64, 16, 512, 128, 192, 512, 8),       # 8-bit shared expert: likewise
     (65, 16, 2816, 704, 2112, 2816, -4),   # the split kernels (down in four runs) with the same bits read as fp16 scales and biases
     (33, 16, 2816, 704, 2112, 2816, -4),   # and with down in eight
+    (96, 16, 1344, 320, 1088, 1347, 4),    # slice kernels, both experts' units in the same launches; odd output rows
+    (256, 16, 1280, 256, 2112, 1280, -4),  # the most rows they take
+    (80, 64, 1280, 256, 3072, 1280, 4),    # the fewest
 ])
 def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, shared_f, y_stride, bits):
     top_k = 8

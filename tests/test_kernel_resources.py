@@ -43,7 +43,7 @@ def kernels():
 
 @pytest.mark.skipif(not os.path.exists(LIB), reason="library not built")
 @pytest.mark.parametrize("name", ["qmm_dense_kernel", "qmm_dense_geglu_kernel", "qmm_split_kernel", "grouped_down_mfma_kernel", "attention_prefill_wide_kernel",
-                                  "attention_prefill_kernel"])
+                                  "attention_prefill_kernel", "grouped_slice_kernel"])
 def test_matrix_core_loops_keep_their_registers(name):
     found = {k[".name"]: k for k in kernels() if f"{len(name)}{name}" in k[".name"]}
     assert found

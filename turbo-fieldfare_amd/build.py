@@ -13,7 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libtf_kernels.so")
-SOURCES = ["tf_context.hip", "tf_gemv.hip", "tf_moe.hip", "tf_lmhead.hip", "tf_prefill.hip", "tf_prefill_quad.hip", "tf_prefill_few.hip", "tf_qmm.hip", "tf_qmm_split.hip", "tf_glue.hip", "tf_sampling.hip", "tf_loader.hip", "tf_attention.hip", "tf_rope.hip", "tf_bench.hip"]
+SOURCES = ["tf_context.hip", "tf_gemv.hip", "tf_moe.hip", "tf_lmhead.hip", "tf_prefill.hip", "tf_prefill_quad.hip", "tf_prefill_slice.hip", "tf_prefill_few.hip", "tf_qmm.hip", "tf_qmm_split.hip", "tf_glue.hip", "tf_sampling.hip", "tf_loader.hip", "tf_attention.hip", "tf_rope.hip", "tf_bench.hip"]
 FLAGS = ["-O3", "--offload-arch=gfx950", "-fPIC", "-std=c++17", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 # Kernel-argument preloading: gfx950 can hand the leading scalar arguments to a wave in registers at launch instead of through
@@ -24,9 +24,11 @@ FLAGS += ["-mllvm", "-amdgpu-kernarg-preload-count=16"]
 # Flags that single files measured faster with.
 #   tf_prefill_quad.hip: the scheduler's register-pressure trackers let the 8-pair gate / up quad kernel fit three blocks a CU (167 registers, no
 #     spill; without them 168 and six spills); the other kernels measured slightly slower with them.
+#   tf_prefill_slice.hip: likewise sums in ordinary registers, which the scaling of a group's products reads.
 #   tf_qmm_split.hip: sums in ordinary registers instead of the second half of the register file: tiles of 64 rows take 178 registers instead of
 #     240 (8-bit shared expert of 200 / 500 / 2048 rows 41.4 / 71.1 / 213 -> 37.3 / 65.0 / 196 us; tiles of 32 rows the same either way).
 EXTRA_FLAGS: dict = {"tf_prefill_quad.hip": ["-mllvm", "-amdgpu-use-amdgpu-trackers=1"],
+                     "tf_prefill_slice.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"],
                      "tf_qmm_split.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=1"]}
 
 

@@ -815,21 +815,31 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     const bool p1_fast = blobs16 && hidden16 && off.gate_W_off % 16 == 0 && off.up_W_off % 16 == 0;
     const bool dn_fast = blobs16 && acts16 && off.down_W_off % 16 == 0;
     int32_t rc;
-    // Fewer than five pairs per expert on average: the quad kernels serve the call (chunks longer than their LDS image in batches); from
-    // there on the matrix-core tile kernels.  Top 8 of 128 experts, quad / tiles, both launches:
-    //     tokens                            32        53        64        72        79        96       128
-    //     experts about equally popular   93/133   103/135   115/136   126/137   124/137   130/134   162/134 us
-    //     rows with a common direction    70/78     91/87     96/75    112/88    110/110   127/92    152/115
-    // So the tiles would pay from about 50 tokens on where a few experts take most of the pairs, and from 100 on where none does.  The host
-    // does not know which, and below the line the quad kernels keep q s + b in 32 bits where the tiles round a weight to fp16: the
-    // line is not moved.  Running both families in one call, each on its chunks, was never better than the better of the two.
+    // Fewer than three pairs per expert on average go to the quad kernels; from there on up to kSharedSliceMaxRows tokens to the slice kernels, more to
+    // the matrix-core tiles.  Top 8 of 128 experts, d 2816, f 704, quad or tiles / slice, both launches, us:
+    //     tokens                              16       32       53       64       96      128      200      300      500
+    //     experts about equally popular     69/78    97/100  115/110  120/112  153/116  155/123  157/129  159/145  171/179
+    //     rows with a common direction      53/49    72/62   104/75   105/76   109/82   111/90   129/106  147/125  163/166
+    // (exactly as many pairs for every one of 64 experts: 3 an expert 55/62, 4 57/62, 6 88/64).  The line above is where a shared expert in the
+    // same call leaves them too: its kernel is chosen by the rows alone, and beside the tiles it would be in launches of its own.  With few experts
+    // the tiles are faster a little earlier (16 experts, 128 / 192 tokens 45/44, 51/59), but a shared expert rides (200 tokens, both 77/72).
+    // Between kSliceRideless and kSharedSplitMaxRows tokens a shared expert rides beside tiles and not here (16 experts, 64 tokens, both 51/56).
+    // Shapes that the slice kernels do not take: quad kernels below five pairs per expert, tiles above.
     const int p1_passes = ((g.d >> 5) + 15) / 16, dn_passes = ((g.f >> 5) + 7) / 8;
     const bool quad_ok = p1_fast && dn_fast && acts16 && g.d <= kQuadMaxD && p1_passes <= 6 && g.f <= kQuadMaxF && dn_passes <= 4 && g.d % 8 == 0 &&
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;
-    const bool quad_pays = !use_mfma || (stream_pairs != 0 && (uint64_t)stream_pairs < (uint64_t)tab.num_experts * 5);
+    const uint64_t experts = tab.num_experts;
+    const bool tiles_carry_shared = stream_tokens > kSliceRideless && stream_tokens <= kSharedSplitMaxRows && stream_pairs >= 5 * experts;
+    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens <= kSharedSliceMaxRows && !tiles_carry_shared &&
+        grouped_slice_ok(tab, cl, n_chunks_upper, stream_pairs, g.d, g.f)) {
+        if (ride && !ride->slice) ride = nullptr;
+        if (ride && ride_taken) *ride_taken = true;
+        return launch_grouped_slice(ctx, st, tab, off, cl, n_chunks_upper, g, sd, ride);
+    }
+    const bool quad_pays = !use_mfma || (stream_pairs != 0 && (uint64_t)stream_pairs < experts * 5);
     if (quad_ok && quad_pays) return launch_grouped_quad(ctx, st, tab, off, cl, n_chunks_upper, g, sd, stream_pairs);
     const bool p1_tiles = use_mfma && p1_fast && acts16, dn_tiles = use_mfma && dn_fast && aligned16(g.route_partials);
-    if (!(p1_tiles && dn_tiles) || (ride && !dense_ride_ok(*ride))) ride = nullptr;
+    if (!(p1_tiles && dn_tiles) || (ride && (ride->slice || !dense_ride_ok(*ride)))) ride = nullptr;
     if (ride && ride_taken) *ride_taken = true;
     // ---- phase 1
     if (p1_tiles) {

@@ -60,8 +60,19 @@ struct DenseRide {
     half_t *y;            // [rows, down->rows], row stride ldy halves
     long ldy;
     int rows;
-    bool split;           // gate / up as launch_geglu_split computes them, down as qmm_split_variant says; else the dense tiles
+    bool split;           // gate / up as launch_geglu_split computes them, down as qmm_split_variant says
+    bool slice;           // both as the slice kernels compute them (neither: the dense tiles)
 };
+
+// Up to here the shared expert's gate / up and down are computed as the split kernels do: in launches of their own beside the quad kernels (53
+// rows of 2112 x 2816: 20 us for both against 50 on the dense tiles), or riding in the routed tiles' launches (the one call, 53 rows, 16 experts
+// of 704 x 2816: 47 us against 56 with dense tiles riding; 32 experts 57 against 58, 64 experts 71 against 75).  The rule asks for the rows
+// alone, never for the experts: the shared expert by itself and the one call give the same bits.
+constexpr uint32_t kSharedSplitMaxRows = 79;
+// From there to here as the slice kernels do, whose shape allows it: in launches of their own (2112 x 2816, 96 / 128 / 200 / 256 rows: 54 / 59 / 62 / 60 us
+// on the dense tiles, 27 / 29 / 35 / 38 so; up to 79 rows 20 - 22 split, 19 - 26 so), or by some of the blocks of the routed slice launches.
+constexpr uint32_t kSharedSliceMaxRows = 256;
+constexpr uint32_t kSliceRideless = 48;
 
 // Operands of the grouped expert stages, as the launch helpers pass them on.
 struct GroupedGeom {
@@ -79,6 +90,14 @@ struct GroupedGeom {
 constexpr int kQuadMaxD = 3072, kQuadMaxF = 1024;
 int32_t launch_grouped_quad(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const tf_expert_offsets &off, const ChunkList &cl,
                             uint32_t n_chunks_upper, const GroupedGeom &g, tf_dtype sd, uint32_t stream_pairs);
+
+// The slice kernels (tf_prefill_slice.hip): the same stages for chunks of a few dozen pairs, activations in registers.
+bool grouped_slice_ok(const ExpertTable &tab, const ChunkList &cl, uint32_t n_chunks_upper, uint32_t pair_count, int d, int f);
+int32_t launch_grouped_slice(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const tf_expert_offsets &off, const ChunkList &cl,
+                             uint32_t n_chunks_upper, const GroupedGeom &g, tf_dtype sd, const DenseRide *ride);
+// and a shared expert's block of rows, in launches of its own or (ride above) beside the routed pairs
+bool shared_slice_ok(const tf_projection *gate);
+int32_t launch_shared_slice(tf_ctx *ctx, hipStream_t st, const DenseRide &ride, tf_dtype sd);
 
 // Dense products whose waves split the contraction (tf_qmm_split.hip).  qmm_split_variant: kSplitNone where the 128 x 256 tiles are the
 // better kernel, otherwise what launch_qmm_split is to be given; operands as qmm_operands_ok() demands.

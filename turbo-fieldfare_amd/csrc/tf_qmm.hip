@@ -612,12 +612,6 @@ int32_t shared_block_acts(tf_ctx *ctx, size_t halves, half_t *&out) {
 }
 
 constexpr uint32_t kSharedBlockMinRows = 8;   // fewer rows go through the single-row chain, bit-identical to decode
-// Up to here the shared expert's gate / up and down are computed as the split kernels do: in launches of their own beside the quad kernels (53
-// rows of 2112 x 2816: 20 us for both against 50 on the dense tiles), or riding in the routed tiles' launches (the one call, 53 rows, 16 experts
-// of 704 x 2816: 47 us against 56 with dense tiles riding; 32 experts 57 against 58, 64 experts 71 against 75).  The rule asks for the rows
-// alone, never for the experts: the shared expert by itself and the one call give the same bits.  From 80 rows on, where top 8 of 128
-// experts leave the quad kernels, the dense tiles ride; the split kernels have not been measured against them there.
-constexpr uint32_t kSharedSplitMaxRows = 79;
 
 // ---- 8-bit projections over a block of rows ----------------------------------------------------------------------
 // Y[M, N] = X[M, K] . W[N, K]^T on the matrix cores with the 8-bit weights expanded on the way into the instruction,
@@ -826,7 +820,9 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
                             qmm_operands_ok(gw, xp, x_stride_elements, (int)d) && aligned16(uw) && aligned16(dw) &&
                             intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX &&
                             geglu_arrays_near(gate, up);
-    const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);      // one choice for the call alone and for a ride
+    // one choice for the call alone and for a ride
+    const bool slice = block_path && query_count > kSharedSplitMaxRows && query_count <= kSharedSliceMaxRows && shared_slice_ok(gate);
+    const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);
     if (plan && !block_path) return TF_OK;
     if (weight_bits == 8 && pointers && even && query_count >= 2) {
         // 8-bit projections.  Up to kShared8MfmaMinRows - 1 rows: rows in groups against each weight row, bit-identical to the
@@ -878,10 +874,12 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
     half_t *acts = nullptr;
     int32_t rc = shared_block_acts(ctx, (size_t)query_count * intermediate, acts);
     if (rc != TF_OK) return rc;
+    const DenseRide ride = {gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count, split, slice};
     if (plan) {
-        *plan = DenseRide{gate, up, down, xp, (long)x_stride_elements, acts, yp, (long)y_stride_elements, (int)query_count, split};
+        *plan = ride;
         return TF_OK;
     }
+    if (slice) return launch_shared_slice(ctx, st, ride, scale_dtype);
     rc = split ? launch_geglu_split(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype)
                : launch_qmm_dense_geglu(ctx, st, gate, up, xp, (long)x_stride_elements, acts, (long)intermediate, (int)query_count, scale_dtype);
     if (rc != TF_OK) return rc;
