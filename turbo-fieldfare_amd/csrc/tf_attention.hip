@@ -365,6 +365,47 @@ __device__ __forceinline__ float column_reduce(float v, Op op) {
     return op(__builtin_bit_cast(float, (uint32_t)q[0]), __builtin_bit_cast(float, (uint32_t)q[1]));
 }
 
+// The online softmax of one tile of 32 keys from t0 on: a lane's eight scores of its column (keys 16 (e / 4) + 4 quad + e % 4) become
+// probabilities.  Maxima are kept in units of log2 (scale2: the scale times log2 e), so that a weight is one subtraction and one exponential.
+// The reference maximum of a column only moves when a score exceeds it by more than kMaxSlack2 (probabilities then reach at most 2^kMaxSlack2,
+// far inside fp16): in most steps no lane's own largest score does, and the column's maximum is not even formed.  d_run is the lane's
+// share of the denominator; the four lanes of a column are added up at the end.  Masks only where a column of the wave does not see the whole
+// tile.  About 45 instructions where forming the maximum and the sum in every step and masking every score took 147.
+constexpr float kLog2e = 1.4426950408889634f, kMaxSlack2 = 11.5f;
+__device__ __forceinline__ void softmax_step(const float4_t acc0, const float4_t acc1, uint32_t t0, int quad, uint32_t first_col, uint32_t last_col, float scale2, float &m_run,
+                                             float &d_run, float &alpha, half8_t &p8) {
+    float sc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sc[e] = (e < 4 ? acc0[e & 3] : acc1[e & 3]) * scale2;
+    if (!__all(t0 >= first_col && t0 + 32u <= last_col)) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const uint32_t p = t0 + (uint32_t)(16 * (e >> 2) + 4 * quad + (e & 3));
+            sc[e] = (p >= first_col && p < last_col) ? sc[e] : -INFINITY;
+        }
+    }
+    float lane_max = sc[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) lane_max = fmaxf(lane_max, sc[e]);
+    alpha = 1.0f;
+    if (__any(lane_max > m_run + kMaxSlack2)) {
+        const float tile_max = column_reduce(lane_max, [](float a, float b) { return fmaxf(a, b); });
+        // stays -inf while the column has seen no key; the first finite maximum costs no rescale (o and d are zero)
+        const bool fresh = m_run == -INFINITY;
+        const float m_new = tile_max > m_run + kMaxSlack2 ? tile_max : m_run;
+        alpha = fresh ? 1.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        d_run *= alpha;
+        m_run = m_new;
+    }
+    const float base = m_run == -INFINITY ? 0.0f : m_run;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const float pe = __builtin_amdgcn_exp2f(sc[e] - base);      // zero for a masked key
+        p8[e] = (half_t)pe;
+        d_run += pe;
+    }
+}
+
 template <int HD>
 __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_prefill_kernel(const half_t *Q, const half_t *K, const half_t *V, half_t *O,
                                                                                            float *m_part, float *d_part, float *o_part, PrefillShape s,
@@ -436,14 +477,15 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
     const attn_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(V + (size_t)kv_head * HD), 0, (int)0xFFFFFFFFu, 0x00020000);
     const uint32_t lane_rows = RPI > 1 ? (uint32_t)(lane / CPR) * NI : 0u, lane_piece = (uint32_t)(lane % CPR) * 16u;
     const uint32_t row_bytes = s.kv_stride * 2u;
-    auto copy_tile = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0) {
+    auto copy_rows = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0, int q) {      // the wave's q-th copy of a tile
         if (wave >= NI) return;               // fewer copies than waves (head_dim 64)
+        const uint32_t n = (uint32_t)wave + (uint32_t)(kAttnWaves * q);
+        const uint32_t p = min(t0 + n + lane_rows, c_hi - 1u);
+        attn_lds_copy16(rsrc, tile + n * BLK, prefill_row(s, p) * row_bytes + lane_piece);
+    };
+    auto copy_tile = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0) {
 #pragma unroll
-        for (int q = 0; q < CPW; ++q) {
-            const uint32_t n = (uint32_t)wave + (uint32_t)(kAttnWaves * q);
-            const uint32_t p = min(t0 + n + lane_rows, c_hi - 1u);
-            attn_lds_copy16(rsrc, tile + n * BLK, prefill_row(s, p) * row_bytes + lane_piece);
-        }
+        for (int q = 0; q < CPW; ++q) copy_rows(rsrc, tile, t0, q);
     };
     const uint32_t k_tile[2] = {(uint32_t)(uintptr_t)k_lds[0], (uint32_t)(uintptr_t)k_lds[1]};
     const uint32_t v_tile[2] = {(uint32_t)(uintptr_t)v_lds[0], (uint32_t)(uintptr_t)v_lds[1]};
@@ -453,7 +495,7 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
 
     // scores of keys 16 j + 4 quad + r of a K tile for column `col`; the reads of a batch of steps are in flight while the
     // previous batch is multiplied
-    auto scores = [&](uint32_t tile, float4_t &acc0, float4_t &acc1) {
+    auto scores = [&](uint32_t tile, float4_t &acc0, float4_t &acc1, auto beside) {      // beside(d): after the matrix work of step d is under way
         const uint32_t at = tile + k_lane;
         acc0 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         acc1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -480,6 +522,7 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
             for (int d = 0; d < DB; ++d) {
                 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, kf[b & 1][2 * d]), qf[b * DB + d], acc0, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, kf[b & 1][2 * d + 1]), qf[b * DB + d], acc1, 0, 0, 0);
+                beside(b * DB + d);
             }
         }
     };
@@ -503,42 +546,22 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
         float4_t acc0, acc1;
-        scores(k_tile[0], acc0, acc1);
+        scores(k_tile[0], acc0, acc1, [](int) {});
         __syncthreads();
         // Step i, first half: start the copies of the tiles two (K) and one (V) ahead, take the scores of tile i + 1, and
         // turn the scores of tile i into probabilities.  Here K tiles i (its scores are in acc0/acc1) and i + 1 and V tile
         // i are in LDS and nobody reads the other two buffers any more.
-        // The reference maximum of a column only moves when a score exceeds it by more than kMaxSlack (probabilities then
-        // reach at most e^kMaxSlack, far inside fp16): after the first tiles the accumulators are hardly ever rescaled.
-        constexpr float kMaxSlack = 8.0f;
+        const float scale2 = s.scale * kLog2e;
         auto first_half = [&](uint32_t i, float &alpha, half8_t &p8, float4_t &next0, float4_t &next1) {
             const uint32_t t0 = c_lo + i * kPrefillKeys, cur = i & 1u;
-            copy_tile(k_rsrc, k_tile[cur], t0 + 2 * kPrefillKeys);
-            copy_tile(v_rsrc, v_tile[cur ^ 1u], t0 + kPrefillKeys);
-            scores(k_tile[cur ^ 1u], next0, next1);   // of tile i + 1 (past the chunk: repeated rows, never used)
-            float sc[8], tile_max = -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t p = t0 + (uint32_t)(16 * (e >> 2) + 4 * quad + (e & 3));
-                const float raw = e < 4 ? acc0[e & 3] : acc1[e & 3];
-                sc[e] = (p >= first_col && p < last_col) ? raw * s.scale : -INFINITY;
-                tile_max = fmaxf(tile_max, sc[e]);
-            }
-            tile_max = column_reduce(tile_max, [](float a, float b) { return fmaxf(a, b); });
-            // stays -inf while the column has seen no key; the first finite maximum costs no rescale (o and d are zero)
-            const bool fresh = m_run == -INFINITY;
-            const float m_new = (fresh || tile_max > m_run + kMaxSlack) ? fmaxf(m_run, tile_max) : m_run;
-            alpha = fresh ? 1.0f : __expf(m_run - m_new);
-            float sum = 0.0f;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pe = exp_weight(sc[e], m_new);
-                p8[e] = (half_t)pe;
-                sum += pe;
-            }
-            sum = column_reduce(sum, [](float a, float b) { return a + b; });
-            d_run = d_run * alpha + sum;
-            m_run = m_new;
+            // The scores of tile i + 1 (past the chunk: repeated rows, never used), and the wave's copies one by one beside them: all at once
+            // they are some hundred cycles in which every wave waits for the load unit.
+            scores(k_tile[cur ^ 1u], next0, next1, [&](int d) {
+                static_assert(2 * CPW == KS, "a copy a step");
+                if (d < CPW) copy_rows(k_rsrc, k_tile[cur], t0 + 2 * kPrefillKeys, d);
+                else copy_rows(v_rsrc, v_tile[cur ^ 1u], t0 + kPrefillKeys, d - CPW);
+            });
+            softmax_step(acc0, acc1, t0, quad, first_col, last_col, scale2, m_run, d_run, alpha, p8);
         };
         // Step i, second half: values.  Slot e of the lane's 8 keys is row 16 (e / 4) + 4 quad + e % 4 of the tile.
         auto second_half = [&](uint32_t i, const half8_t &p8, const float4_t &next0, const float4_t &next1) {
@@ -583,6 +606,7 @@ __global__ __launch_bounds__(kAttnThreads, HD > 256 ? 1 : 2) void attention_pref
         }
     }
 
+    d_run = column_reduce(d_run, [](float a, float b) { return a + b; });
     if (!col_live || (HD < 128 && quad >= 2)) return;      // no barrier follows
     if (num_chunks == 1u) {
         // out[t, head, :] = o / d, zero where the column saw no key
@@ -683,13 +707,13 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
     const attn_rsrc_t k_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(K + (size_t)kv_head * HD), 0, (int)0xFFFFFFFFu, 0x00020000);
     const attn_rsrc_t v_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<half_t *>(V + (size_t)kv_head * HD), 0, (int)0xFFFFFFFFu, 0x00020000);
     const uint32_t row_bytes = s.kv_stride * 2u;
+    auto copy_row = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0, int q, uint32_t lane16) {      // the wave's q-th row of a tile
+        const uint32_t n = (uint32_t)wave + (uint32_t)(kWideWaves * q);
+        attn_lds_copy16(rsrc, tile + n * BLK, prefill_row(s, min(t0 + n, c_hi - 1u)) * row_bytes + lane16);
+    };
     auto copy_tile = [&](attn_rsrc_t rsrc, uint32_t tile, uint32_t t0, uint32_t lane16) {
 #pragma unroll
-        for (int q = 0; q < CPW; ++q) {
-            const uint32_t n = (uint32_t)wave + (uint32_t)(kWideWaves * q);
-            const uint32_t p = min(t0 + n, c_hi - 1u);
-            attn_lds_copy16(rsrc, tile + n * BLK, prefill_row(s, p) * row_bytes + lane16);
-        }
+        for (int q = 0; q < CPW; ++q) copy_row(rsrc, tile, t0, q, lane16);
     };
     const uint32_t k_tile = (uint32_t)(uintptr_t)k_lds[0], v_tile = (uint32_t)(uintptr_t)v_lds[0];      // buffer b: + b TILEB
     const uint32_t p_base = (uint32_t)(uintptr_t)p_lds, p_tile = p_base + (uint32_t)lane * 16u, f_base = (uint32_t)(uintptr_t)col_lds;
@@ -697,7 +721,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
     // four elements 4 col .. of the wave's 64
     const uint32_t k_lane = (uint32_t)(col * BLK + quad * 16), v_lane = (uint32_t)(4 * quad * BLK + wave * 128 + col * 8);
 
-    auto scores = [&](uint32_t tile, float4_t &acc0, float4_t &acc1) {
+    auto scores = [&](uint32_t tile, float4_t &acc0, float4_t &acc1, auto beside) {      // beside(b): after the b-th of eight batches of matrix work is under way
         const uint32_t at = tile + k_lane;
         acc0 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
         acc1 = float4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -720,6 +744,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
                 acc0 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, f[2 * d]), qf[2 * b + d], acc0, 0, 0, 0);
                 acc1 = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, f[2 * d + 1]), qf[2 * b + d], acc1, 0, 0, 0);
             }
+            beside(b);
         }
     };
 
@@ -729,39 +754,21 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
         copy_tile(v_rsrc, v_tile, c_lo, (uint32_t)lane * 16u);
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
-        constexpr float kMaxSlack = 8.0f;      // as above: the reference maximum moves when a score exceeds it by more
         for (uint32_t i = 0; i < n_tiles; ++i) {
             // K and V tile i are in LDS and nobody reads the other two buffers any more (past the chunk: repeated rows, never used)
             const uint32_t t0 = c_lo + i * kPrefillKeys, cur = (i & 1u) * TILEB, other = TILEB - cur;
+            // The wave's eight rows of the next tiles are asked for one by one beside the score products: all at once they are a thousand
+            // cycles in which every wave waits for the load unit.
             uint32_t lane16 = p_tile - p_base;         // made anew in every step, here and below: there are no registers to keep it in
             asm volatile("" : "+v"(lane16));
-            copy_tile(k_rsrc, k_tile + other, t0 + kPrefillKeys, lane16);
-            copy_tile(v_rsrc, v_tile + other, t0 + kPrefillKeys, lane16);
             float4_t acc0, acc1;
-            scores(k_tile + cur, acc0, acc1);
-            float sc[8], tile_max = -INFINITY;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint32_t p = t0 + (uint32_t)(16 * (e >> 2) + 4 * quad + (e & 3));
-                const float raw = e < 4 ? acc0[e & 3] : acc1[e & 3];
-                sc[e] = (p >= first_col && p < last_col) ? raw * s.scale : -INFINITY;
-                tile_max = fmaxf(tile_max, sc[e]);
-            }
-            tile_max = column_reduce(tile_max, [](float a, float b) { return fmaxf(a, b); });
-            const bool fresh = m_run == -INFINITY;
-            const float m_new = (fresh || tile_max > m_run + kMaxSlack) ? fmaxf(m_run, tile_max) : m_run;
-            const float alpha = fresh ? 1.0f : __expf(m_run - m_new);
-            float sum = 0.0f;
-            half8_t p8;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const float pe = exp_weight(sc[e], m_new);
-                p8[e] = (half_t)pe;
-                sum += pe;
-            }
-            sum = column_reduce(sum, [](float a, float b) { return a + b; });
-            d_run = d_run * alpha + sum;
-            m_run = m_new;
+            scores(k_tile + cur, acc0, acc1, [&](int b) {
+                static_assert(2 * CPW == KS / 2, "a row a batch");
+                if (b < CPW) copy_row(k_rsrc, k_tile + other, t0 + kPrefillKeys, b, lane16);
+                else copy_row(v_rsrc, v_tile + other, t0 + kPrefillKeys, b - CPW, lane16);
+            });
+            float alpha; half8_t p8;
+            softmax_step(acc0, acc1, t0, quad, first_col, last_col, s.scale * kLog2e, m_run, d_run, alpha, p8);
             asm volatile("ds_write_b128 %0, %1" ::"v"(p_tile + (uint32_t)wave * 1024u), "v"(p8) : "memory");
             lane16 = p_tile - p_base;
             asm volatile("" : "+v"(lane16));
@@ -816,6 +823,7 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
 
     // the columns' denominators (or the states' m and d) from the waves that kept them; a wave's elements of all columns from itself
     __syncthreads();
+    d_run = column_reduce(d_run, [](float a, float b) { return a + b; });
     if (quad == 0) {
         if (num_chunks == 1u) {
             col_lds[wave * kTileHeads + col] = d_run > 0.0f ? 1.0f / d_run : 0.0f;      // zero where the column saw no key
@@ -866,7 +874,7 @@ inline float attn_us(const AttnCost &c, uint32_t blocks, uint32_t chunks, uint32
     return c.start + c.tile * (float)(goes * tiles) + (chunks > 1 ? c.merge + c.thousand_states * 1e-3f * (float)states : 0.0f);
 }
 
-// merge of the chunks' partial states of one (query, head) column: out = sum_c w_c o_c / sum_c w_c d_c, w_c = exp(m_c - max m);
+// merge of the chunks' partial states of one (query, head) column: out = sum_c w_c o_c / sum_c w_c d_c, w_c = 2^(m_c - max m);
 // chunks are added in ascending order; a chunk that saw no key has weight zero and its o is not read
 __global__ __launch_bounds__(128) void attention_prefill_combine_kernel(const float *m_part, const float *d_part, const float *o_part, half_t *O,
                                                                         uint32_t head_dim, uint32_t num_chunks, uint32_t num_q_heads,
@@ -877,7 +885,7 @@ __global__ __launch_bounds__(128) void attention_prefill_combine_kernel(const fl
     for (uint32_t c = 0; c < num_chunks; ++c) m_max = fmaxf(m_max, m_row[c]);
 #pragma unroll
     for (uint32_t c = 0; c < kMaxPrefillChunks; ++c) {
-        w[c] = c < num_chunks ? exp_weight(m_row[c], m_max) : 0.0f;
+        w[c] = c < num_chunks && m_row[c] != -INFINITY ? __builtin_amdgcn_exp2f(m_row[c] - m_max) : 0.0f;      // maxima in units of log2
         if (c < num_chunks) den += d_row[c] * w[c];
     }
     const float inv = den > 0.0f ? 1.0f / den : 0.0f;
