@@ -193,3 +193,46 @@ def test_keys_are_cut_into_chunks_where_the_merge_is_worth_it(start, count, hd, 
     assert launches_of(kk, lambda stream: kk.lib.tf_prefill_attention_causal(kk.handle, stream, q.data_ptr(), 0, k.data_ptr(), 0, v.data_ptr(), 0, out.data_ptr(),
                                                                              0, C.byref(p), 0)) == launches
     kk.close()
+
+
+@pytest.mark.parametrize("start,count,window,hd,hq,hkv", [
+    (0, 33, 0, 64, 4, 4),            # one key seen by the first column, the second tile masked but for one
+    (300, 31, 0, 128, 8, 2),
+    (700, 65, 300, 256, 4, 2),       # a window: tiles masked at both ends
+    (400, 37, 0, 512, 16, 2),        # head_dim 512, blocks of 64 columns
+    (1500, 500, 0, 512, 16, 2),      # ... and of 128
+])
+def test_scores_that_rise_and_fall_along_the_keys(start, count, window, hd, hq, hkv):
+    # Planted keys lift one query's score within the slack the reference maximum leaves (5, 7), over it (12, 25, 60) and leave the later keys
+    # far below (40 in the first tile), so that of a wave's columns, and of a column's four lanes, one alone asks for the rescale.
+    import ctypes as C
+    import torch
+    n, scale = start + count, hd ** -0.5
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(n + hd)
+    q, k, v = (torch.randn(rows, heads, hd, device="cuda", generator=gen).half() for rows, heads in ((count, hq), (n, hkv), (n, hkv)))
+    last = count - 1
+    lo = max(0, n - window) if window else 0
+    for g in range(hkv):
+        h = g * (hq // hkv) + g % (hq // hkv)
+        for t, at, score in ((last, lo + 3, 5.0), (last, lo + 7, 7.0), (last, (lo + n) // 2, 12.0), (last, (lo + n) // 2 + 9, 25.0), (last, n - 1, 60.0),
+                             (last // 2, lo + 1, 40.0)):
+            row = q[t, h].float()
+            k[at, g] = (row * (score / (scale * row.square().sum()))).half()
+    out = torch.full((count, hq, hd), float("nan"), device="cuda", dtype=torch.float16)
+    kk = ctx()
+    kk.reserve(max_q_heads=hq, max_attention_block_tokens=count)
+    p = tfk.PrefillAttentionParams(start, count, hd, hq, hkv, n, window, hkv * hd, hq * hd, hq * hd, scale)
+    kk.check(kk.lib.tf_prefill_attention_causal(kk.handle, None, q.data_ptr(), 0, k.data_ptr(), 0, v.data_ptr(), 0, out.data_ptr(), 0, C.byref(p), 0))
+    torch.cuda.synchronize()
+    pos, row = torch.arange(n, device="cuda")[None, :], torch.arange(start, n, device="cuda")[:, None]
+    hidden = (pos > row) | ((pos <= row - window) if window else torch.zeros_like(pos > row))
+    for h in range(hq):
+        g = h // (hq // hkv)
+        scores = (q[:, h].double() @ k[:, g].double().T.contiguous()) * scale
+        weights, values = torch.softmax(scores.masked_fill(hidden, float("-inf")), 1), v[:, g].double()
+        want, spread = weights @ values, weights @ values.abs()
+        # A weight is rounded to fp16 (2^-11 of it, or 2^-25 where it is subnormal, of a denominator of at least one) and so is the result.  A score
+        # is a 32-bit sum of hd products, converted to log2 units: at most 64 of its own roundings, of a score up to 64, on either side of the quotient.
+        bound = 2.0 ** -11 * (spread + want.abs()) + n * 2.0 ** -25 * values.abs().max() + 2 * 64 * 64 * 2.0 ** -24 * spread + 2.0 ** -24
+        assert torch.all((out[:, h].double() - want).abs() <= bound), h

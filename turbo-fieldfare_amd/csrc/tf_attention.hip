@@ -370,7 +370,9 @@ __device__ __forceinline__ float column_reduce(float v, Op op) {
 // The reference maximum of a column only moves when a score exceeds it by more than kMaxSlack2 (probabilities then reach at most 2^kMaxSlack2,
 // far inside fp16): in most steps no lane's own largest score does, and the column's maximum is not even formed.  d_run is the lane's
 // share of the denominator; the four lanes of a column are added up at the end.  Masks only where a column of the wave does not see the whole
-// tile.  About 45 instructions where forming the maximum and the sum in every step and masking every score took 147.
+// tile.  51 vector instructions in a step without masks or rescale; with the maximum and the sum formed and every score masked in every step it
+// took 102 and 21 scalar ones after the last product alone.  With the copies beside the products (below): head_dim 512, 128 queries over 32768 keys
+// 230 -> 205 us, 2048 at 0 168 -> 137; head_dim 256, window 1024, 2048 at 0 67.5 -> 59.
 constexpr float kLog2e = 1.4426950408889634f, kMaxSlack2 = 11.5f;
 __device__ __forceinline__ void softmax_step(const float4_t acc0, const float4_t acc1, uint32_t t0, int quad, uint32_t first_col, uint32_t last_col, float scale2, float &m_run,
                                              float &d_run, float &alpha, half8_t &p8) {
@@ -862,7 +864,8 @@ __global__ __launch_bounds__(64 * kWideWaves, 2) void attention_prefill_wide_ker
 }
 
 // What a block attention call takes, in microseconds, fitted to 16 / 8, 16 / 2, 16 / 1, 8 / 8, 8 / 1 and 4 / 4 heads, 1 to 2048 queries over 256
-// to 18000 keys (7 % off on average): start-up, 32 keys of the longest walk, the merge's launch, and a thousand partial states written and merged.
+// to 18000 keys (7 % off on average; steps have become up to 15 % cheaper since,
+// but prices scaled down by 12 % changed none of 16 timed shapes): start-up, 32 keys of the longest walk, the merge's launch, and a thousand partial states written and merged.
 struct AttnCost {
     float start, tile, merge, thousand_states;
 };
@@ -1136,8 +1139,8 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
             if (rc != TF_OK) return rc;
         }
         // head_dim 512: the wide kernel where the model prices it lower.  Both kernels have one block on a compute unit, so the wide one wins wherever
-        // its blocks, half as many a chunk, still fill the chip: 128 queries over 32768 keys (256 blocks either way) 310 -> 218 us, 500 over
-        // 2000 120 -> 81, 160 over 24160 493 -> 205; but 77 over 3077 (120 blocks for 240) 44 -> 48 and 128 over 768 (48 for 96) 37 -> 43.
+        // its blocks, half as many a chunk, still fill the chip: 128 queries over 32768 keys (256 blocks either way) 308 -> 203 us, 500 over
+        // 2000 119 -> 78, 160 over 24160 460 -> 178; but 77 over 3077 (120 blocks for 240) 44 -> 47 and 128 over 768 (48 for 96) 32 -> 39.
         bool wide = false;
         if (hd == 512) {
             const uint32_t wide_blocks = (s.count * group + kWideCols - 1) / kWideCols, wide_base = wide_blocks * s.num_kv_heads, cus = (uint32_t)ctx->num_cus;
@@ -1148,7 +1151,7 @@ int32_t tf_prefill_attention_causal(tf_ctx *ctx, tf_stream stream, const void *q
             auto us = [&](uint32_t c) { return attn_us(kWideCost, wide_base, c, span, states_of(c), cus); };
             for (uint32_t c = 2; c <= most && states_of(c) * (2 + (size_t)hd) * sizeof(float) <= ctx->attn_scratch_bytes; ++c)
                 if (us(c) < us(best)) best = c;
-            wide = us(best) < 0.97f * attn_us(cost, base, chunks, span, states_of(chunks), target);      // clearly: 1000 queries of 4 / 4 heads over 2000 keys 57 -> 60 at equal prices
+            wide = us(best) < 0.97f * attn_us(cost, base, chunks, span, states_of(chunks), target);      // clearly: 1000 queries of 4 / 4 heads over 2000 keys 58 -> 59 at equal prices
             if (wide) {
                 col_blocks = wide_blocks;
                 base = wide_base;
