@@ -4,6 +4,8 @@
 // equals its tokens done one by one, bit for bit.
 #include <math.h>
 
+#include <type_traits>
+
 #include "tf_common.hpp"
 #include "tf_context.hpp"
 #include "tf_epilogue_heads.hpp"
@@ -48,82 +50,101 @@ __global__ __launch_bounds__(256) void rope_neox_kernel(half_t *data, uint32_t p
 // of an element (NeoX pairing, head_dim / 2 away) sits 32 lanes further.  What bounds the step is the rotation angle - powf and
 // sincosf, some 200 instructions - not the bytes, and the angle depends on (token, pair) only: the block computes the token's
 // sines and cosines once, into LDS, for all of its heads (four at a time, heads_per_wave rounds).  With a block per head and an
-// angle per head the step took 91 us at 2048 tokens x 32 heads of 256; 18 us now (33.5 MB
-// read and written), and 15 -> 5 us at 500 tokens x 20 heads of 512.
-// grid (head groups, tokens).  VEC: every head starts at a multiple of its lanes' piece (16 bytes at most).  The arithmetic does
-// not depend on VEC or heads_per_wave: a block of tokens equals its tokens done one by one, bit for bit.
-template <int EPL, bool VEC>
+// angle per head the step took 91 us at 2048 tokens x 32 heads of 256 (33.5 MB read and written).
+// With eight heads a wave all waves of a call are resident at once and what is left is the issue of vector instructions, a hundred and eighty
+// a head: angles and weights read again for every head, partners fetched through LDS, a square root and a division in all lanes for one
+// number.  So a wave asks for all of its heads at the start, keeps both weights and its lanes' angles in registers, gets (x0, x1) from one
+// lane swap, and takes the square roots and divisions of all heads in one go, head r's in lane r.
+// 82 instructions a head.  2048 tokens x 32 heads of 256: 21.0 -> 15.6 us; 500 tokens: 10.1 -> 9.1; one token 3.4 -> 2.9; 20 heads of 512, 128
+// tokens: 5.4 -> 4.5 (kernel times under the profiler).
+// grid (head groups, tokens).  VEC: every head starts at a multiple of its lanes' piece (16 bytes at most).  HPW: heads a wave.  The arithmetic
+// does not depend on VEC or HPW: a block of tokens equals its tokens done one by one, bit for bit.
+template <int EPL, bool VEC, int HPW>
 __global__ __launch_bounds__(256) void qkv_epilogue_wave_kernel(half_t *q, half_t *k, half_t *v, const uint16_t *q_weight, const uint16_t *k_weight,
                                                                 uint32_t num_q_heads, uint32_t num_kv_heads, uint32_t position, float theta,
-                                                                uint32_t rotated_pairs, float eps, uint32_t q_token_stride, uint32_t kv_token_stride,
-                                                                uint32_t heads_per_wave) {
+                                                                uint32_t rotated_pairs, float eps, uint32_t q_token_stride, uint32_t kv_token_stride) {
     constexpr uint32_t kHeadDim = EPL * 64, kHalfDim = kHeadDim / 2;
     typedef half_t piece_t __attribute__((ext_vector_type(EPL)));
     __shared__ float cosine[kHalfDim], sine[kHalfDim];
-    const uint32_t t = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint32_t t = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const EpilogueHeads kinds = {num_q_heads, num_kv_heads};
-    const uint32_t heads = kinds.count(), head0 = blockIdx.x * 4 * heads_per_wave + wave;
+    const uint32_t heads = kinds.count(), head0 = blockIdx.x * 4 * HPW + wave;
     auto head_at = [&](uint32_t h) {
         return h < num_q_heads ? q + (size_t)t * q_token_stride + (size_t)h * kHeadDim
                : h < num_q_heads + num_kv_heads ? k + (size_t)t * kv_token_stride + (size_t)(h - num_q_heads) * kHeadDim
                                                 : v + (size_t)t * kv_token_stride + (size_t)(h - num_q_heads - num_kv_heads) * kHeadDim;
     };
-    auto load = [&](uint32_t h, float x[EPL]) {
-        const half_t *src = head_at(kinds.read(h)) + lane * EPL;
-        if constexpr (VEC) {
-            const piece_t p = *reinterpret_cast<const piece_t *>(src);
+    piece_t piece[HPW];
 #pragma unroll
-            for (int j = 0; j < EPL; ++j) x[j] = (float)p[j];
+    for (int r = 0; r < HPW; ++r) {
+        const half_t *src = head_at(kinds.read(head0 + 4 * r)) + lane * EPL;
+        if constexpr (VEC) {
+            piece[r] = *reinterpret_cast<const piece_t *>(src);
         } else {
 #pragma unroll
-            for (int j = 0; j < EPL; ++j) x[j] = (float)src[j];
+            for (int j = 0; j < EPL; ++j) piece[r][j] = src[j];
         }
-    };
-    auto load_weight = [&](uint32_t h, float wv[EPL]) {
-        const uint16_t *w = (kinds.takes_q_weight(h) ? q_weight : k_weight) + lane * EPL;
+    }
+    // the weights of the wave's first and of its last head: q heads come first, so there are no others
+    float first_w[EPL], last_w[EPL];
+    const bool first_q = kinds.takes_q_weight(head0), last_q = kinds.takes_q_weight(head0 + 4 * (HPW - 1));
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) wv[j] = bf16_to_f32(w[j]);
-    };
-    float x[EPL], wv[EPL];
-    load(head0, x);
-    load_weight(head0, wv);
+    for (int j = 0; j < EPL; ++j) {
+        first_w[j] = bf16_to_f32((first_q ? q_weight : k_weight)[lane * EPL + j]);
+        last_w[j] = HPW > 1 ? bf16_to_f32((last_q ? q_weight : k_weight)[lane * EPL + j]) : first_w[j];
+    }
     for (uint32_t pair = threadIdx.x; pair < rotated_pairs; pair += blockDim.x) {
         float sn, c;
         sincosf((float)(position + t) * rope_frequency(pair, kHeadDim, theta), &sn, &c);
         cosine[pair] = c;
         sine[pair] = sn;
     }
-    __syncthreads();
-    for (uint32_t round = 0; round < heads_per_wave; ++round) {
-        const uint32_t h = head0 + 4 * round;
-        if (h >= heads) break;
-        float next[EPL], next_w[EPL];
-        if (round + 1 < heads_per_wave) {
-            load(h + 4, next);
-            load_weight(h + 4, next_w);
-        }
+    // 1 / rms of head r
+    auto inverse = [&](float sum) { return 1.0f / sqrtf(sum / (float)kHeadDim + eps); };
+    float sums = 0.0f;
+#pragma unroll
+    for (int r = 0; r < HPW; ++r) {
         float acc = 0.0f;
 #pragma unroll
-        for (int j = 0; j < EPL; ++j) acc = fmaf(x[j], x[j], acc);
+        for (int j = 0; j < EPL; ++j) acc = fmaf((float)piece[r][j], (float)piece[r][j], acc);
         acc = wave_sum(acc);
-        const float inv = 1.0f / sqrtf(acc / (float)kHeadDim + eps);
-        const bool is_v = h >= num_q_heads + num_kv_heads;
+        sums = HPW == 1 ? acc : (int)lane == r ? acc : sums;
+    }
+    const float invs = inverse(sums);
+    __syncthreads();
+    // element j of a lane: x0 of its pair times x0_by[j] plus x1 times x1_by[j]
+    const bool is_x0 = lane < 32;
+    float x0_by[EPL], x1_by[EPL];
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) {
+        const uint32_t pair = (lane & 31) * EPL + j;
+        const float sn = sine[pair], c = cosine[pair];      // beyond rotated_pairs: never used
+        x0_by[j] = is_x0 ? c : sn;
+        x1_by[j] = is_x0 ? -sn : c;
+    }
+#pragma unroll
+    for (int r = 0; r < HPW; ++r) {
+        const uint32_t h = head0 + 4 * r;
+        if (h >= heads) break;
+        const float inv = HPW == 1 ? invs : __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(invs), r));
+        const bool is_v = h >= num_q_heads + num_kv_heads, use_first = kinds.takes_q_weight(h) == first_q;
         float out[EPL];
 #pragma unroll
         for (int j = 0; j < EPL; ++j) {
-            float xv = x[j] * inv;
-            if (!is_v) xv *= wv[j];
+            float xv = (float)piece[r][j] * inv;
+            if (!is_v) xv *= use_first ? first_w[j] : last_w[j];
             asm volatile("" : "+v"(xv));   // the fp32 product is rounded to half, not fused into the conversion
             out[j] = (float)(half_t)xv;
         }
         if (!is_v) {
 #pragma unroll
             for (int j = 0; j < EPL; ++j) {
-                const uint32_t pair = (lane & 31) * EPL + j;
-                const float other = __shfl_xor(out[j], 32, kWave);
-                float x0 = lane < 32 ? out[j] : other, x1 = lane < 32 ? other : out[j];
-                if (pair < rotated_pairs) rotate(x0, x1, sine[pair], cosine[pair]);
-                out[j] = lane < 32 ? x0 : x1;
+                const uint32_t own = __float_as_uint(out[j]);
+                const auto both = __builtin_amdgcn_permlane32_swap(own, own, false, false);      // lanes 0..31 twice, lanes 32..63 twice
+                const float x0 = __uint_as_float(both[0]), x1 = __uint_as_float(both[1]);
+                float turned = fmaf(x0, x0_by[j], x1 * x1_by[j]);
+                asm volatile("" : "+v"(turned));   // an fp32 value before it becomes a half, as above
+                out[j] = (lane & 31) * EPL + j < rotated_pairs ? turned : out[j];
             }
         }
         half_t *dst = head_at(h) + lane * EPL;
@@ -135,11 +156,6 @@ __global__ __launch_bounds__(256) void qkv_epilogue_wave_kernel(half_t *q, half_
         } else {
 #pragma unroll
             for (int j = 0; j < EPL; ++j) dst[j] = (half_t)out[j];
-        }
-#pragma unroll
-        for (int j = 0; j < EPL; ++j) {
-            x[j] = next[j];
-            wv[j] = next_w[j];
         }
     }
 }
@@ -224,15 +240,20 @@ int32_t launch_qkv_epilogue(tf_ctx *ctx, tf_stream stream, void *q, uint64_t q_o
         const dim3 grid((groups + 4 * per_wave - 1) / (4 * per_wave), tokens);
         const unsigned piece = head_dim / 64 * 2;
         const bool vec = aligned(qp, piece) && aligned(kp, piece) && aligned(vp, piece) && q_token_stride * 2 % piece == 0 && kv_token_stride * 2 % piece == 0;
-        auto launch = [&](auto kernel) {
-            hipLaunchKernelGGL(kernel, grid, dim3(256), 0, st, qp, kp, vp, qw, kw, num_q_heads, num_kv_heads, position, theta, rotated_pairs, eps,
-                               q_token_stride, kv_token_stride, per_wave);
+        auto launch = [&](auto epl, auto vectors) {
+            auto with = [&](auto heads) {
+                hipLaunchKernelGGL((qkv_epilogue_wave_kernel<decltype(epl)::value, decltype(vectors)::value, decltype(heads)::value>), grid, dim3(256), 0, st, qp, kp, vp, qw,
+                                   kw, num_q_heads, num_kv_heads, position, theta, rotated_pairs, eps, q_token_stride, kv_token_stride);
+            };
+            per_wave == 8 ? with(std::integral_constant<int, 8>{}) : per_wave == 4 ? with(std::integral_constant<int, 4>{})
+            : per_wave == 2 ? with(std::integral_constant<int, 2>{}) : with(std::integral_constant<int, 1>{});
         };
+        auto either = [&](auto epl) { vec ? launch(epl, std::true_type{}) : launch(epl, std::false_type{}); };
         switch (head_dim) {
-            case 64: launch(qkv_epilogue_wave_kernel<1, true>); break;
-            case 128: vec ? launch(qkv_epilogue_wave_kernel<2, true>) : launch(qkv_epilogue_wave_kernel<2, false>); break;
-            case 256: vec ? launch(qkv_epilogue_wave_kernel<4, true>) : launch(qkv_epilogue_wave_kernel<4, false>); break;
-            default: vec ? launch(qkv_epilogue_wave_kernel<8, true>) : launch(qkv_epilogue_wave_kernel<8, false>); break;
+            case 64: launch(std::integral_constant<int, 1>{}, std::true_type{}); break;
+            case 128: either(std::integral_constant<int, 2>{}); break;
+            case 256: either(std::integral_constant<int, 4>{}); break;
+            default: either(std::integral_constant<int, 8>{}); break;
         }
         return check_launch(ctx, who);
     }
