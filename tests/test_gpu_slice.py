@@ -1,0 +1,149 @@
+"""The slice kernels (routed experts and a shared expert's rows of blocks of up to 256 tokens) against 64-bit products, on numbers and through
+work lists that the ordinary cases do not reach."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import ctx, launches_of, tfk
+
+pytestmark = pytest.mark.gpu
+TOP_K = 8
+
+
+def affine(gen, rows, cols, fp16, size=1.0):
+    """Codes, scales and biases, and the exact weights in 64 bits: zero-mean groups, weights of about 0.06 `size`."""
+    W = torch.randint(0, 256, (rows, cols // 2), dtype=torch.uint8, device="cuda", generator=gen)
+    s = (torch.rand((rows, cols // 64), device="cuda", generator=gen) * 0.016 + 0.004) * size
+    b = s * -7.5 + (torch.rand(s.shape, device="cuda", generator=gen) - 0.5) * 0.02 * size
+    s, b = (t.to(torch.float16 if fp16 else torch.bfloat16) for t in (s, b))
+    q = torch.stack([W & 15, W >> 4], 2).reshape(rows, cols).double()
+    return (W, s, b), q * s.double().repeat_interleave(64, 1) + b.double().repeat_interleave(64, 1)
+
+
+def gelu(v):
+    return v / (1 + torch.exp(-2 * (0.7978845608028654 * (v + 0.044715 * v ** 3)).clamp(-20, 20)))
+
+
+def half(v):
+    return v.half().double()
+
+
+class Experts:
+    """A pool of experts, their exact weights, and a work list of `tokens` rows over them."""
+
+    def __init__(self, seed, tokens, experts, d, f, fp16=False, size=(1.0, 1.0), edit=None):
+        self.gen = gen = torch.Generator(device="cuda")
+        gen.manual_seed(seed)
+        self.tokens, self.experts, self.d, self.f, self.fp16, self.n = tokens, experts, d, f, fp16, tokens * TOP_K
+        mats = [[affine(gen, *shape, fp16, s) for shape, s in (((f, d), size[0]), ((f, d), size[0]), ((d, f), size[1]))] for _ in range(experts)]
+        if edit:
+            edit(mats)
+        self.weights = [[m[1] for m in e] for e in mats]
+        offsets, at = [], 0
+        for t in (t for m in mats[0] for t in m[0]):
+            offsets.append(at)
+            at = (at + t.numel() * t.element_size() + 15) // 16 * 16
+        self.off, self.stride = tfk.ExpertOffsets(*offsets), (at + 255) // 256 * 256
+        self.pool = torch.zeros((experts, self.stride), dtype=torch.uint8, device="cuda")
+        for row, e in zip(self.pool, mats):
+            for o, t in zip(offsets, (t for m in e for t in m[0])):
+                raw = t.contiguous().view(torch.uint8).ravel()
+                row[o:o + raw.numel()] = raw
+        self.idx = torch.rand((tokens, experts), device="cuda", generator=gen).add(torch.linspace(1, 0, experts, device="cuda") ** 4).topk(TOP_K).indices.int().contiguous()
+        self.wts = torch.rand((tokens, TOP_K), device="cuda", generator=gen).half()
+        i32 = dict(dtype=torch.int32, device="cuda")
+        self.capacity = experts + self.n // 128 + 1
+        self.pairs, self.count = torch.zeros((self.n, 4), **i32), torch.zeros(1, **i32)
+        self.chunks = torch.zeros((self.capacity, 3), **i32)
+        offs, counts = torch.zeros(experts, **i32), torch.zeros(experts, **i32)
+        k = ctx()
+        k.check(k.lib.tf_prefill_group_pairs_device(k.handle, None, self.idx.data_ptr(), self.wts.data_ptr(), tokens, TOP_K, experts, self.pairs.data_ptr(),
+                                                    offs.data_ptr(), counts.data_ptr(), self.chunks.data_ptr(), self.count.data_ptr()))
+        torch.cuda.synchronize()
+
+    def run(self, x, stride=None, pairs=None, chunks=None, count=None, capacity=None, pair_count=None):
+        n = pair_count or self.n
+        acts, partials = torch.zeros((n, self.f), dtype=torch.float16, device="cuda"), torch.zeros((self.n, self.d), dtype=torch.float16, device="cuda")
+        pairs, chunks, count = (self.pairs if pairs is None else pairs), (self.chunks if chunks is None else chunks), (self.count if count is None else count)
+        k = ctx()
+        k.check(k.lib.tf_prefill_grouped_routed_moe_resident(k.handle, None, x.data_ptr(), 0, stride or self.d, pairs.data_ptr(), chunks.data_ptr(), count.data_ptr(),
+                                                             capacity or self.capacity, n, self.pool.data_ptr(), self.stride, self.experts, C.byref(self.off),
+                                                             acts.data_ptr(), partials.data_ptr(), self.d, self.f, TOP_K, tfk.TF_FP16 if self.fp16 else tfk.TF_BF16))
+        torch.cuda.synchronize()
+        return acts, partials.view(self.tokens, TOP_K, self.d)
+
+    def exact_acts(self, x):
+        """What the gate / up launch is to leave, pair by pair, before its rounding."""
+        out = torch.empty((self.n, self.f), dtype=torch.float64, device="cuda")
+        for e in range(self.experts):
+            rows = (self.pairs[:, 1] == e).nonzero().ravel()
+            if rows.numel():
+                v = x[self.pairs[rows, 0].long()].double()
+                out[rows] = gelu(v @ self.weights[e][0].T.contiguous()) * (v @ self.weights[e][1].T.contiguous())
+        return out
+
+    def exact_partials(self, acts):
+        """What the down launch is to leave for these activations."""
+        out = torch.empty((self.tokens, TOP_K, self.d), dtype=torch.float64, device="cuda")
+        for e in range(self.experts):
+            rows = (self.pairs[:, 1] == e).nonzero().ravel()
+            if rows.numel():
+                out[self.pairs[rows, 0].long(), self.pairs[rows, 2].long()] = acts[rows].double() @ self.weights[e][2].T.contiguous()
+        return out
+
+
+def check_rounded(got, want):
+    # Rounding to fp16 is off by 2^-11 of a value at most, or by 2^-25 where it is subnormal.  The sums before it, of nibbles that the matrix unit
+    # reads as fp16 subnormals, have a deviation of 2e-6 to 7e-6 of the outputs' norm (measured against 64-bit sums, at outputs near zero); the largest of
+    # some hundred thousand is 3e-5 off, a half of what is allowed here.  An operand rounded to the step of a subnormal number costs 3e-4 and more.
+    off, rms = (got.double() - want).abs(), float(want.norm()) / want.numel() ** 0.5
+    bound = want.abs() * 2.0 ** -11 + 2.0 ** -25 + 4 * 2.0 ** -16 * rms
+    assert torch.all(off <= bound), float((off / bound).max())
+
+
+@pytest.mark.parametrize("size", [1e-3, 1e-4, 1e-5])
+@pytest.mark.parametrize("tokens,experts,d,f,fp16", [(80, 8, 1344, 320, False), (24, 48, 1280, 704, True)])
+def test_small_activations_keep_their_bits(tokens, experts, d, f, fp16, size):
+    # Rows of 1e-3 to 1e-5, most of whose numbers are below fp16's normal range (6e-5) or would be after a division by sixteen; weights so
+    # large that the results are of ordinary size.
+    e = Experts(0x51CE + tokens, tokens, experts, d, f, fp16, size=(0.3 / size, 1.0))
+    x = (torch.randn((tokens, d), device="cuda", generator=e.gen) * size).half()
+    acts, _ = e.run(x)
+    check_rounded(acts, e.exact_acts(x))
+    e = Experts(0x52CE + tokens, tokens, experts, d, f, fp16, size=((size / 4) ** 0.5, 0.3 / size))       # activations of about `size`
+    x = torch.randn((tokens, d), device="cuda", generator=e.gen).half()
+    acts, partials = e.run(x)
+    assert 0.1 * size < float(acts.double().norm() / acts.numel() ** 0.5) < 10 * size
+    check_rounded(partials, e.exact_partials(acts))
+
+
+def shared_block(x, mats, d, f, fp16, x_stride=None):
+    k, rows = ctx(), x.shape[0]
+    y = torch.full((rows, d), float("nan"), dtype=torch.float16, device="cuda")
+    scratch = torch.zeros(f, dtype=torch.float16, device="cuda")
+    gate, up, down = (tfk.projection(*m[0], r, c) for m, (r, c) in zip(mats, ((f, d), (f, d), (d, f))))
+    k.check(k.lib.tf_prefill_shared_expert_int4_block(k.handle, None, x.data_ptr(), 0, y.data_ptr(), 0, C.byref(gate), C.byref(up), C.byref(down),
+                                                      *(v for _ in range(3) for v in (scratch.data_ptr(), 0, f * 2)), rows, d, f, x_stride or d, d, 4,
+                                                      tfk.TF_FP16 if fp16 else tfk.TF_BF16))
+    torch.cuda.synchronize()
+    return y
+
+
+@pytest.mark.parametrize("size", [1e-3, 1e-4, 1e-5])
+@pytest.mark.parametrize("stage", ["gate / up", "down"])
+@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (256, 1280, 704, True)])
+def test_shared_expert_keeps_the_bits_of_small_activations(rows, d, f, fp16, stage, size):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + d)
+    first, last = (0.3 / size, 1.0) if stage == "gate / up" else ((size / 4) ** 0.5, 0.3 / size)
+    mats = [affine(gen, *shape, fp16, s) for shape, s in (((f, d), first), ((f, d), first), ((d, f), last))]
+    x = (torch.randn((rows, d), device="cuda", generator=gen) * (size if stage == "gate / up" else 1.0)).half()
+    y = shared_block(x, mats, d, f, fp16)
+    # the stage boundary: gate, up and their product leave as fp16
+    product = lambda a, m: a @ m[1].T.contiguous()
+    want = product(half(gelu(half(product(x.double(), mats[0]))) * half(product(x.double(), mats[1]))), mats[2])
+    # besides the last rounding one activation in some hundred may be a rounding step off (its gate, its up or itself): one percent of 2^-10 or so
+    # of the sums
+    assert float((y.double() - want).norm() / want.norm()) < 3.5e-4

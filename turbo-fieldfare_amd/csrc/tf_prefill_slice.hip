@@ -13,10 +13,13 @@ namespace {
 // the A operands of v_mfma_f32_32x32x16_f16, for as long as its block works on these pairs.  Weight rows pass by it, 32 at a time: 128
 // bytes of each, the lines that its slice covers, come through a wave-private ring in LDS (two tiles deep, copied by the load unit: nothing but
 // whole 128-byte lines is asked for, and no register waits for memory), and nibbles masked out of the words are the B operand as they are:
-// read as fp16 subnormals they are exactly q 2^-24.  A group's four instructions start from zero; their sums are then multiplied by the
+// read as fp16 subnormals they are exactly q 2^-24.  (Every word is shifted for each of its four masks.  With two masks fewer shifts, 16 q against
+// activations of a sixteenth, activations below 2^-10 lose up to four bits: at 1e-4 0.6 % of the result.  The shifts cost 1 %: both launches of 128 / 256
+// tokens 110.6 / 120.8 -> 111.7 / 121.3 us.)  A group's four instructions start from zero; their sums are then multiplied by the
 // row's scale in fp32, and the bias terms of a slice are one more instruction: bias times the sums of the activations, those split into three
-// bf16 parts, exact.  So a weight is q s + b in 32 bits, as in the quad kernels, and a 32 x 64 piece of weights costs 20 + NR vector
-// instructions against the 64 that rounding it to fp16 takes in the tile kernels.
+// bf16 parts, exact.  So a weight is q s + b in 32 bits, as in the quad kernels, and a 32 x 64 piece of weights costs 28 + NR vector
+// instructions against the 64 that rounding it to fp16 takes in the tile kernels.  The sums of subnormal operands come out with
+// an error of 2e-6 to 7e-6 of the outputs' norm (against 64-bit sums; those of the quad kernels likewise).
 //
 // A row's slices lie with different waves: SLICES of them (11 at 2816 columns) share a tile, their sums meet in LDS and are added in slice
 // order; with few slices (3 at 704 columns) a block holds several such groups of waves, each on tiles of its own.  One block of up to twelve
@@ -130,8 +133,7 @@ __device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][
         for (int d = 0; d < 4; ++d) {
             uint32_t word = w[g][d];
             asm volatile("" : "+v"(word));       // the operands are made here, word by word: all of a tile's at once would not fit the registers
-            const uint32_t high = word >> 8;
-            const u32x4 q = {word & 0x000F000Fu, word & 0x00F000F0u, high & 0x000F000Fu, high & 0x00F000F0u};
+            const u32x4 q = {word & 0x000F000Fu, word >> 4 & 0x000F000Fu, word >> 8 & 0x000F000Fu, word >> 12 & 0x000F000Fu};
             c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[g][d], __builtin_bit_cast(half8_t, q), c, 0, 0, 0);
         }
         const uint32_t sv = s[g >> 1];
@@ -455,8 +457,7 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
             uint32_t part[3][kSliceGroups];
 #pragma unroll
             for (int g = 0; g < kSliceGroups; ++g) {
-                // a group's 32 values of this lane in the order the nibble masks give: (0, 4), (1, 5) / 16, (2, 6), (3, 7) / 16 of every eight
-                const half2_t sixteenth = {(half_t)0.0625f, (half_t)0.0625f};
+                // a group's 32 values of this lane in the order the nibble masks give: (0, 4), (1, 5), (2, 6), (3, 7) of every eight
                 const bool mine = g >= skip;
                 float16_t total;
 #pragma unroll
@@ -464,12 +465,8 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
 #pragma unroll
                 for (int d = 0; d < 4; ++d) {
                     const u32x4 v = mine ? raw[g][d] : u32x4{0u, 0u, 0u, 0u};
-                    u32x4 o;
-                    o[0] = __builtin_amdgcn_perm(v[2], v[0], 0x05040100u);
-                    o[1] = as_u32(as_half2(__builtin_amdgcn_perm(v[2], v[0], 0x07060302u)) * sixteenth);
-                    o[2] = __builtin_amdgcn_perm(v[3], v[1], 0x05040100u);
-                    o[3] = as_u32(as_half2(__builtin_amdgcn_perm(v[3], v[1], 0x07060302u)) * sixteenth);
-                    x[g][d] = __builtin_bit_cast(half8_t, o);
+                    x[g][d] = __builtin_bit_cast(half8_t, u32x4{__builtin_amdgcn_perm(v[2], v[0], 0x05040100u), __builtin_amdgcn_perm(v[2], v[0], 0x07060302u),
+                                                                __builtin_amdgcn_perm(v[3], v[1], 0x05040100u), __builtin_amdgcn_perm(v[3], v[1], 0x07060302u)});
                     // the sum of all 64 values of the lane's pair: the values as they came against ones, the same in all sixteen rows
                     const half_t one = (half_t)1.0f;
                     total = __builtin_amdgcn_mfma_f32_32x32x16_f16(half8_t{one, one, one, one, one, one, one, one}, __builtin_bit_cast(half8_t, v), total, 0, 0, 0);
