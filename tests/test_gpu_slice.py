@@ -147,3 +147,62 @@ def test_shared_expert_keeps_the_bits_of_small_activations(rows, d, f, fp16, sta
     # besides the last rounding one activation in some hundred may be a rounding step off (its gate, its up or itself): one percent of 2^-10 or so
     # of the sums
     assert float((y.double() - want).norm() / want.norm()) < 3.5e-4
+
+
+def cut(pairs, run, empty_every=0):
+    """The pairs' work list in runs of at most `run`, a chunk without pairs behind every `empty_every`-th."""
+    expert, chunks, at = pairs[:, 1].tolist(), [], 0
+    while at < len(expert):
+        end = at
+        while end < len(expert) and end - at < run and expert[end] == expert[at]:
+            end += 1
+        chunks.append((expert[at], at, end - at))
+        at = end
+        if empty_every and len(chunks) % empty_every == 0:
+            chunks.append((3, at, 0))
+    return chunks
+
+
+@pytest.mark.parametrize("tokens,experts,d,f", [(24, 48, 1344, 320), (110, 16, 1280, 704)])
+def test_results_do_not_depend_on_the_work_list(tokens, experts, d, f):
+    # The kernels hold 256 chunks of a list at a time.  Lists of more room than they fill, of more than 256 chunks, of chunks without pairs in front, between
+    # and behind: the same bits.
+    e = Experts(0x53CE + tokens, tokens, experts, d, f)
+    x = torch.randn((tokens, d), device="cuda", generator=e.gen).half()
+    acts, partials = e.run(x)
+    lists = [(cut(e.pairs, 128), 0), (cut(e.pairs, 128), 1000), (cut(e.pairs, 1), 0), (cut(e.pairs, 3, 2), 40), ([(1, 0, 0)] * 300 + cut(e.pairs, 40, 3) + [(2, 0, 0)] * 300, 0),
+             (cut(e.pairs, 5) + [(0, 0, 0)] * 256, 1)]
+    for chunks, room in lists:
+        table = torch.full((len(chunks) + room, 3), 0x7FFFFFFF, dtype=torch.int32, device="cuda")      # what lies behind the list is never used
+        table[:len(chunks)] = torch.tensor(chunks, dtype=torch.int32)
+        got_acts, got = e.run(x, chunks=table, count=torch.tensor([len(chunks)], dtype=torch.int32, device="cuda"), capacity=len(chunks) + room)
+        assert torch.equal(got_acts, acts) and torch.equal(got, partials), (len(chunks), room)
+    check_rounded(acts, e.exact_acts(x))
+
+
+@pytest.mark.parametrize("tokens,experts", [(24, 48), (32, 64), (32, 85)])
+def test_few_tokens_are_their_three_calls(tokens, experts):
+    e = Experts(0x54CE + tokens, tokens, experts, 1280, 256)
+    gen, d = e.gen, e.d
+    W, s, b = torch.randint(0, 256, (experts, d), dtype=torch.uint8, device="cuda", generator=gen), *(
+        (torch.rand((experts, d // 64), device="cuda", generator=gen) * 0.02 * m).bfloat16() for m in (1, -127.5))
+    eff, gain = torch.full((d,), d ** -0.5, device="cuda").bfloat16(), torch.ones(experts, device="cuda").bfloat16()
+    x = torch.randn((tokens, d), device="cuda", generator=gen).half()
+    i32, f16 = dict(dtype=torch.int32, device="cuda"), dict(dtype=torch.float16, device="cuda")
+    router = [v for t in (W, s, b, x, eff, gain) for v in (t.data_ptr(), 0)]
+    k, out = ctx(), []
+    for one_call in (False, True):
+        idx, wts, h2 = torch.zeros((tokens, TOP_K), **i32), torch.zeros((tokens, TOP_K), **f16), torch.zeros((tokens, d), **f16)
+        acts, partials = torch.zeros((e.n, e.f), **f16), torch.zeros((e.n, d), **f16)
+        head = (k.handle, None, *router, idx.data_ptr(), 0, wts.data_ptr(), 0, tokens, experts, d, TOP_K, d)
+        if one_call:
+            k.check(k.lib.tf_prefill_routed_moe_few_tokens(*head, x.data_ptr(), 0, d, e.pool.data_ptr(), e.stride, C.byref(e.off), acts.data_ptr(), partials.data_ptr(),
+                                                           h2.data_ptr(), 0, e.f, tfk.TF_BF16))
+        else:
+            offs, counts = torch.zeros(experts, **i32), torch.zeros(experts, **i32)
+            k.check(k.lib.tf_prefill_router_group_block(*head, e.pairs.data_ptr(), offs.data_ptr(), counts.data_ptr(), e.chunks.data_ptr(), e.count.data_ptr()))
+            acts, partials = e.run(x)
+            k.check(k.lib.tf_prefill_moe_reduce_token_major(k.handle, None, partials.data_ptr(), 0, wts.data_ptr(), 0, h2.data_ptr(), 0, tokens, TOP_K, d))
+        torch.cuda.synchronize()
+        out.append([t.reshape(-1) for t in (idx, wts, acts, partials, h2)])
+    assert all(torch.equal(a, b) for a, b in zip(*out))

@@ -831,7 +831,7 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     const uint64_t experts = tab.num_experts;
     const bool tiles_carry_shared = stream_tokens > kSliceRideless && stream_tokens <= kSharedSplitMaxRows && stream_pairs >= 5 * experts;
     if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens <= kSharedSliceMaxRows && !tiles_carry_shared &&
-        grouped_slice_ok(tab, cl, n_chunks_upper, stream_pairs, g.d, g.f)) {
+        grouped_slice_ok(tab, cl, stream_pairs, g.d, g.f)) {
         if (ride && !ride->slice) ride = nullptr;
         if (ride && ride_taken) *ride_taken = true;
         return launch_grouped_slice(ctx, st, tab, off, cl, n_chunks_upper, g, sd, ride);

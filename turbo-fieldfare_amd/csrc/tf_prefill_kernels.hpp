@@ -92,7 +92,7 @@ int32_t launch_grouped_quad(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab,
                             uint32_t n_chunks_upper, const GroupedGeom &g, tf_dtype sd, uint32_t stream_pairs);
 
 // The slice kernels (tf_prefill_slice.hip): the same stages for chunks of a few dozen pairs, activations in registers.
-bool grouped_slice_ok(const ExpertTable &tab, const ChunkList &cl, uint32_t n_chunks_upper, uint32_t pair_count, int d, int f);
+bool grouped_slice_ok(const ExpertTable &tab, const ChunkList &cl, uint32_t pair_count, int d, int f);
 int32_t launch_grouped_slice(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const tf_expert_offsets &off, const ChunkList &cl,
                              uint32_t n_chunks_upper, const GroupedGeom &g, tf_dtype sd, const DenseRide *ride);
 // and a shared expert's block of rows, in launches of its own or (ride above) beside the routed pairs

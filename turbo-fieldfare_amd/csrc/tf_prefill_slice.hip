@@ -40,7 +40,7 @@ constexpr uint32_t kSliceWBytes = 32 * 128;      // one wave's weights of a tile
 constexpr uint32_t kSliceSlot = kSliceWBytes + 512;      // and its scales and biases, eight bytes a row each
 constexpr int kSliceCopies = 6;                  // requests a tile
 constexpr uint32_t kSliceSums = 64 * 16 * 4;     // one wave's sums of a tile; half of it twice where they fit in half
-constexpr int kSliceListRounds = 4;              // the work list is looked at 64 chunks at a time: at most 256
+constexpr int kSliceListRounds = 4;              // the work list is looked at 64 chunks at a time, four times 64 in one trip to memory; the table holds as many
 constexpr uint32_t kSliceList = 64 * kSliceListRounds;
 constexpr uint32_t kSliceRing = 0, kSliceSumsAt = kSliceMaxWaves * 2 * kSliceSlot, kSliceTableAt = kSliceSumsAt + kSliceMaxWaves * kSliceSums,
                    kSliceRowsAt = kSliceTableAt + 3 * 4 * kSliceList, kSlicePairsAt = kSliceRowsAt + 4 * kSliceBatch, kSliceLds = kSlicePairsAt + 16 * kSliceBatch;
@@ -143,7 +143,10 @@ __device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][
     }
 }
 
-template <bool GATE_UP, int SD>
+// LONG: the work list has room for more chunks than the table.  A share of such a list is found by a walk over it, and chunks beyond the table come from
+// memory.  Which of the two it is never shows in the results; both launches of 128 tokens (128 experts) 118 / 111 us and, from a list with room for 400 chunks
+// that has no more than the other, 119 / 111; of 80 tokens 104 / 108.
+template <bool GATE_UP, int SD, bool LONG>
 __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(SliceArgs a) {
     constexpr int kRows = GATE_UP ? 16 : 32;           // output columns of a tile: 16 of gate with the same 16 of up, or 32
     __shared__ __align__(128) uint8_t lds_area[kSliceLds];
@@ -155,19 +158,30 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
     // ---- the work list: for every chunk the cost of those before it, where its pairs start, its expert and how many pairs it has
     uint32_t n_chunks = 0u, cost = 0u;                 // cost: of all units
     const uint32_t routed_positions = a.list_cap != 0u ? positions_of(a.routed) : 0u;
-    tf_prefill_group mine[kSliceListRounds];
-    if (a.list_cap != 0u) {
+    tf_prefill_group mine[kSliceListRounds];           // a lane's of the kSliceList chunks in hand
+    uint32_t through[kSliceListRounds], own_cost[kSliceListRounds];
+    auto take_chunks = [&](uint32_t from) {
 #pragma unroll
-        for (int r = 0; r < kSliceListRounds; ++r) mine[r] = a.list[min(64u * r + (uint32_t)lane, a.list_cap - 1u)];      // no branch: one trip to memory
+        for (int r = 0; r < kSliceListRounds; ++r) mine[r] = a.list[min(from + 64u * r + (uint32_t)lane, a.list_cap - 1u)];      // no branch: one trip to memory
+    };
+    auto add_costs = [&](uint32_t from) {
+#pragma unroll
+        for (int r = 0; r < kSliceListRounds; ++r) {
+            own_cost[r] = from + 64u * r + (uint32_t)lane < n_chunks ? slice_chunk_cost(mine[r].pair_count, routed_positions) : 0u;
+            through[r] = cost + slice_running_sum(own_cost[r]);
+            cost = (uint32_t)__builtin_amdgcn_readlane((int)through[r], 63);
+        }
+    };
+    if (a.list_cap != 0u) {
+        take_chunks(0u);
         n_chunks = uniform_u32(min(*a.list_count, a.list_cap));
     }
-    uint32_t through[kSliceListRounds], own_cost[kSliceListRounds];
-#pragma unroll
-    for (int r = 0; r < kSliceListRounds; ++r) {
-        own_cost[r] = 64u * r + (uint32_t)lane < n_chunks ? slice_chunk_cost(mine[r].pair_count, routed_positions) : 0u;
-        through[r] = cost + slice_running_sum(own_cost[r]);
-        cost = (uint32_t)__builtin_amdgcn_readlane((int)through[r], 63);
-    }
+    add_costs(0u);
+    if constexpr (LONG)
+        for (uint32_t from = kSliceList; from < n_chunks; from += kSliceList) {
+            take_chunks(from);
+            add_costs(from);
+        }
     // ---- the block's part: neighbours in the order of the work sit on one XCD, so that the units of a popular expert find its rows in one L2
     const uint32_t blocks = gridDim.x;
     uint32_t block = (blocks & 7u) == 0u ? (blockIdx.x & 7u) * (blocks >> 3) + (blockIdx.x >> 3) : blockIdx.x, of = blocks;
@@ -185,14 +199,55 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
     }
     const SliceProblem p = shared ? a.shared : a.routed;
     const uint32_t positions = positions_of(p);
+    struct Place {
+        uint32_t chunk, batch, tile;
+    };
+    // If the tile at which `spent` of all units' cost is behind belongs to one of 64 chunks, a lane each, from `base` on: into `at`
+    auto place_among = [&](uint32_t spent, uint32_t base, uint32_t cost_before, uint32_t chunk_pairs, Place &at) {
+        const uint64_t owners = __ballot(spent - cost_before < slice_chunk_cost(chunk_pairs, positions));      // wraps far beyond for a chunk that comes later
+        if (owners == 0ull) return false;
+        const int owner = (int)__builtin_ctzll(owners);
+        const uint32_t pairs = (uint32_t)__builtin_amdgcn_readlane((int)chunk_pairs, owner), whole = slice_unit_cost(kSliceBatch, positions);
+        uint32_t rest = spent - (uint32_t)__builtin_amdgcn_readlane((int)cost_before, owner);
+        at.chunk = base + (uint32_t)owner;
+        at.batch = min(rest / whole, (pairs - 1u) / kSliceBatch);
+        rest -= at.batch * whole;
+        at.tile = (rest > kSliceUnitCost ? rest - kSliceUnitCost : 0u) / slice_tile_cost(min(pairs - at.batch * kSliceBatch, kSliceBatch));
+        return true;
+    };
+    Place first, last;                                 // the block's first tile, and the one behind its last
+    uint32_t table_from = 0u;                          // the table holds the chunks from here on: all of them, or (LONG) those from the block's first on
+    auto share_at = [&](uint32_t i) { return (uint32_t)((uint64_t)cost * (block + i) / of); };
+    bool placed = false;
+    if constexpr (LONG)
+        if (n_chunks > kSliceList) {
+            const uint32_t from_cost = share_at(0u), to_cost = share_at(1u);
+            first = last = Place{n_chunks, 0u, 0u};
+            bool found_first = from_cost >= cost, found_last = to_cost >= cost;
+            cost = 0u;
+            for (uint32_t from = 0u; from < n_chunks && !(found_first && found_last); from += kSliceList) {
+                take_chunks(from);
+                add_costs(from);
+#pragma unroll
+                for (int r = 0; r < kSliceListRounds; ++r) {
+                    const uint32_t pairs = from + 64u * r + (uint32_t)lane < n_chunks ? mine[r].pair_count : 0u;
+                    if (!found_first) found_first = place_among(from_cost, from + 64u * r, through[r] - own_cost[r], pairs, first);
+                    if (!found_last) found_last = place_among(to_cost, from + 64u * r, through[r] - own_cost[r], pairs, last);
+                }
+            }
+            table_from = first.chunk;
+            take_chunks(table_from);
+            placed = true;
+        }
+    auto packed = [&](const tf_prefill_group &chunk) { return min(chunk.expert, a.num_experts - 1u) << 16 | chunk.pair_count; };
     if (wave == 0) {
 #pragma unroll
         for (int r = 0; r < kSliceListRounds; ++r) {
             const uint32_t entry = table + 4u * (64u * r + (uint32_t)lane);
-            const bool there = 64u * r + (uint32_t)lane < n_chunks;
-            lds_put4(entry, shared ? 0u : through[r] - own_cost[r]);
+            const bool there = table_from + 64u * r + (uint32_t)lane < n_chunks;
+            lds_put4(entry, shared ? 0u : through[r] - own_cost[r]);       // where all chunks are here
             lds_put4(entry + 4u * kSliceList, shared ? 0u : mine[r].pair_start);
-            lds_put4(entry + 8u * kSliceList, !there ? 0u : shared ? a.shared_rows : min(mine[r].expert, a.num_experts - 1u) << 16 | mine[r].pair_count);
+            lds_put4(entry + 8u * kSliceList, !there ? 0u : shared ? a.shared_rows : packed(mine[r]));
         }
     }
     slice_barrier();
@@ -211,8 +266,14 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
     };
     auto unit_of = [&](uint32_t chunk, uint32_t batch) {
         uint32_t start, what;
-        asm volatile("ds_read_b32 %0, %2 offset:%3\n\tds_read_b32 %1, %2 offset:%4\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(start), "=&v"(what) : "v"(table + 4u * min(chunk, kSliceList - 1u)), "n"(4 * kSliceList), "n"(8 * kSliceList) : "memory");
+        if (!LONG || chunk - table_from < kSliceList) {
+            asm volatile("ds_read_b32 %0, %2 offset:%3\n\tds_read_b32 %1, %2 offset:%4\n\ts_waitcnt lgkmcnt(0)"
+                         : "=&v"(start), "=&v"(what) : "v"(table + 4u * (chunk - table_from)), "n"(4 * kSliceList), "n"(8 * kSliceList) : "memory");
+        } else {                                           // a share of more than kSliceList chunks
+            const tf_prefill_group far = a.list[chunk];
+            start = far.pair_start;
+            what = packed(far);
+        }
         start = uniform_u32(start);
         what = uniform_u32(what);
         const uint32_t left = (what & 0xFFFFu) - batch * kSliceBatch, count = min(left, kSliceBatch);
@@ -228,32 +289,21 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
         }
         return Unit{n_chunks, 0u, 0u, 0u, 0u, 0u};
     };
-    struct Place {
-        uint32_t chunk, batch, tile;
-    };
-    // the tile at which `spent` of all units' cost is behind
-    auto place_of = [&](uint32_t spent) {
-        Place at = {n_chunks, 0u, 0u};
-        if (spent >= cost) return at;
-        for (uint32_t r = 0; 64u * r < n_chunks; ++r) {
-            uint32_t from, what;
-            asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
-                         : "=&v"(from), "=&v"(what) : "v"(table + 4u * (64u * r + (uint32_t)lane)), "n"(8 * kSliceList) : "memory");
-            const uint64_t owners = __ballot(spent - from < slice_chunk_cost(what & 0xFFFFu, positions));      // wraps far beyond for a chunk that comes later
-            if (owners != 0ull) {
-                const int owner = (int)__builtin_ctzll(owners);
-                const uint32_t pairs = (uint32_t)__builtin_amdgcn_readlane((int)what, owner) & 0xFFFFu, whole = slice_unit_cost(kSliceBatch, positions);
-                uint32_t rest = spent - (uint32_t)__builtin_amdgcn_readlane((int)from, owner);
-                at.chunk = 64u * r + (uint32_t)owner;
-                at.batch = min(rest / whole, (pairs - 1u) / kSliceBatch);
-                rest -= at.batch * whole;
-                at.tile = (rest > kSliceUnitCost ? rest - kSliceUnitCost : 0u) / slice_tile_cost(min(pairs - at.batch * kSliceBatch, kSliceBatch));
-                break;
+    if (!placed) {
+        auto place_of = [&](uint32_t spent) {
+            Place at = {n_chunks, 0u, 0u};
+            if (spent >= cost) return at;
+            for (uint32_t r = 0; 64u * r < n_chunks; ++r) {
+                uint32_t from, what;
+                asm volatile("ds_read_b32 %0, %2\n\tds_read_b32 %1, %2 offset:%3\n\ts_waitcnt lgkmcnt(0)"
+                             : "=&v"(from), "=&v"(what) : "v"(table + 4u * (64u * r + (uint32_t)lane)), "n"(8 * kSliceList) : "memory");
+                if (place_among(spent, 64u * r, from, what & 0xFFFFu, at)) break;
             }
-        }
-        return at;
-    };
-    const Place first = place_of((uint32_t)((uint64_t)cost * block / of)), last = place_of((uint32_t)((uint64_t)cost * (block + 1u) / of));      // last: the one behind
+            return at;
+        };
+        first = place_of(share_at(0u));
+        last = place_of(share_at(1u));
+    }
     if (first.chunk == last.chunk && first.batch == last.batch && first.tile == last.tile) return;
 
     // ---- requests of weights
@@ -556,16 +606,17 @@ void launch_slice(tf_ctx *ctx, hipStream_t st, const SliceArgs &a, tf_dtype sd) 
     // as many waves as the problems use: twelve, or fewer where their slices leave a remainder
     const int waves = std::max(a.list_cap ? a.routed.slices * a.routed.row_groups : 0, a.shared_rows ? a.shared.slices * a.shared.row_groups : 0);
     const dim3 grid((uint32_t)ctx->num_cus), block((uint32_t)(64 * waves));
-    if (sd == TF_BF16) hipLaunchKernelGGL((grouped_slice_kernel<GATE_UP, 0>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((grouped_slice_kernel<GATE_UP, 1>), grid, block, 0, st, a);
+    auto launch = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, a); };
+    if (a.list_cap > kSliceList) sd == TF_BF16 ? launch(grouped_slice_kernel<GATE_UP, 0, true>) : launch(grouped_slice_kernel<GATE_UP, 1, true>);
+    else sd == TF_BF16 ? launch(grouped_slice_kernel<GATE_UP, 0, false>) : launch(grouped_slice_kernel<GATE_UP, 1, false>);
 }
 
 }  // namespace
 
 namespace tfk {
 
-bool grouped_slice_ok(const ExpertTable &tab, const ChunkList &cl, uint32_t n_chunks_upper, uint32_t pair_count, int d, int f) {
-    return tab.pool != nullptr && cl.dev != nullptr && n_chunks_upper <= kSliceList && pair_count != 0 && pair_count < 65536 && tab.num_experts <= 65536 &&
+bool grouped_slice_ok(const ExpertTable &tab, const ChunkList &cl, uint32_t pair_count, int d, int f) {
+    return tab.pool != nullptr && cl.dev != nullptr && pair_count != 0 && pair_count < 65536 && tab.num_experts <= 65536 &&
            d >= kSliceMinCols && slice_width_ok(d) && slice_width_ok(f);
 }
 
