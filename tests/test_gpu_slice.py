@@ -206,3 +206,16 @@ def test_few_tokens_are_their_three_calls(tokens, experts):
         torch.cuda.synchronize()
         out.append([t.reshape(-1) for t in (idx, wts, acts, partials, h2)])
     assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
+def test_a_number_of_pairs_that_is_no_number_of_tokens_goes_to_the_tiles():
+    # 2396 pairs of top 8 are not those of a number of token rows: such a list may be of any length and goes, like the 300 rows it is taken from, to the tiles.
+    tokens, n = 300, 300 * TOP_K - 4
+    e = Experts(0x55CE, tokens, 16, 1280, 256)
+    x = torch.randn((tokens, e.d), device="cuda", generator=e.gen).half()
+    _, want = e.run(x)
+    chunks = torch.tensor(cut(e.pairs[:n], 128), dtype=torch.int32, device="cuda")
+    _, got = e.run(x, chunks=chunks, count=torch.tensor([len(chunks)], dtype=torch.int32, device="cuda"), capacity=len(chunks), pair_count=n)
+    there = torch.zeros((tokens, TOP_K), dtype=torch.bool, device="cuda")
+    there[e.pairs[:n, 0].long(), e.pairs[:n, 2].long()] = True
+    assert torch.equal(got[there], want[there]) and not got[~there].any()

@@ -830,7 +830,7 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;
     const uint64_t experts = tab.num_experts;
     const bool tiles_carry_shared = stream_tokens > kSliceRideless && stream_tokens <= kSharedSplitMaxRows && stream_pairs >= 5 * experts;
-    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens <= kSharedSliceMaxRows && !tiles_carry_shared &&
+    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens != 0 && stream_tokens <= kSharedSliceMaxRows && !tiles_carry_shared &&
         grouped_slice_ok(tab, cl, stream_pairs, g.d, g.f)) {
         if (ride && !ride->slice) ride = nullptr;
         if (ride && ride_taken) *ride_taken = true;
