@@ -180,6 +180,22 @@ def test_results_do_not_depend_on_the_work_list(tokens, experts, d, f):
     check_rounded(acts, e.exact_acts(x))
 
 
+@pytest.mark.parametrize("tokens,experts,d,f,pad", [(60, 16, 512, 128, 0), (300, 16, 1280, 256, 0),      # matrix-core tiles
+                                                    (6, 64, 1280, 256, 0),                                # quad kernels
+                                                    (6, 64, 1280, 256, 4)])                               # rows off 16 bytes: a row at a time, the next pair fetched ahead
+def test_other_kernels_pass_over_chunks_without_pairs(tokens, experts, d, f, pad):
+    # A list of the same runs with chunks of no pairs in front, between and behind, these ones starting where the pairs end
+    e = Experts(0x56CE + tokens + pad, tokens, experts, d, f)
+    x = torch.randn((tokens, d + pad), device="cuda", generator=e.gen).half()
+    acts, partials = e.run(x, stride=d + pad)
+    runs = cut(e.pairs, 128)
+    chunks = [(1, 0, 0)] + [c for run in runs for c in (run, (2, run[1] + run[2], 0))] + [(0, e.n, 0)] * 3
+    table = torch.tensor(chunks, dtype=torch.int32, device="cuda")
+    got_acts, got = e.run(x, stride=d + pad, chunks=table, count=torch.tensor([len(chunks)], dtype=torch.int32, device="cuda"), capacity=len(chunks))
+    assert torch.equal(got_acts, acts) and torch.equal(got, partials)
+    assert float((acts.double() - e.exact_acts(x[:, :d])).norm() / acts.double().norm()) < 1e-3 and float((partials.double() - e.exact_partials(acts)).norm() / partials.double().norm()) < 1e-3
+
+
 @pytest.mark.parametrize("tokens,experts", [(24, 48), (32, 64), (32, 85)])
 def test_few_tokens_are_their_three_calls(tokens, experts):
     e = Experts(0x54CE + tokens, tokens, experts, 1280, 256)

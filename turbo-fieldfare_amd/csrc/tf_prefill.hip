@@ -684,7 +684,7 @@ __global__ __launch_bounds__(256) void grouped_down_short_kernel(ExpertTable tab
                                                                  uint32_t acts_pair_base, half_t *route_partials, int d, int f,
                                                                  int top_k) {
     tf_prefill_group ch;
-    if (!get_chunk(cl, blockIdx.y, ch)) return;
+    if (!get_chunk(cl, blockIdx.y, ch) || ch.pair_count == 0u) return;      // (the first pair is fetched ahead of the loop)
     const uint8_t *base = expert_base(tab, ch.expert);
     if (!base) return;
     const int lane = threadIdx.x & 63;

@@ -298,6 +298,7 @@ __device__ __forceinline__ void grouped_phase1_body(const GroupedP1Args &a, uint
     ch.expert = uniform_u32(ch.expert);
     ch.pair_start = uniform_u32(ch.pair_start);
     ch.pair_count = uniform_u32(ch.pair_count);
+    if (ch.pair_count == 0u) return;      // its last row would be no row
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
     if (!base) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -400,6 +401,7 @@ __device__ __forceinline__ void grouped_down_body(const GroupedDownArgs &a, uint
     ch.expert = uniform_u32(ch.expert);
     ch.pair_start = uniform_u32(ch.pair_start);
     ch.pair_count = uniform_u32(ch.pair_count);
+    if (ch.pair_count == 0u) return;      // its last row would be no row
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
     if (!base) return;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
