@@ -298,9 +298,8 @@ __device__ __forceinline__ void grouped_phase1_body(const GroupedP1Args &a, uint
     ch.expert = uniform_u32(ch.expert);
     ch.pair_start = uniform_u32(ch.pair_start);
     ch.pair_count = uniform_u32(ch.pair_count);
-    if (ch.pair_count == 0u) return;      // its last row would be no row
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
-    if (!base) return;
+    if (!base || ch.pair_count == 0u) return;      // the last row of no pairs would be no row
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n0 = (int)col_tile * kP1BN + wave * 32;
     // the pairs of a chunk ascend by token: offsets are taken from the first pair's row
@@ -401,9 +400,8 @@ __device__ __forceinline__ void grouped_down_body(const GroupedDownArgs &a, uint
     ch.expert = uniform_u32(ch.expert);
     ch.pair_start = uniform_u32(ch.pair_start);
     ch.pair_count = uniform_u32(ch.pair_count);
-    if (ch.pair_count == 0u) return;      // its last row would be no row
     const uint8_t *base = uniform_ptr(expert_base(tab, ch.expert));
-    if (!base) return;
+    if (!base || ch.pair_count == 0u) return;      // the last row of no pairs would be no row
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n0 = (int)col_tile * kDownBN + wave * kQmmWaveN;
     QmmARows<kGroupedWaves> arow;
