@@ -455,14 +455,14 @@ def test_quad_kernels_given_more_batches_than_blocks(T, E, run, singles, blocks_
 
 
 @pytest.mark.parametrize("T,E,d,f,fp16_scales", [
-    (24, 16, 1344, 320, False),     # last slices of one group; two slices of f: six groups of waves
-    (40, 32, 2816, 704, True),      # production widths, fp16 scales and biases
+    (24, 48, 1344, 320, False),     # last slices of one group; two slices of f: six groups of waves
+    (40, 48, 2816, 704, True),      # production widths, fp16 scales and biases
     (100, 16, 1280, 256, False),    # whole slices; chunks of up to 100 pairs: batches of 32
     (90, 12, 2880, 448, False),     # scales off word boundaries; twelve slices, the last of one group
     (80, 8, 1536, 3072, True),      # the widest rows of the down product
 ])
 def test_slice_kernels_match_oracle(T, E, d, f, fp16_scales):
-    # From three pairs per expert on: up to 8, 16 and 32 pairs a unit, units cut out of longer chunks, blocks whose share crosses into other units
+    # From three pairs per expert on, of 48 experts or 80 tokens: up to 8, 16 and 32 pairs a unit, units cut out of longer chunks, blocks whose share crosses into other units
     top_k = 8
     r = resident_pipeline(T, E, d, f, top_k, 0x5100 + T, zipf=True, from_router=False, fp16_scales=fp16_scales)
     counts = np.bincount(r["idx"].ravel(), minlength=E)
@@ -478,7 +478,7 @@ def test_slice_kernels_match_oracle(T, E, d, f, fp16_scales):
 @pytest.mark.parametrize("run", [1, 3, 33, 128])
 def test_slice_kernels_share_out_any_work_list(run):
     # A pair's sums do not depend on whom it shares a unit with, and chunks without pairs are passed over.
-    T, E, d, f, top_k = 24, 16, 1344, 320, 8
+    T, E, d, f, top_k = 24, 48, 1344, 320, 8
     r = resident_pipeline(T, E, d, f, top_k, 0x5200, zipf=True, from_router=False)
     pairs, n = r["sorted_pairs"], T * top_k
     chunks, at = [(0, 0, 0)], 0

@@ -235,3 +235,23 @@ def test_a_number_of_pairs_that_is_no_number_of_tokens_goes_to_the_tiles():
     there = torch.zeros((tokens, TOP_K), dtype=torch.bool, device="cuda")
     there[e.pairs[:n, 0].long(), e.pairs[:n, 2].long()] = True
     assert torch.equal(got[there], want[there]) and not got[~there].any()
+
+
+@pytest.mark.parametrize("tokens,experts,f,shared_f,launches", [
+    (96, 16, 256, 1088, 2), (256, 16, 256, 1088, 2), (80, 128, 704, 2112, 2),      # in the slice launches
+    (33, 16, 256, 1088, 2), (64, 40, 256, 1088, 2), (79, 47, 256, 1088, 2),        # few experts, up to 79 rows: its split tiles in the launches of the routed tiles
+    (53, 48, 256, 1088, 4), (79, 64, 256, 1088, 4), (53, 128, 704, 2112, 4),       # more experts: the slice kernels, and the split kernels behind them
+    (257, 16, 256, 1088, 2),                                                       # dense tiles in the launches of the routed tiles
+    (96, 16, 192, 1088, 4),                                                        # routed rows that only the tiles take: the slice kernels behind them
+])
+def test_what_a_shared_expert_rides_in(tokens, experts, f, shared_f, launches):
+    d, n, k = 1280, tokens * TOP_K, ctx()
+    i32, f16, u8 = (dict(dtype=t, device="cuda") for t in (torch.int32, torch.float16, torch.uint8))
+    pool, x, acts, partials, y = torch.zeros(experts * 65536, **u8), torch.zeros((tokens, d), **f16), torch.zeros((n, f), **f16), torch.zeros((n, d), **f16), torch.zeros((tokens, d), **f16)
+    pairs, chunks, count, cap = torch.zeros((n, 4), **i32), torch.zeros((experts + n // 128 + 1, 3), **i32), torch.zeros(1, **i32), experts + n // 128 + 1
+    w, scratch, off = torch.zeros(d * shared_f, **u8), torch.zeros(shared_f, **f16), tfk.ExpertOffsets(*(4096 * i for i in range(9)))      # recorded, never run
+    gate, up, down = tfk.projection(w, w, w, shared_f, d), tfk.projection(w, w, w, shared_f, d), tfk.projection(w, w, w, d, shared_f)
+    assert launches_of(k, lambda stream: k.lib.tf_prefill_grouped_routed_moe_resident_shared(
+        k.handle, stream, x.data_ptr(), 0, d, pairs.data_ptr(), chunks.data_ptr(), count.data_ptr(), cap, n, pool.data_ptr(), 65536, experts, C.byref(off), acts.data_ptr(),
+        partials.data_ptr(), d, f, TOP_K, tfk.TF_BF16, x.data_ptr(), 0, y.data_ptr(), 0, C.byref(gate), C.byref(up), C.byref(down),
+        *(v for _ in range(3) for v in (scratch.data_ptr(), 0, shared_f * 2)), tokens, shared_f, d, d, 4)) == launches

@@ -820,17 +820,22 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     //     tokens                              16       32       53       64       96      128      200      300      500
     //     experts about equally popular     69/78    97/100  115/110  120/112  153/116  155/123  157/129  159/145  171/179
     //     rows with a common direction      53/49    72/62   104/75   105/76   109/82   111/90   129/106  147/125  163/166
-    // (exactly as many pairs for every one of 64 experts: 3 an expert 55/62, 4 57/62, 6 88/64).  The line above is where a shared expert in the
-    // same call leaves them too: its kernel is chosen by the rows alone, and beside the tiles it would be in launches of its own.  With few experts
-    // the tiles are faster a little earlier (16 experts, 128 / 192 tokens 45/44, 51/59), but a shared expert rides (200 tokens, both 77/72).
-    // Between kSliceRideless and kSharedSplitMaxRows tokens a shared expert rides beside tiles and not here (16 experts, 64 tokens, both 51/56).
+    // What the quad kernels gain where every expert has exactly the same few pairs (48 tokens, 3 an expert: 89/100) no router gives them.
+    // Up to kSharedSplitMaxRows tokens a shared expert in the same call rides beside the tiles and not beside slices: with few experts that is worth
+    // more than the slice kernels, from kSliceMinExperts on less (both, popular experts, 16 experts of 16 / 32 / 48 tokens 46/51, 47/57, 50/59; 40 of
+    // 32 / 40: 57/66, 62/64; 48 of 24 / 40 / 79: 73/64, 76/70, 82/79; 64 of 24 / 40 / 79: 75/67, 76/72, 95/85; the routed stages alone 41/30, 41/35, 45/37;
+    // 50/44, 51/44; 53/42, 74/49, 75/57; 53/45, 75/51, 84/62).
+    // Beyond, the shared expert takes the slice arithmetic whatever the experts, and what it rides beside has to be slices (both, 16 experts of
+    // 96 / 128 / 192 / 256 tokens 68/53, 75/60, 77/75, 80/91; 64 92/73, 97/80, 100/96, 108/107).  So few experts of many tokens pay for it: the routed
+    // stages alone, 16 experts 53/45, 59/51, 66/61, 67/74, about equally popular 48/45, 54/52, 59/62, 67/75; 64 82/64, 84/70, 91/84, 95/92.
+    // The line above is where a shared expert leaves the slice kernels too.
     // Shapes that the slice kernels do not take: quad kernels below five pairs per expert, tiles above.
     const int p1_passes = ((g.d >> 5) + 15) / 16, dn_passes = ((g.f >> 5) + 7) / 8;
     const bool quad_ok = p1_fast && dn_fast && acts16 && g.d <= kQuadMaxD && p1_passes <= 6 && g.f <= kQuadMaxF && dn_passes <= 4 && g.d % 8 == 0 &&
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;
     const uint64_t experts = tab.num_experts;
-    const bool tiles_carry_shared = stream_tokens > kSliceRideless && stream_tokens <= kSharedSplitMaxRows && stream_pairs >= 5 * experts;
-    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens != 0 && stream_tokens <= kSharedSliceMaxRows && !tiles_carry_shared &&
+    const bool few_experts = experts < kSliceMinExperts && stream_tokens <= kSharedSplitMaxRows;
+    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens != 0 && stream_tokens <= kSharedSliceMaxRows && !few_experts &&
         grouped_slice_ok(tab, cl, stream_pairs, g.d, g.f)) {
         if (ride && !ride->slice) ride = nullptr;
         if (ride && ride_taken) *ride_taken = true;

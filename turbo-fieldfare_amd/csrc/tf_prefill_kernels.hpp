@@ -72,7 +72,7 @@ constexpr uint32_t kSharedSplitMaxRows = 79;
 // From there to here as the slice kernels do, whose shape allows it: in launches of their own (2112 x 2816, 96 / 128 / 200 / 256 rows: 54 / 59 / 62 / 60 us
 // on the dense tiles, 27 / 29 / 35 / 38 so; up to 79 rows 20 - 22 split, 19 - 26 so), or by some of the blocks of the routed slice launches.
 constexpr uint32_t kSharedSliceMaxRows = 256;
-constexpr uint32_t kSliceRideless = 48;
+constexpr uint32_t kSliceMinExperts = 48;      // of the routed stages, up to kSharedSplitMaxRows tokens (run_grouped)
 
 // Operands of the grouped expert stages, as the launch helpers pass them on.
 struct GroupedGeom {
