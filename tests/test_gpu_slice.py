@@ -255,3 +255,75 @@ def test_what_a_shared_expert_rides_in(tokens, experts, f, shared_f, launches):
         k.handle, stream, x.data_ptr(), 0, d, pairs.data_ptr(), chunks.data_ptr(), count.data_ptr(), cap, n, pool.data_ptr(), 65536, experts, C.byref(off), acts.data_ptr(),
         partials.data_ptr(), d, f, TOP_K, tfk.TF_BF16, x.data_ptr(), 0, y.data_ptr(), 0, C.byref(gate), C.byref(up), C.byref(down),
         *(v for _ in range(3) for v in (scratch.data_ptr(), 0, shared_f * 2)), tokens, shared_f, d, d, 4)) == launches
+
+
+def same_kind(got, want):
+    """Infinities of the same sign, and NaN, in the same places (a finite product beyond fp16's range is an infinity too); which are finite in both"""
+    want = want.half()
+    assert torch.equal(got.isnan(), want.isnan())
+    assert torch.equal(got == float("inf"), want == float("inf")) and torch.equal(got == float("-inf"), want == float("-inf"))
+    return want.isfinite()
+
+
+def with_odd_rows(x):
+    """Some rows get infinities and NaN: one, one of either sign far apart, two of one sign side by side, in the last columns; returns which rows."""
+    x = x.clone()
+    inf, nan = float("inf"), float("nan")
+    edits = [{3: inf}, {700: -inf}, {5: nan}, {64: inf, x.shape[1] - 65: -inf}, {130: inf, 131: inf}, {x.shape[1] - 1: inf}, {x.shape[1] - 70: -inf, 0: nan}]
+    odd = torch.zeros(x.shape[0], dtype=torch.bool, device="cuda")
+    for i, edit in enumerate(edits):
+        row = i * x.shape[0] // len(edits)
+        odd[row] = True
+        for column, v in edit.items():
+            x[row, column] = v
+    return x, odd
+
+
+def one_huge_activation(mats, column=37):
+    """Rows of gate and up so large that their product is beyond fp16's range where gelu lets it through"""
+    for i in (0, 1):
+        (W, s, b), w = mats[i]
+        s[column] *= 4096
+        b[column] *= 4096
+        w[column] *= 4096
+
+
+@pytest.mark.parametrize("tokens,experts,d,f,fp16", [(24, 48, 1344, 320, False), (90, 16, 1280, 704, True)])
+def test_infinities_and_nan_stay_in_their_rows_and_keep_their_signs(tokens, experts, d, f, fp16):
+    e = Experts(0x57CE + tokens, tokens, experts, d, f, fp16)
+    x = torch.randn((tokens, d), device="cuda", generator=e.gen).half()
+    acts, partials = e.run(x)
+    odd_x, odd = with_odd_rows(x)
+    odd_acts, odd_partials = e.run(odd_x)
+    odd_pairs = odd[e.pairs[:, 0].long()]
+    assert torch.equal(odd_acts[~odd_pairs], acts[~odd_pairs]) and torch.equal(odd_partials[~odd], partials[~odd])
+    same_kind(odd_acts, e.exact_acts(odd_x))
+    assert odd_acts[odd_pairs].isinf().any() and odd_acts[odd_pairs].isnan().any()
+    # the down launch: activations of which one is an infinity
+    e = Experts(0x58CE + tokens, tokens, experts, d, f, fp16, edit=lambda mats: [one_huge_activation(m) for m in mats])
+    acts, partials = e.run(x)
+    assert 0.2 < float(acts.isinf().any(1).float().mean()) < 0.8 and not acts.isnan().any()
+    want = e.exact_partials(acts)
+    finite = same_kind(partials, want)
+    assert partials.isinf().any() and finite.any()
+    small = e.pairs[acts.abs().amax(1) < 100]          # pairs without such an activation, in the units of those with one
+    there = (small[:, 0].long(), small[:, 2].long())
+    assert len(small) > 10
+    check_rounded(partials[there], want[there])
+
+
+@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (200, 1280, 704, True)])
+def test_infinities_and_nan_through_a_shared_expert(rows, d, f, fp16):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + d)
+    mats = [affine(gen, *shape, fp16) for shape in ((f, d), (f, d), (d, f))]
+    x = torch.randn((rows, d), device="cuda", generator=gen).half()
+    y = shared_block(x, mats, d, f, fp16)
+    odd_x, odd = with_odd_rows(x)
+    odd_y = shared_block(odd_x, mats, d, f, fp16)
+    assert torch.equal(odd_y[~odd], y[~odd]) and not odd_y[odd].isfinite().any()
+    one_huge_activation(mats)
+    y = shared_block(x, mats, d, f, fp16)
+    product = lambda a, m: a @ m[1].T.contiguous()
+    same_kind(y, product(half(gelu(half(product(x.double(), mats[0]))) * half(product(x.double(), mats[1]))), mats[2]))
+    assert y.isinf().any() and y.isfinite().any()

@@ -105,14 +105,44 @@ __device__ __forceinline__ uint32_t slice_chunk_cost(uint32_t pairs, uint32_t po
 
 // The sixteen sums of a lane, one tile: 32 weight rows (the lane's row is lane & 31) against pairs acc_row(r, lane), of which the first
 // NR sums (2 NR pairs) are wanted.  x: the wave's activations, xs: the parts of their sums.  Units of 2^-24.
-template <int SD, int NR>
-__device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][4], const bf16x8_t xs, const u32x4 (&w)[kSliceGroups], const u32x2 s, const u32x2 b,
-                                               float16_t &acc) {
+// ODD: the pairs of the lanes with lane_odd have infinities or NaN among these activations (and zeros for xs).  Their sums are taken over the weights
+// themselves, rounded to fp16 as the tile kernels do: infinities of the sign that weight and activation give, where q s and b apart would give NaN (a nibble
+// of zero, the parts of an infinite sum).  The other pairs' are the same as ever.
+template <int SD, int NR, bool ODD>
+__device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][4], const bf16x8_t xs, const u32x4 (&w)[kSliceGroups], u32x2 s, u32x2 b,
+                                               bool lane_odd, float16_t &acc) {
     float16_t zero;
 #pragma unroll
     for (int r = 0; r < 16; ++r) zero[r] = 0.0f;
+    acc = zero;
+    auto masked = [&](const half8_t row, bool of_odd) {                  // zeros for the pairs of the other kind
+        u32x4 v = __builtin_bit_cast(u32x4, row);
+        asm volatile("" : "+v"(v));              // made here, again for every tile
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = lane_odd == of_odd ? v[j] : 0u;
+        return __builtin_bit_cast(half8_t, v);
+    };
+    if constexpr (ODD) {
+#pragma unroll
+        for (int g = 0; g < kSliceGroups; ++g) {
+            const uint32_t s16 = (g & 1) ? s[g >> 1] >> 16 : s[g >> 1] & 0xFFFFu, b16 = (g & 1) ? b[g >> 1] >> 16 : b[g >> 1] & 0xFFFFu;
+            const float sc = sb_to_f32<SD>((uint16_t)s16), bias = sb_to_f32<SD>((uint16_t)b16);
+#pragma unroll
+            for (int d = 0; d < 4; ++d) {
+                uint32_t word = w[g][d];
+                asm volatile("" : "+v"(word));   // as below
+                half8_t weight;
+#pragma unroll
+                for (int j = 0; j < 8; ++j)      // (a weight beyond fp16 stays finite: the other pairs' zeros meet it too)
+                    weight[j] = (half_t)fminf(fmaxf(fmaf((float)(word >> (4 * (j >> 1) + 16 * (j & 1)) & 15u), sc, bias), -65504.0f), 65504.0f);
+                asm volatile("" : "+v"(weight));
+                acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(masked(x[g][d], true), weight, acc, 0, 0, 0);
+            }
+            asm volatile("" : "+v"(s), "+v"(b));
+        }
+    }
     if constexpr (SD == 0) {
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, __builtin_bit_cast(bf16x8_t, u32x4{b[0], b[1], b[0], b[1]}), zero, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, __builtin_bit_cast(bf16x8_t, u32x4{b[0], b[1], b[0], b[1]}), acc, 0, 0, 0);
     } else {
         // an fp16 bias is the sum of two bf16 numbers, of its upper eight and its lower three bits
         u32x2 hi, lo;
@@ -123,7 +153,7 @@ __device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][
             hi[j] = (h0 >> 16) | h1;
             lo[j] = (__float_as_uint(b0 - __uint_as_float(h0)) >> 16) | (__float_as_uint(b1 - __uint_as_float(h1)) & 0xFFFF0000u);
         }
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, __builtin_bit_cast(bf16x8_t, u32x4{lo[0], lo[1], lo[0], lo[1]}), zero, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, __builtin_bit_cast(bf16x8_t, u32x4{lo[0], lo[1], lo[0], lo[1]}), acc, 0, 0, 0);
         acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(xs, __builtin_bit_cast(bf16x8_t, u32x4{hi[0], hi[1], hi[0], hi[1]}), acc, 0, 0, 0);
     }
 #pragma unroll
@@ -134,7 +164,7 @@ __device__ __forceinline__ void slice_multiply(const half8_t (&x)[kSliceGroups][
             uint32_t word = w[g][d];
             asm volatile("" : "+v"(word));       // the operands are made here, word by word: all of a tile's at once would not fit the registers
             const u32x4 q = {word & 0x000F000Fu, word >> 4 & 0x000F000Fu, word >> 8 & 0x000F000Fu, word >> 12 & 0x000F000Fu};
-            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(x[g][d], __builtin_bit_cast(half8_t, q), c, 0, 0, 0);
+            c = __builtin_amdgcn_mfma_f32_32x32x16_f16(ODD ? masked(x[g][d], false) : x[g][d], __builtin_bit_cast(half8_t, q), c, 0, 0, 0);
         }
         const uint32_t sv = s[g >> 1];
         const float sc = SD == 0 ? __uint_as_float((g & 1) ? sv & 0xFFFF0000u : sv << 16) : f16_to_f32((uint16_t)((g & 1) ? sv >> 16 : sv & 0xFFFFu));
@@ -503,6 +533,7 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
         if (!early) ask_next();
         half8_t x[kSliceGroups][4];
         bf16x8_t xs;
+        bool lane_odd = false;
         {
             uint32_t part[3][kSliceGroups];
 #pragma unroll
@@ -521,6 +552,7 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
                     const half_t one = (half_t)1.0f;
                     total = __builtin_amdgcn_mfma_f32_32x32x16_f16(half8_t{one, one, one, one, one, one, one, one}, __builtin_bit_cast(half8_t, v), total, 0, 0, 0);
                 }
+                lane_odd = lane_odd || !(fabsf(total[0]) < INFINITY);          // of 64 fp16 numbers: an infinity or NaN is among them
                 float rest = total[0] * 5.9604644775390625e-8f;                // in units of 2^24, as the products come out
 #pragma unroll
                 for (int p = 0; p < 3; ++p) {                                   // eight bits each
@@ -532,14 +564,16 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const uint32_t p0 = part[0][2 * j] >> 16 | part[0][2 * j + 1], p1 = part[1][2 * j] >> 16 | part[1][2 * j + 1], p2 = part[2][2 * j] >> 16 | part[2][2 * j + 1];
-                v[j] = kb ? p2 : p0;
-                v[2 + j] = kb ? 0u : p1;
+                v[j] = lane_odd ? 0u : kb ? p2 : p0;
+                v[2 + j] = lane_odd || kb ? 0u : p1;
             }
             xs = __builtin_bit_cast(bf16x8_t, v);
         }
 
         // the tiles of the unit
         const uint32_t pieces = unit.count <= 8u ? 1u : unit.count <= 16u ? 2u : 4u;
+        // (beyond the unit's pairs, and in waves without a slice, the registers hold anything)
+        const uint32_t kind = working && ((uint32_t)__ballot(lane_odd) & (0xFFFFFFFFu >> (kSliceBatch - unit.count))) != 0u ? 0u : pieces;
         for (uint32_t t = 0; t < count; ++t) {
             const uint32_t at = done + t;
             // this tile's requests have landed; the next one's, if it has been asked for, may still be on their way.  What a wave
@@ -559,9 +593,10 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
             if (t > 0) reduce(unit.first, unit.count, at - 1u, tile0 + t - 1u, pieces);
             if (t + 1u < count) ask_next();                                     // the last tile's turn comes behind the next unit's activations
             float16_t acc;
-            if (pieces == 1u) slice_multiply<SD, 4>(x, xs, w, s, b, acc);
-            else if (pieces == 2u) slice_multiply<SD, 8>(x, xs, w, s, b, acc);
-            else slice_multiply<SD, 16>(x, xs, w, s, b, acc);
+            if (kind == 1u) slice_multiply<SD, 4, false>(x, xs, w, s, b, false, acc);
+            else if (kind == 2u) slice_multiply<SD, 8, false>(x, xs, w, s, b, false, acc);
+            else if (__builtin_expect(kind != 0u, 1)) slice_multiply<SD, 16, false>(x, xs, w, s, b, false, acc);
+            else slice_multiply<SD, 16, true>(x, xs, w, s, b, lane_odd, acc);
             const uint32_t to = own_sums + (pieces <= 2u ? (at & 1u) * (kSliceSums / 2) : 0u);
             if (pieces > 2u) __builtin_amdgcn_s_barrier();                      // the tile before has been added up
             lds_put16(to, f32x4{acc[0], acc[1], acc[2], acc[3]});
