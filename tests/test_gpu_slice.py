@@ -196,6 +196,34 @@ def test_other_kernels_pass_over_chunks_without_pairs(tokens, experts, d, f, pad
     assert float((acts.double() - e.exact_acts(x[:, :d])).norm() / acts.double().norm()) < 1e-3 and float((partials.double() - e.exact_partials(acts)).norm() / partials.double().norm()) < 1e-3
 
 
+@pytest.mark.parametrize("tokens,experts,d,f,pad,shift", [(24, 48, 1344, 320, 8, 4), (90, 16, 1280, 704, 136, 12), (90, 16, 1280, 256, 0, 8)])
+def test_padded_rows_and_pairs_off_sixteen_bytes(tokens, experts, d, f, pad, shift):
+    # Rows of a longer stride, and a pair list that is aligned to four bytes as its entries are: the same bits.
+    e = Experts(0x59CE + tokens + f, tokens, experts, d, f)
+    x = torch.randn((tokens, d), device="cuda", generator=e.gen).half()
+    acts, partials = e.run(x)
+    padded = torch.full((tokens, d + pad), float("nan"), dtype=torch.float16, device="cuda")
+    padded[:, :d] = x
+    raw = torch.zeros(e.n * 4 + 8, dtype=torch.int32, device="cuda")
+    moved = raw[shift // 4:shift // 4 + e.n * 4]
+    moved.copy_(e.pairs.ravel())
+    assert moved.data_ptr() % 16 == shift
+    got_acts, got = e.run(padded, stride=d + pad, pairs=moved)
+    assert torch.equal(got_acts, acts) and torch.equal(got, partials)
+    check_rounded(acts, e.exact_acts(x))
+
+
+@pytest.mark.parametrize("rows,d,f,pad", [(97, 1344, 1088, 8), (256, 1280, 704, 24)])
+def test_shared_expert_of_padded_rows(rows, d, f, pad):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(rows + d + pad)
+    mats = [affine(gen, *shape, False) for shape in ((f, d), (f, d), (d, f))]
+    x = torch.randn((rows, d), device="cuda", generator=gen).half()
+    padded = torch.full((rows, d + pad), float("nan"), dtype=torch.float16, device="cuda")
+    padded[:, :d] = x
+    assert torch.equal(shared_block(padded, mats, d, f, False, x_stride=d + pad), shared_block(x, mats, d, f, False))
+
+
 @pytest.mark.parametrize("tokens,experts", [(24, 48), (32, 64), (32, 85)])
 def test_few_tokens_are_their_three_calls(tokens, experts):
     e = Experts(0x54CE + tokens, tokens, experts, 1280, 256)

@@ -358,8 +358,9 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
                 const uint8_t *w = GATE_UP ? p.w[t >> 1] + expert_at + (size_t)(row0 + 8u * (t & 1)) * row_bytes : p.w[0] + expert_at + (size_t)(row0 + 8u * t) * row_bytes;
                 slice_copy16(uniform_ptr(w) + w_lane, to + 1024u * t);      // (non-temporal: 2.33 -> 2.5 us a tile)
             }
-            slice_copy4(s_lane + (expert_at + (size_t)row0 * sb_row_bytes), to + kSliceWBytes);
-            slice_copy4(b_lane + (expert_at + (size_t)row0 * sb_row_bytes), to + kSliceWBytes + 256u);
+            const uint64_t sb_at = expert_at + (size_t)row0 * sb_row_bytes;
+            slice_copy4(GATE_UP ? s_lane + sb_at : uniform_ptr(p.s[0] + sb_at) + sb_lane, to + kSliceWBytes);
+            slice_copy4(GATE_UP ? b_lane + sb_at : uniform_ptr(p.b[0] + sb_at) + sb_lane, to + kSliceWBytes + 256u);
             stay_in_order();
         }
         ++asked;
@@ -450,6 +451,14 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
         }
     };
 
+    // The unit's pairs, 16 bytes each, into LDS: word by word, they are aligned to four bytes; past the last the last again
+    auto copy_pairs = [&](const Unit &u, uint32_t to) {
+        uint32_t l = (uint32_t)lane;
+        asm volatile("" : "+v"(l));                            // addresses are made here, no registers keep them
+#pragma unroll
+        for (uint32_t h = 0; h < 2u; ++h)
+            slice_copy4(reinterpret_cast<const uint32_t *>(a.pairs + (u.first + min(16u * h + (l >> 2), u.count - 1u))) + (l & 3u), to + 256u * h);
+    };
     // the unit before: its pairs, its last tile; done: tiles behind this block
     uint32_t before_first = 0u, before_pairs = 0u, before_tile = 0u, before_pieces = 0u, before_count = 0u, done = 0u;
     for (uint32_t tile0 = first.tile;; tile0 = 0u) {
@@ -460,7 +469,7 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
         uint32_t pairs_at = lds + kSlicePairsAt;
         if (done == 0u) {
             pairs_at = ring + kSliceSlot + kSliceWBytes;
-            if (!shared && lane < 32) slice_copy16(a.pairs + (unit.first + min((uint32_t)i, unit.count - 1u)), pairs_at);
+            if (!shared) copy_pairs(unit, pairs_at);
             stay_in_order();
             ask_next();
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kSliceCopies) : "memory");
@@ -609,7 +618,7 @@ __global__ __launch_bounds__(64 * kSliceMaxWaves) void grouped_slice_kernel(Slic
             // every wave has seen this unit's pairs: the next unit's may take their place (landed by the wait of the second tile from here)
             if (t == 0u && wave == 0 && !closing && !shared) {
                 const Unit next = unit_after(unit);
-                if (next.count != 0u && lane < 32) slice_copy16(a.pairs + (next.first + min((uint32_t)i, next.count - 1u)), lds + kSlicePairsAt);
+                if (next.count != 0u) copy_pairs(next, lds + kSlicePairsAt);
                 stay_in_order();
             }
         }
