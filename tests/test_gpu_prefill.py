@@ -600,8 +600,9 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (40, 16, 192, 64, 1088, 192, 4),       # odd numbers of groups in both stages
     (40, 16, 192, 64, 1088, 195, 4),       # output rows that cannot leave as 16-byte pieces: the two calls one after the other
     # dense tiles
-    (96, 16, 2816, 704, 2112, 2816, 4),    # production row widths
-    (97, 16, 2816, 704, 2112, 2816, -4),   # the same bits read as fp16 scales and biases (other numbers, the same equality)
+    (257, 16, 2816, 704, 2112, 2816, 4),   # production row widths
+    (300, 16, 2816, 704, 2112, 2816, -4),  # the same bits read as fp16 scales and biases (other numbers, the same equality)
+    (90, 16, 1216, 320, 1088, 1216, -4),   # rows too short for the slice kernels
     (200, 16, 256, 192, 128, 264, 4),      # two row tiles of the shared expert, padded output rows
     (1100, 8, 128, 64, 64, 128, 4),        # nine shared row tiles: the shared tiles numbered by XCD
     (96, 8, 512, 128, 192, 515, 4),        # output rows that cannot leave as 16-byte pieces: the two calls one after the other
@@ -609,9 +610,14 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (64, 16, 512, 128, 192, 512, 8),       # 8-bit shared expert: likewise
     (65, 16, 2816, 704, 2112, 2816, -4),   # the split kernels (down in four runs) with the same bits read as fp16 scales and biases
     (33, 16, 2816, 704, 2112, 2816, -4),   # and with down in eight
-    (96, 16, 1344, 320, 1088, 1347, 4),    # slice kernels, both experts' units in the same launches; odd output rows
+    (53, 64, 1280, 320, 1088, 1280, 4),    # from 48 experts on the slice kernels, the split kernels behind them: the two calls
+    # slice kernels, both experts' units in the same launches
+    (96, 16, 2816, 704, 2112, 2816, 4),    # production row widths
+    (97, 16, 2816, 704, 2112, 2816, -4),   # fp16 scales and biases
+    (96, 16, 1344, 320, 1088, 1347, 4),    # odd output rows
     (256, 16, 1280, 256, 2112, 1280, -4),  # the most rows they take
     (80, 64, 1280, 256, 3072, 1280, 4),    # the fewest
+    (90, 16, 1280, 192, 1088, 1280, 4),    # routed rows that only the tiles take, a shared expert that the slice kernels take: the two calls
 ])
 def test_routed_and_shared_expert_in_one_call_equal_the_two_calls(T, E, d, f, shared_f, y_stride, bits):
     top_k = 8
