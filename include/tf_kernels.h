@@ -339,9 +339,9 @@ int32_t tf_shared_expert_int8_down(tf_ctx *ctx, tf_stream stream, const tf_proje
  * chain's bits come from two launches over all rows, activations in the buffer the context owns).
  * Otherwise the rows go through the matrix cores: gate and up in one pass with both sums rounded to fp16 before GeGLU
  * (the chain's stage boundary), activations in a buffer the context owns, then the down projection; weights are
- * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm (80 to 256 rows of 1280 to 3072 columns: q*s+b in 32 bits), so
- * results agree with the row chain within the shared expert's tolerance, not bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is
- * left untouched.  weight_bits == 8 (PrefillSharedExpert's default): up to 15 rows in groups against each weight row,
+ * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm (80 to 192 rows, of 2688 columns and more to 256 rows, with d 1280 to
+ * 3072 and intermediate 256 to 3072: q*s+b in 32 bits), so results agree with the row chain within the shared expert's tolerance, not
+ * bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is left untouched.  weight_bits == 8 (PrefillSharedExpert's default): up to 15 rows in groups against each weight row,
  * bit-identical to repeated tf_shared_expert_int8; from 16 aligned rows on on the matrix cores with every weight
  * rounded to fp16 first, within the 8-bit shared expert's tolerance of the row chain (scales keep their precision
  * down to 2^-24; a weight below fp16's normal range, 6e-5, is kept to 6e-8).  query_count == 0 is a no-op.  d, intermediate > 0,

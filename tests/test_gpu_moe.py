@@ -482,8 +482,10 @@ def _random_affine(gen, rows, cols, bits, fp16, small):
     (4, 65, 2816, 2112, False, "groups"),
     # dense tiles: rows too wide for the split kernels, more rows than the slice kernels take, rows too short for them
     (4, 16, 4160, 64, False, None), (4, 257, 2816, 2112, True, None), (4, 257, 2816, 2112, False, "groups"), (4, 100, 1216, 1088, True, "rows"),
+    (4, 256, 1280, 3072, False, None), (4, 193, 2560, 704, True, None),
     # slice kernels: two, one and four pieces of pairs in the last unit, small scales
-    (4, 80, 2816, 2112, True, None), (4, 97, 1344, 1088, False, "rows"), (4, 140, 2816, 2112, True, "groups"), (4, 256, 1280, 3072, False, None),
+    (4, 80, 2816, 2112, True, None), (4, 97, 1344, 1088, False, "rows"), (4, 140, 2816, 2112, True, "groups"), (4, 192, 1280, 3072, False, None),
+    (4, 256, 2816, 2112, False, None),
     # 8 bits: 32 x 32, 64 x 32 and 64 x 64 down tiles, fp16 scales, small scales through each
     (8, 16, 2816, 2112, True, "rows"), (8, 97, 2816, 2112, False, "groups"), (8, 129, 2816, 2112, False, None), (8, 200, 2816, 2112, True, None),
     (8, 200, 2816, 2112, False, "rows"), (8, 33, 1088, 1984, True, None),

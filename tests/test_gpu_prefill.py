@@ -603,6 +603,7 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (257, 16, 2816, 704, 2112, 2816, 4),   # production row widths
     (300, 16, 2816, 704, 2112, 2816, -4),  # the same bits read as fp16 scales and biases (other numbers, the same equality)
     (90, 16, 1216, 320, 1088, 1216, -4),   # rows too short for the slice kernels
+    (256, 16, 1280, 256, 2112, 1280, -4),  # more rows of their length than the slice kernels take
     (200, 16, 256, 192, 128, 264, 4),      # two row tiles of the shared expert, padded output rows
     (1100, 8, 128, 64, 64, 128, 4),        # nine shared row tiles: the shared tiles numbered by XCD
     (96, 8, 512, 128, 192, 515, 4),        # output rows that cannot leave as 16-byte pieces: the two calls one after the other
@@ -610,12 +611,15 @@ def test_grouped_gemm_on_matrix_cores_matches_oracle(T, E, d, f, zipf):
     (64, 16, 512, 128, 192, 512, 8),       # 8-bit shared expert: likewise
     (65, 16, 2816, 704, 2112, 2816, -4),   # the split kernels (down in four runs) with the same bits read as fp16 scales and biases
     (33, 16, 2816, 704, 2112, 2816, -4),   # and with down in eight
-    (53, 64, 1280, 320, 1088, 1280, 4),    # from 48 experts on the slice kernels, the split kernels behind them: the two calls
+    (53, 64, 1280, 320, 1088, 1280, 4),    # more experts
+    (53, 64, 2816, 320, 1088, 2816, 4),    # from 48 experts of long rows on the slice kernels, the split kernels behind them: the two calls
+    (53, 96, 1280, 320, 1088, 1280, 4),    # and of short ones with fewer than five pairs an expert
     # slice kernels, both experts' units in the same launches
     (96, 16, 2816, 704, 2112, 2816, 4),    # production row widths
     (97, 16, 2816, 704, 2112, 2816, -4),   # fp16 scales and biases
     (96, 16, 1344, 320, 1088, 1347, 4),    # odd output rows
-    (256, 16, 1280, 256, 2112, 1280, -4),  # the most rows they take
+    (256, 16, 2816, 256, 2112, 2816, -4),  # the most rows they take
+    (192, 16, 1280, 256, 2112, 1280, -4),  # and of up to 2560 columns
     (80, 64, 1280, 256, 3072, 1280, 4),    # the fewest
     (90, 16, 1280, 192, 1088, 1280, 4),    # routed rows that only the tiles take, a shared expert that the slice kernels take: the two calls
 ])

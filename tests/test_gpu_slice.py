@@ -133,7 +133,7 @@ def shared_block(x, mats, d, f, fp16, x_stride=None):
 
 @pytest.mark.parametrize("size", [1e-3, 1e-4, 1e-5])
 @pytest.mark.parametrize("stage", ["gate / up", "down"])
-@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (256, 1280, 704, True)])
+@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (192, 1280, 704, True), (256, 2688, 704, False)])
 def test_shared_expert_keeps_the_bits_of_small_activations(rows, d, f, fp16, stage, size):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(rows + d)
@@ -213,7 +213,7 @@ def test_padded_rows_and_pairs_off_sixteen_bytes(tokens, experts, d, f, pad, shi
     check_rounded(acts, e.exact_acts(x))
 
 
-@pytest.mark.parametrize("rows,d,f,pad", [(97, 1344, 1088, 8), (256, 1280, 704, 24)])
+@pytest.mark.parametrize("rows,d,f,pad", [(97, 1344, 1088, 8), (192, 1280, 704, 24), (256, 2688, 704, 40)])
 def test_shared_expert_of_padded_rows(rows, d, f, pad):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(rows + d + pad)
@@ -265,15 +265,16 @@ def test_a_number_of_pairs_that_is_no_number_of_tokens_goes_to_the_tiles():
     assert torch.equal(got[there], want[there]) and not got[~there].any()
 
 
-@pytest.mark.parametrize("tokens,experts,f,shared_f,launches", [
-    (96, 16, 256, 1088, 2), (256, 16, 256, 1088, 2), (80, 128, 704, 2112, 2),      # in the slice launches
-    (33, 16, 256, 1088, 2), (64, 40, 256, 1088, 2), (79, 47, 256, 1088, 2),        # few experts, up to 79 rows: its split tiles in the launches of the routed tiles
-    (53, 48, 256, 1088, 4), (79, 64, 256, 1088, 4), (53, 128, 704, 2112, 4),       # more experts: the slice kernels, and the split kernels behind them
-    (257, 16, 256, 1088, 2),                                                       # dense tiles in the launches of the routed tiles
-    (96, 16, 192, 1088, 4),                                                        # routed rows that only the tiles take: the slice kernels behind them
+@pytest.mark.parametrize("tokens,experts,d,f,shared_f,launches", [
+    (96, 16, 1280, 256, 1088, 2), (192, 16, 2560, 256, 1088, 2), (256, 16, 2688, 256, 1088, 2), (80, 128, 1280, 704, 2112, 2),      # in the slice launches
+    (33, 16, 2816, 256, 1088, 2), (64, 40, 1280, 256, 1088, 2), (79, 47, 2816, 256, 1088, 2),        # few experts, up to 79 rows: its split tiles in the launches of the routed tiles
+    (79, 64, 2560, 256, 1088, 2), (53, 84, 1280, 256, 1088, 2),                                      # and more experts of up to 2560 columns, from five pairs each on
+    (53, 48, 2816, 256, 1088, 4), (79, 64, 2688, 256, 1088, 4), (53, 85, 1280, 704, 2112, 4),        # longer rows, fewer pairs: the slice kernels, and the split kernels behind them
+    (257, 16, 2816, 256, 1088, 2), (193, 16, 2560, 256, 1088, 2),                                    # dense tiles in the launches of the routed tiles
+    (96, 16, 1280, 192, 1088, 4),                                                                    # routed rows that only the tiles take: the slice kernels behind them
 ])
-def test_what_a_shared_expert_rides_in(tokens, experts, f, shared_f, launches):
-    d, n, k = 1280, tokens * TOP_K, ctx()
+def test_what_a_shared_expert_rides_in(tokens, experts, d, f, shared_f, launches):
+    n, k = tokens * TOP_K, ctx()
     i32, f16, u8 = (dict(dtype=t, device="cuda") for t in (torch.int32, torch.float16, torch.uint8))
     pool, x, acts, partials, y = torch.zeros(experts * 65536, **u8), torch.zeros((tokens, d), **f16), torch.zeros((n, f), **f16), torch.zeros((n, d), **f16), torch.zeros((tokens, d), **f16)
     pairs, chunks, count, cap = torch.zeros((n, 4), **i32), torch.zeros((experts + n // 128 + 1, 3), **i32), torch.zeros(1, **i32), experts + n // 128 + 1
@@ -340,7 +341,7 @@ def test_infinities_and_nan_stay_in_their_rows_and_keep_their_signs(tokens, expe
     check_rounded(partials[there], want[there])
 
 
-@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (200, 1280, 704, True)])
+@pytest.mark.parametrize("rows,d,f,fp16", [(97, 1344, 1088, False), (192, 1280, 704, True)])
 def test_infinities_and_nan_through_a_shared_expert(rows, d, f, fp16):
     gen = torch.Generator(device="cuda")
     gen.manual_seed(rows + d)

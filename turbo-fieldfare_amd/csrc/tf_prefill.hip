@@ -815,7 +815,7 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     const bool p1_fast = blobs16 && hidden16 && off.gate_W_off % 16 == 0 && off.up_W_off % 16 == 0;
     const bool dn_fast = blobs16 && acts16 && off.down_W_off % 16 == 0;
     int32_t rc;
-    // Fewer than three pairs per expert on average go to the quad kernels; from there on up to kSharedSliceMaxRows tokens to the slice kernels, more to
+    // Fewer than three pairs per expert on average go to the quad kernels; from there on up to slice_max_rows tokens to the slice kernels, more to
     // the matrix-core tiles.  Top 8 of 128 experts, d 2816, f 704, quad or tiles / slice, both launches, us:
     //     tokens                              16       32       53       64       96      128      200      300      500
     //     experts about equally popular     69/78    97/100  115/110  120/112  153/116  155/123  157/129  159/145  171/179
@@ -824,18 +824,25 @@ int32_t run_grouped(tf_ctx *ctx, hipStream_t st, const ExpertTable &tab, const t
     // Up to kSharedSplitMaxRows tokens a shared expert in the same call rides beside the tiles and not beside slices: with few experts that is worth
     // more than the slice kernels, from kSliceMinExperts on less (both, popular experts, 16 experts of 16 / 32 / 48 tokens 46/51, 47/57, 50/59; 40 of
     // 32 / 40: 57/66, 62/64; 48 of 24 / 40 / 79: 73/64, 76/70, 82/79; 64 of 24 / 40 / 79: 75/67, 76/72, 95/85; the routed stages alone 41/30, 41/35, 45/37;
-    // 50/44, 51/44; 53/42, 74/49, 75/57; 53/45, 75/51, 84/62).
+    // 50/44, 51/44; 53/42, 74/49, 75/57; 53/45, 75/51, 84/62).  That is so where the rows are long: of up to 2560 columns the ride is worth more wherever there is
+    // one, from five pairs per expert on (both, 64 experts, equally popular and popular, 1280 x 640 of 56 tokens 42/55, 33/47; 2048 x 768 of 40 / 72
+    // 59/66, 43/51; 64/69, 48/61; 2560 x 640 68/69, 50/57; 68/71, 54/62); with fewer, slices beat the quad kernels at every width (128 experts, 56 or
+    // 72 tokens, both: 1280 x 640 74/68, 57/47; 2048 x 768 107/103, 83/60).
     // Beyond, the shared expert takes the slice arithmetic whatever the experts, and what it rides beside has to be slices (both, 16 experts of
     // 96 / 128 / 192 / 256 tokens 68/53, 75/60, 77/75, 80/91; 64 92/73, 97/80, 100/96, 108/107).  So few experts of many tokens pay for it: the routed
-    // stages alone, 16 experts 53/45, 59/51, 66/61, 67/74, about equally popular 48/45, 54/52, 59/62, 67/75; 64 82/64, 84/70, 91/84, 95/92.
+    // stages alone, 16 experts 53/45, 59/51, 66/61, 67/74, about equally popular 48/45, 54/52, 59/62, 67/75; 64 82/64, 84/70, 91/84, 95/92; the worst, 32 equally
+    // popular experts of 256 tokens, 62/82, and of 2880 x 2880 196/277).  The tiles for these alone would leave the shared expert in launches of its own
+    // (16 experts, 256 tokens, both 65 + 39), and its kernel cannot ask for the experts: alone and in one call it gives the same bits.  For the same reason a shared
+    // expert of 80 rows and more pays two launches of its own where only one of the two has widths for the slice kernels (both, 128 experts of 192 x 2816, 96 / 200
+    // tokens 78/85, 84/94; routed 704 and shared 3136, 163/179, 167/192).
     // The line above is where a shared expert leaves the slice kernels too.
     // Shapes that the slice kernels do not take: quad kernels below five pairs per expert, tiles above.
     const int p1_passes = ((g.d >> 5) + 15) / 16, dn_passes = ((g.f >> 5) + 7) / 8;
     const bool quad_ok = p1_fast && dn_fast && acts16 && g.d <= kQuadMaxD && p1_passes <= 6 && g.f <= kQuadMaxF && dn_passes <= 4 && g.d % 8 == 0 &&
                          g.f % 4 == 0 && aligned(g.route_partials, 8) && aligned(g.acts, 8) && tab.pool != nullptr;
     const uint64_t experts = tab.num_experts;
-    const bool few_experts = experts < kSliceMinExperts && stream_tokens <= kSharedSplitMaxRows;
-    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens != 0 && stream_tokens <= kSharedSliceMaxRows && !few_experts &&
+    const bool ride_pays = stream_tokens <= kSharedSplitMaxRows && (experts < kSliceMinExperts || ((uint32_t)g.d < kSliceWideCols && stream_pairs >= 5 * experts));
+    if (p1_fast && dn_fast && acts16 && stream_pairs >= 3 * experts && stream_tokens != 0 && stream_tokens <= slice_max_rows((uint32_t)g.d) && !ride_pays &&
         grouped_slice_ok(tab, cl, stream_pairs, g.d, g.f)) {
         if (ride && !ride->slice) ride = nullptr;
         if (ride && ride_taken) *ride_taken = true;

@@ -71,7 +71,12 @@ struct DenseRide {
 constexpr uint32_t kSharedSplitMaxRows = 79;
 // From there to here as the slice kernels do, whose shape allows it: in launches of their own (2112 x 2816, 96 / 128 / 200 / 256 rows: 54 / 59 / 62 / 60 us
 // on the dense tiles, 27 / 29 / 35 / 38 so; up to 79 rows 20 - 22 split, 19 - 26 so), or by some of the blocks of the routed slice launches.
-constexpr uint32_t kSharedSliceMaxRows = 256;
+// The last row of that range depends on the columns: of 2560 and fewer, 200 to 256 tokens are no faster with both in slice launches than with both on the
+// tiles, and slower where experts are popular (128 experts, equally popular and popular, one call with a shared expert, tiles/slices, us: 1280 x 640
+// 200 tokens 69/69 52/53, 256 69/73 52/63; 2048 x 768 120/111 74/76, 122/119 75/86; 2560 x 640 134/119 71/78, 133/127 82/92; but 144 tokens
+// 69/65 50/47, 119/100 67/61, 136/110 70/66).  At 2816 x 704 163/134 88/88 and 166/142 90/102; rows with a common direction, routed stages, 200 tokens 129/106.
+constexpr uint32_t kSliceWideCols = 2688;
+inline uint32_t slice_max_rows(uint32_t cols) { return cols >= kSliceWideCols ? 256u : 192u; }
 constexpr uint32_t kSliceMinExperts = 48;      // of the routed stages, up to kSharedSplitMaxRows tokens (run_grouped)
 
 // Operands of the grouped expert stages, as the launch helpers pass them on.

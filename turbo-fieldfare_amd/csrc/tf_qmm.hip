@@ -821,7 +821,7 @@ int32_t shared_expert_block_impl(tf_ctx *ctx, tf_stream stream, const void *x, u
                             intermediate % TF_GROUP_SIZE == 0 && query_count <= (uint32_t)INT32_MAX &&
                             geglu_arrays_near(gate, up);
     // one choice for the call alone and for a ride
-    const bool slice = block_path && query_count > kSharedSplitMaxRows && query_count <= kSharedSliceMaxRows && shared_slice_ok(gate);
+    const bool slice = block_path && query_count > kSharedSplitMaxRows && query_count <= slice_max_rows(d) && shared_slice_ok(gate);
     const bool split = block_path && query_count <= kSharedSplitMaxRows && geglu_split_ok(gate, x_stride_elements);
     if (plan && !block_path) return TF_OK;
     if (weight_bits == 8 && pointers && even && query_count >= 2) {
