@@ -341,10 +341,11 @@ int32_t tf_shared_expert_int8_down(tf_ctx *ctx, tf_stream stream, const tf_proje
  * (the chain's stage boundary), activations in a buffer the context owns, then the down projection; weights are
  * expanded to fp16 half(q*s+b) per group as in tf_int4_qmm (80 to 192 rows, of 2688 columns and more to 256 rows, with d 1280 to
  * 3072 and intermediate 256 to 3072: q*s+b in 32 bits), so results agree with the row chain within the shared expert's tolerance, not
- * bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is left untouched.  weight_bits == 8 (PrefillSharedExpert's default): up to 15 rows in groups against each weight row,
- * bit-identical to repeated tf_shared_expert_int8; from 16 aligned rows on on the matrix cores with every weight
- * rounded to fp16 first, within the 8-bit shared expert's tolerance of the row chain (scales keep their precision
- * down to 2^-24; a weight below fp16's normal range, 6e-5, is kept to 6e-8).  query_count == 0 is a no-op.  d, intermediate > 0,
+ * bit for bit, and the caller's scratch (still validated: one row each, lengths in BYTES) is left untouched.
+ * weight_bits == 8 (PrefillSharedExpert's default): up to 15 rows in groups against each weight row, bit-identical to
+ * repeated tf_shared_expert_int8; from 16 aligned rows on on the matrix cores with every weight rounded to fp16 first,
+ * within the 8-bit shared expert's tolerance of the row chain (scales keep their precision down to 2^-24; a weight below
+ * fp16's normal range, 6e-5, is kept to 6e-8).  query_count == 0 is a no-op.  d, intermediate > 0,
  * strides >= d (TF_ERR_INVALID_ARGUMENT); gate/up = (intermediate, d), down = (d, intermediate) or
  * TF_ERR_DIMENSION_MISMATCH. */
 int32_t tf_prefill_shared_expert_int4_block(tf_ctx *ctx, tf_stream stream,
@@ -755,8 +756,9 @@ int32_t tf_prefill_grouped_routed_moe_resident(tf_ctx *ctx, tf_stream stream,
  * shared expert's matrix-core tiles (up to 79 rows its split contractions) are placed ahead of the routed tiles in the same two
  * launches (gate / up / GeGLU, then down) instead of under-filling the chip in launches of their own, and from 80 to 256 rows some of
  * the blocks of the routed launches take them; results are bit-identical to the two calls.
- * Applies when the routed pairs go to the matrix-core tile or slice kernels and the shared expert is 4-bit with at least 8 rows and
- * 16-byte aligned operands; otherwise the two calls are made one after the other.  Arguments: those of the routed call, then
+ * Applies when the routed pairs go to the matrix-core tile kernels and the shared expert is 4-bit with at least 8 rows and 16-byte
+ * aligned operands, or when both go to the slice kernels (the shared expert from 80 rows on); otherwise, as where only one of the two
+ * goes to the slice kernels, the two calls are made one after the other.  Arguments: those of the routed call, then
  * those of the shared call (its d is the routed d, its scale dtype the routed one; query_count token rows). */
 int32_t tf_prefill_grouped_routed_moe_resident_shared(tf_ctx *ctx, tf_stream stream,
                                                const void *hidden, uint64_t hidden_offset, uint32_t hidden_stride_elements,
